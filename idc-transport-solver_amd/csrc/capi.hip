@@ -18,8 +18,6 @@ enum class Pattern { WavefrontGraph, WavefrontEager, Staggered, StaggeredGE };
 
 static bool is_staggered(Pattern p) { return p == Pattern::Staggered || p == Pattern::StaggeredGE; }
 
-constexpr int kXcds = 8;  // MI355X: workgroup b runs on XCD b mod 8, each XCD with its own L2
-
 struct tsw_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -110,6 +108,19 @@ struct tsw_ctx {
     // launch groups by (DG degree, compute waves, material path), side streams for the groups.
     std::vector<std::unique_ptr<tsw_ctx>> batch;
     double batch_dt = 0.0;
+    // Work counters of persistent lane-split launches (kSplitWorkInts words): each launch uses one set and
+    // clears the other, so the launches that share it must be ordered on one stream or by events.
+    struct SplitWork {
+        DBuf buf;
+        int set = 0;
+        int *get(hipStream_t s) {
+            if (!buf.ptr) {
+                buf.reserve(sizeof(int) * kSplitWorkInts);
+                TSW_HIP(hipMemsetAsync(buf.ptr, 0, sizeof(int) * kSplitWorkInts, s));
+            }
+            return buf.as<int>();
+        }
+    };
     struct Group {
         int p = 0, waves = 0, max_ny = 0;
         bool mat = false;
@@ -130,7 +141,9 @@ struct tsw_ctx {
         // 16-byte aligned): members in row bands of at most `rows` rows, items {slot, band * nq + ordinate}
         bool split = false;
         int rows = 0;
-        DBuf work;  // persistent launch: the item counter
+        SplitWork work;  // persistent launch: the item counters, and its items ordered by queue
+        std::vector<int> qitems;
+        DBuf dev_qitems;
         std::vector<int> band_rows;  // per member slot, fixed when the items are built
     };
     // Engine of each batch member, chosen per DG degree (tsw_batch_set): the staggered kernels through
@@ -147,7 +160,8 @@ struct tsw_ctx {
         std::vector<unsigned char> host;
         std::vector<int> items;
         DBuf params, dev_items, traces, stage;
-        DBuf xtr64, xtr32, work;  // lane-split sweeps: exchange records per source, persistent-launch counter
+        DBuf xtr64, xtr32;  // lane-split sweeps: exchange records per source
+        SplitWork work;     // their persistent launches' item counters
         size_t xtr64_n = 0, xtr32_n = 0;
     } multi;
     // Sweeps of this problem on the caller's layout by the lane-split kernel where it is built and its
@@ -304,6 +318,8 @@ struct tsw_ctx {
 constexpr size_t kScratchBytes = size_t(128) << 20;  // 128 MiB per GPU
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 constexpr int kMaxScratchDevices = 64;
+// Largest reference-layout array of the lane-split kernel: dropped stores are addressed at its end, in 32 bits.
+constexpr size_t kSplitRefBytes = (size_t(1) << 32) - 256;
 constexpr int kSplitBatchPrefetch = 4;  // prefetch depth of the batch's lane-split groups
 static std::mutex g_scratch_mu;
 static void *g_scratch_ptr[kMaxScratchDevices] = {};
@@ -2396,13 +2412,24 @@ int split_lanes_of(int p) { return p == 1 ? 2 : 4; }
 
 // Rows per band of a problem (a batch member, or a single problem) on the lane-split kernel: the fewest
 // bands of at most R rows (R: the tuning key batch_split_rows, else the batch autotuner's choice for the
-// degree, else the rows one workgroup of 512 threads holds), split evenly.
+// degree, else the rows one workgroup of 512 threads, two storer waves among them, holds, or 64 at degree 2),
+// split evenly.  Degree 2: four compute waves, one per SIMD, against six (256 x 256, S8, 64 materials, FP64: 270 against
+// 296 us; 280 x 280 S12 lattice: 468 against 481); degrees 1 and 3 lose with fewer rows (a longer chain of bands:
+// 280 x 280 Q1 246 against 215 us).
 int split_band_rows(const tsw_ctx *ctx, int p, int ny) {
-    int R = 512 / split_lanes_of(p);
+    int R = p == 2 ? 64 : 384 / split_lanes_of(p);
     const int want = ctx->batch_split_rows_opt > 0 ? ctx->batch_split_rows_opt : ctx->split_rows_p[p & 3];
     if (want > 0) R = std::min(R, want);
     const int nb = (ny + R - 1) / R;
     return (ny + nb - 1) / nb;
+}
+
+// Prefetch depth of the lane-split kernel on the reference layout: 3 for FP64 Q3, whose ring of 4 spills (256 x 256, S8,
+// 64 materials: 461 against 556 us), else kSplitBatchPrefetch, unless the tuning key batch_split_prefetch sets it.
+template <typename T>
+int split_prefetch(const tsw_ctx *c, int p) {
+    if (c->batch_split_pf_opt > 0) return c->batch_split_pf_opt;
+    return p == 3 && sizeof(T) == 8 ? 3 : kSplitBatchPrefetch;
 }
 
 // Whether this context's sweeps can run the staggered kernel on the caller's layout for `psi`.
@@ -2418,6 +2445,7 @@ template <typename T>
 bool split_ref_plan(tsw_ctx *c, const double *sig, double dt, DiagSweepParams<T> &base, size_t &lds) {
     const Geom &g = c->g;
     if (c->ref_split_opt < 0 || g.p < 1) return false;
+    if (c->g.npsi() * sizeof(double) > kSplitRefBytes) return false;
     // a set band_rows, prefetch, one_wave or lane_split asks for the diagonal-layout kernels
     if (c->band_rows_opt != 0 || c->prefetch_opt != 0 || c->one_wave_opt != 0 || c->split_opt != 0) return false;
     const bool f64 = sizeof(T) == 8;
@@ -2425,7 +2453,7 @@ bool split_ref_plan(tsw_ctx *c, const double *sig, double dt, DiagSweepParams<T>
     base = make_diag_params<T>(c, dt, nullptr, nullptr, false, nullptr);
     if (!base.ainv) return false;
     const int br = split_band_rows(c, g.p, g.ny);
-    lds = split_sweep_lds_bytes<T>(g.p, br, g.nx, base.M);
+    lds = split_sweep_lds_bytes<T>(g.p, br, base.M);
     if (lds == 0) return false;
     base.split = 1;
     base.direct = 0;
@@ -2438,76 +2466,48 @@ bool split_ref_plan(tsw_ctx *c, const double *sig, double dt, DiagSweepParams<T>
     return true;
 }
 
-// One persistent launch of the lane-split kernel sweeping every ordinate of each array arr[r] in place
-// (reference layout, 16-byte aligned), with base from split_ref_plan: items {source, band * nq + ordinate},
-// band-major; per-source inflow traces from the arrays' halos and per-source exchange records.  Counted
-// as arr.size() sweeps.
+// The lane-split kernel sweeping every ordinate of each array arr[r] in place (reference layout, 16-byte
+// aligned), with base from split_ref_plan, in launches of up to kSplitSources sources; per-source exchange
+// records.  Counted as arr.size() sweeps.
 template <typename T>
-void split_ref_sweep(tsw_ctx *c, const DiagSweepParams<T> &base, size_t lds, const std::vector<double *> &arr) {
+void split_ref_sweep(tsw_ctx *c, DiagSweepParams<T> base, size_t lds, const std::vector<double *> &arr) {
     const Geom &g = c->g;
-    const int n = (int)arr.size(), nb = base.nbands;
-    const size_t ntx = (size_t)g.nq * g.ny * (g.p + 1), nty = (size_t)g.nq * g.nx * (g.p + 1);
-    T *tr = static_cast<T *>(c->multi.traces.reserve(sizeof(T) * (ntx + nty) * n));
     auto &M = c->multi;
     hipStream_t s = c->stream;
+    const int n = (int)arr.size(), nb = base.nbands, most = std::min(n, kSplitSources);
     const size_t per = nb > 1 ? (size_t)g.nq * (nb - 1) * g.nx * (g.p + 1) : 0;  // records of one source
-    T *xtr = nullptr;
     if (per) {
         DBuf &xb = sizeof(T) == 8 ? M.xtr64 : M.xtr32;
         size_t &have = sizeof(T) == 8 ? M.xtr64_n : M.xtr32_n;
-        if (have < per * n) {  // every record empty (the sentinel); a sweep leaves them empty again
-            xb.reserve(sizeof(T) * per * n);
-            have = per * n;
+        if (have < per * most) {  // every record empty (the sentinel); a sweep leaves them empty again
+            xb.reserve(sizeof(T) * per * most);
+            have = per * most;
             launch_exchange_fill<T>(xb.as<T>(), have, s);
         }
-        xtr = xb.as<T>();
+        base.xtr = xb.as<T>();
+        base.abort_flag = abort_flag_of(c);
     }
-    M.host.resize(sizeof(DiagSweepParams<T>) * n);
-    DiagSweepParams<T> *ps = reinterpret_cast<DiagSweepParams<T> *>(M.host.data());
-    for (int r = 0; r < n; ++r) {
-        ps[r] = base;
-        ps[r].qref = arr[r];
-        ps[r].psi_ref = arr[r];
-        ps[r].tin_x = tr + (ntx + nty) * r;
-        ps[r].tin_y = tr + (ntx + nty) * r + ntx;
-        if (per) {
-            ps[r].xtr = xtr + per * r;
-            ps[r].abort_flag = abort_flag_of(c);
-        }
-    }
-    M.items.clear();
-    for (int band = 0; band < nb; ++band)
-        for (int r = 0; r < n; ++r)
-            for (int q = 0; q < g.nq; ++q) {
-                M.items.push_back(r);
-                M.items.push_back(band * g.nq + q);
-            }
-    TSW_HIP(hipMemcpyAsync(M.params.reserve(M.host.size()), M.host.data(), M.host.size(), hipMemcpyHostToDevice, s));
-    TSW_HIP(hipMemcpyAsync(M.dev_items.reserve(sizeof(int) * M.items.size()), M.items.data(),
-                           sizeof(int) * M.items.size(), hipMemcpyHostToDevice, s));
-    DiagSweepParams<T> rep{};
-    rep.qref = reinterpret_cast<const double *>(1);
-    rep.ainv = base.ainv;
-    rep.split = 1;
-    rep.prefetch = c->batch_split_pf_opt > 0 ? c->batch_split_pf_opt : kSplitBatchPrefetch;
-    if (c->batch_persistent_opt > 0) {
-        rep.work = static_cast<int *>(M.work.reserve(sizeof(int)));
-        TSW_HIP(hipMemsetAsync(rep.work, 0, sizeof(int), s));
-    }
-    const DiagSweepParams<T> *dp = M.params.as<DiagSweepParams<T>>();
+    base.prefetch = split_prefetch<T>(c, g.p);
     if (c->stall_test && per) {  // tuning key stall_test: every bounded wait of the banded sweep gives up
         c->stall_test = false;
         int *flag = abort_flag_of(c);
         *c->abort_host = 1;
         TSW_HIP(hipMemcpyAsync(flag, c->abort_host, sizeof(int), hipMemcpyHostToDevice, s));
     }
+    int *work = c->batch_persistent_opt > 0 ? M.work.get(s) : nullptr;
     hipEvent_t e0 = next_event(c), e1 = next_event(c);
     TSW_HIP(hipEventRecord(e0, s));
-    launch_diag_inflow_batch<T>(dp, n, g.p, s);
-    launch_diag_sweep_batch<T>(rep, dp, M.dev_items.as<int2>(), (int)M.items.size() / 2, base.band_rows, lds, g.p, s);
+    for (int r0 = 0; r0 < n; r0 += kSplitSources) {
+        SplitSources src{};
+        const int k = std::min(n - r0, kSplitSources);
+        for (int r = 0; r < k; ++r) src.psi[r] = arr[r0 + r];
+        base.work = work;
+        base.work_set = M.work.set;
+        launch_split_ref<T>(base, src, k, lds, g.p, s);
+        M.work.set ^= 1;
+    }
     TSW_HIP(hipEventRecord(e1, s));
     c->sweeps_done += n;
-    TSW_HIP(hipStreamSynchronize(s));  // the host tables may be rebuilt by the next launch
 }
 
 // The lane-split sweep on the caller's layout of arrays arr (16-byte aligned, ref_sweep_ok) when it is
@@ -3873,9 +3873,10 @@ int tsw_batch_set(tsw_ctx *ctx, int nprob, const tsw_problem *probs, const doubl
             // the lane-split kernel where it is built for the degree and the member's tables fit its LDS
             const int sbr = g.p >= 1 ? split_band_rows(ctx, g.p, g.ny) : 0;
             ctx->split_able[b] = ctx->batch_split_opt >= 0 && g.p >= 1 && sub->mat.valid &&
+                                 g.npsi() * sizeof(double) <= kSplitRefBytes &&
                                  diag_inverses<double>(sub.get(), dt) && diag_inverses<float>(sub.get(), dt) &&
-                                 split_sweep_lds_bytes<double>(g.p, sbr, g.nx, sub->mat.M) != 0 &&
-                                 split_sweep_lds_bytes<float>(g.p, sbr, g.nx, sub->mat.M) != 0;
+                                 split_sweep_lds_bytes<double>(g.p, sbr, sub->mat.M) != 0 &&
+                                 split_sweep_lds_bytes<float>(g.p, sbr, sub->mat.M) != 0;
             ctx->batch.push_back(std::move(sub));
         }
         ctx->batch_ref_ok = true;  // 32-bit byte offsets into every member's array
@@ -3943,7 +3944,7 @@ void batch_group_params(tsw_ctx *ctx, tsw_ctx::Group &G, bool corr, const std::v
                 sp.xtr = lanes_records<T>(sub, sp.nbands);
                 sp.abort_flag = abort_flag_of(ctx);  // a stall is reported (and the records refilled) by sync(ctx)
             }
-            const size_t b = split_sweep_lds_bytes<T>(g.p, G.rows, g.nx, sp.M);
+            const size_t b = split_sweep_lds_bytes<T>(g.p, G.rows, sp.M);
             require(b != 0, TSW_E_UNSUPPORTED, "lane-split batch group does not fit one CU's LDS");
             lds = std::max(lds, b);
         }
@@ -4070,6 +4071,52 @@ void lanes_batch_launch(tsw_ctx *ctx, size_t k, int threads, size_t lds, hipStre
     lanes_launch<T>(LG.p, rep, threads, lds, s, dp, LG.dev_items.as<int4>(), (int)LG.items.size());
 }
 
+// The items of a lane-split group (w: sorted (band, -work, slot, band * nq + ordinate)) as queues of the
+// persistent launch, one per XCD: runs of neighbouring ordinates of one member's quadrant (at most kQueueRun,
+// evenly split) go whole to the queue with the least work so far, heaviest members first, and each queue keeps
+// the band-major order.
+constexpr int kQueueRun = 12;
+void split_queues(tsw_ctx *ctx, tsw_ctx::Group &G, const std::vector<std::tuple<int, long long, int, int>> &w) {
+    std::vector<std::vector<int>> queue_of(G.members.size());  // per slot and ordinate
+    long long load[kXcds] = {};
+    for (const auto &t : w) {
+        if (std::get<0>(t) != 0) break;  // band 0 holds every (slot, ordinate) once, heaviest first
+        const int slot = std::get<2>(t), q = std::get<3>(t);
+        const Geom &g = ctx->batch[G.members[slot]]->g;
+        auto &qo = queue_of[slot];
+        if (qo.empty()) qo.assign(g.nq, -1);
+        if (qo[q] >= 0) continue;
+        int quad = 0;
+        while (quad < 3 && q >= g.quad_off[quad + 1]) ++quad;
+        const int q0 = g.quad_off[quad], n = g.quad_off[quad + 1] - q0, runs = (n + kQueueRun - 1) / kQueueRun;
+        const int run = (q - q0) * runs / n;
+        const int x = (int)(std::min_element(load, load + kXcds) - load);
+        for (int k = q0; k < q0 + n; ++k)
+            if ((k - q0) * runs / n == run) {
+                qo[k] = x;
+                load[x] -= std::get<1>(t);
+            }
+    }
+    std::vector<int> queue[kXcds];
+    for (const auto &t : w) {
+        const int slot = std::get<2>(t), v = std::get<3>(t);
+        auto &Q = queue[queue_of[slot][v % queue_of[slot].size()]];
+        Q.push_back(slot);
+        Q.push_back(v);
+    }
+    G.qitems.clear();
+    int table[kXcds + 1] = {0};
+    for (int x = 0; x < kXcds; ++x) {
+        G.qitems.insert(G.qitems.end(), queue[x].begin(), queue[x].end());
+        table[x + 1] = (int)G.qitems.size() / 2;
+    }
+    TSW_HIP(hipMemcpyAsync(G.dev_qitems.reserve(sizeof(int) * G.qitems.size()), G.qitems.data(),
+                           sizeof(int) * G.qitems.size(), hipMemcpyHostToDevice, ctx->stream));
+    TSW_HIP(hipMemcpyAsync(G.work.get(ctx->stream) + kSplitWorkTable, table, sizeof(table), hipMemcpyHostToDevice,
+                           ctx->stream));
+    TSW_HIP(hipStreamSynchronize(ctx->stream));  // table goes out of scope
+}
+
 // Launch groups of the members `members` by their engines: staggered groups by (DG degree, compute waves,
 // material path, layout), work items {member slot, ordinate} heaviest first; lane groups by DG degree, items
 // {member slot, ordinate block, band} band-major, heaviest members first within a band.
@@ -4107,7 +4154,6 @@ void build_batch_groups(tsw_ctx *ctx, const std::vector<int> &members) {
             G.mat = sub->mat.valid;
             G.ref = e == tsw_ctx::kEngRef || split;
             G.split = split;
-            if (split) G.work.reserve(sizeof(int));
         }
         auto &G = ctx->groups[it->second];
         G.members.push_back(b);
@@ -4152,6 +4198,7 @@ void build_batch_groups(tsw_ctx *ctx, const std::vector<int> &members) {
         }
         TSW_HIP(hipMemcpyAsync(G.dev_items.reserve(sizeof(int) * G.items.size()), G.items.data(),
                                sizeof(int) * G.items.size(), hipMemcpyHostToDevice, ctx->stream));
+        if (G.split) split_queues(ctx, G, w);
     }
     for (auto &LG : ctx->lane_groups) {
         std::vector<std::tuple<long long, int>> order;  // (-work, slot)
@@ -4212,12 +4259,17 @@ void batch_group_launch(tsw_ctx *ctx, tsw_ctx::Group &G, bool corr, const std::v
     rep.prefetch = ctx->prefetch_opt;
     if (G.split) {
         rep.split = 1;
-        rep.prefetch = ctx->batch_split_pf_opt > 0 ? ctx->batch_split_pf_opt : kSplitBatchPrefetch;
-        // persistent launch: the counter was zeroed on the context's stream before the fork
-        if (ctx->batch_persistent_opt > 0 && G.work.ptr) rep.work = G.work.as<int>();
+        rep.prefetch = split_prefetch<T>(ctx, G.p);
+        if (ctx->batch_persistent_opt > 0) {
+            rep.work = G.work.get(ctx->stream);
+            rep.work_set = G.work.set;
+            G.work.set ^= 1;
+        }
     }
-    launch_diag_sweep_batch<T>(rep, probs, G.dev_items.as<int2>(), (int)G.items.size() / 2,
-                               G.split ? G.rows : G.max_ny, lds, G.p, sd);
+    const bool queues = rep.work != nullptr;
+    launch_diag_sweep_batch<T>(rep, probs, queues ? G.dev_qitems.as<int2>() : G.dev_items.as<int2>(),
+                               (int)(queues ? G.qitems.size() : G.items.size()) / 2, G.split ? G.rows : G.max_ny, lds,
+                               G.p, sd);
 }
 
 // One batched sweep over the current groups, all on the side streams, timed as one sweep.  Converted
@@ -4268,7 +4320,7 @@ void batch_sweep(tsw_ctx *ctx, bool conv64, bool inplace64, bool corr, const std
             else lanes_batch_inflow<float>(ctx, j, ctx->stream);
         }
     for (auto &gd : diag)
-        if (gd.second) {
+        if (gd.second && !gd.first->split) {  // (the lane-split kernel reads the halos itself)
             if (inplace64) batch_group_inflow<double>(ctx, *gd.first);
             else batch_group_inflow<float>(ctx, *gd.first);
         }
@@ -4276,9 +4328,6 @@ void batch_sweep(tsw_ctx *ctx, bool conv64, bool inplace64, bool corr, const std
         if (lanes)
             for (auto &LG : ctx->lane_groups)
                 if (LG.work.ptr) TSW_HIP(hipMemsetAsync(LG.work.ptr, 0, sizeof(int), ctx->stream));
-        for (auto &gd : diag)
-            if (gd.first->split && gd.first->work.ptr)
-                TSW_HIP(hipMemsetAsync(gd.first->work.ptr, 0, sizeof(int), ctx->stream));
     }
     TSW_HIP(hipEventRecord(ctx->fork_ev, ctx->stream));
     int k = 0;

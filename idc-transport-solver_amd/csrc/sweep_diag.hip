@@ -16,33 +16,38 @@ TSW_SWEEP_EXTERN(float, 2)
 TSW_SWEEP_EXTERN(float, 3)
 TSW_SWEEP_EXTERN(float, 4)
 
-// LDS of the lane-split sweep for bands of BR rows (0: not built for (T, P) or too many rows)
+// LDS of the lane-split sweep for bands of BR rows(0: not built for (T, P) or
+// too many rows)
 template <typename T, int P>
-size_t split_lds_total(int BR, int nx, int M) {
+size_t split_lds_total(int BR, int M, bool ref) {
     if constexpr (!split_supported<T, P>()) {
         return 0;
     } else {
-        constexpr int LG = split_lanes<P>(), rpw = 64 / LG;
-        const int slots = (BR + rpw - 1) / rpw * rpw;
-        if (slots * LG > 512) return 0;
-        return SplitLds<T, P>(slots, nx, M).total;
+        const int threads = (split_lanes<P>() * BR + 63) / 64 * 64, slots = threads / split_lanes<P>();
+        if (slots > (ref ? split_max_slots<P, true>() : split_max_slots<P, false>())) return 0;
+        return ref ? SplitLds<T, P, true>(slots, M).total : SplitLds<T, P, false>(slots, M).total;
     }
 }
 
+// (the kernel's static LDS, the taken item, comes on top)
 template <typename T>
-size_t split_sweep_lds_bytes(int p, int rows, int nx, int M) {
+size_t split_lds_bytes(int p, int rows, int M, bool ref) {
     size_t total = 0;
     switch (p) {
-        case 1: total = split_lds_total<T, 2>(rows, nx, M); break;
-        case 2: total = split_lds_total<T, 3>(rows, nx, M); break;
-        case 3: total = split_lds_total<T, 4>(rows, nx, M); break;
+        case 1: total = split_lds_total<T, 2>(rows, M, ref); break;
+        case 2: total = split_lds_total<T, 3>(rows, M, ref); break;
+        case 3: total = split_lds_total<T, 4>(rows, M, ref); break;
         default: break;
     }
     const size_t bytes = total * sizeof(T);
-    return bytes <= max_lds_per_block() ? bytes : 0;
+    return bytes + 16 <= max_lds_per_block() ? bytes : 0;
 }
-template size_t split_sweep_lds_bytes<double>(int, int, int, int);
-template size_t split_sweep_lds_bytes<float>(int, int, int, int);
+template <typename T>
+size_t split_sweep_lds_bytes(int p, int rows, int M) {
+    return split_lds_bytes<T>(p, rows, M, true);
+}
+template size_t split_sweep_lds_bytes<double>(int, int, int);
+template size_t split_sweep_lds_bytes<float>(int, int, int);
 
 template <typename T>
 size_t diag_sweep_lds_bytes(const DiagSweepParams<T> &sp, int p) {
@@ -53,15 +58,7 @@ size_t diag_sweep_lds_bytes(const DiagSweepParams<T> &sp, int p) {
     if (sp.wave1 && BR > 64) return 0;
     if (sp.split) {
         if (!sp.ainv || sp.wave1) return 0;
-        size_t total = 0;
-        switch (p) {
-            case 1: total = split_lds_total<T, 2>(BR, sp.nx, sp.M); break;
-            case 2: total = split_lds_total<T, 3>(BR, sp.nx, sp.M); break;
-            case 3: total = split_lds_total<T, 4>(BR, sp.nx, sp.M); break;
-            default: break;
-        }
-        const size_t bytes = total * sizeof(T);
-        return bytes <= max_lds_per_block() ? bytes : 0;
+        return split_lds_bytes<T>(p, BR, sp.M, false);
     }
     const int cthreads = ((BR + 63) / 64) * 64;
     const int M = sp.ainv ? sp.M : 0;
@@ -128,6 +125,17 @@ void launch_diag_sweep_batch(const DiagSweepParams<T> &rep, const DiagSweepParam
         default: throw Error(TSW_E_UNSUPPORTED, "DG degree not built");
     }
 }
+template <typename T>
+void launch_split_ref(const DiagSweepParams<T> &sp, const SplitSources &src, int n, size_t lds, int p, hipStream_t s) {
+    switch (p) {
+        case 1: launch_split_ref_p<T, 2>(sp, src, n, lds, s); break;
+        case 2: launch_split_ref_p<T, 3>(sp, src, n, lds, s); break;
+        case 3: launch_split_ref_p<T, 4>(sp, src, n, lds, s); break;
+        default: throw Error(TSW_E_UNSUPPORTED, "lane-split sweep built for DG degrees 1-3");
+    }
+}
+template void launch_split_ref<double>(const DiagSweepParams<double> &, const SplitSources &, int, size_t, int, hipStream_t);
+template void launch_split_ref<float>(const DiagSweepParams<float> &, const SplitSources &, int, size_t, int, hipStream_t);
 template <typename T>
 void launch_diag_inflow_batch(const DiagSweepParams<T> *probs, int nprob, int p, hipStream_t s) {
     switch (p) {

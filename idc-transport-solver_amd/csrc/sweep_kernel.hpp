@@ -638,8 +638,8 @@ void launch_ds_d(const DiagSweepParams<T> &sp, size_t lds, hipStream_t s, const 
     const int rows = batch ? max_ny : band_rows_of(sp);
     if (sp.split) {
         if constexpr (MAT && split_supported<T, P>() && ((MODE & 4) == 0 || MODE == 5)) {
-            constexpr int LG = split_lanes<P>(), RPW = 64 / LG;  // lanes per row, rows per wavefront
-            const int threads = LG * ((rows + RPW - 1) / RPW * RPW);  // LG lanes for each row slot
+            // LG lanes for each row slot, in whole wavefronts, and the reference layout's storer waves
+            const int threads = (split_lanes<P>() * rows + 63) / 64 * 64 + ((MODE & 4) != 0 ? 64 * kSplitStorers : 0);
             if (threads > 512) throw Error(TSW_E_ARG, "lane-split sweep needs bands of at most 512 / lanes rows");
             if (batch) {
                 auto kern = k_diag_sweep_split<T, P, MODE, D, true>;
@@ -653,14 +653,14 @@ void launch_ds_d(const DiagSweepParams<T> &sp, size_t lds, hipStream_t s, const 
                     TSW_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
                     grid = std::max(1, std::min(nitems, std::max(per_cu, 1) * cus));
                 }
-                hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, s, sp, batch, items, sp.work, nitems);
+                hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, s, sp, batch, items, sp.work, sp.work_set);
             } else {
                 if constexpr ((MODE & 4) != 0) throw Error(TSW_E_ARG, "reference-layout lane-split sweep is built for batches");
                 auto kern = k_diag_sweep_split<T, P, MODE, D, false>;
                 if (lds > 64 * 1024)
                     TSW_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-                hipLaunchKernelGGL(kern, dim3(sp.nq * (sp.nbands > 1 ? sp.nbands : 1)), dim3(threads), lds, s, sp,
-                                   nullptr, nullptr, nullptr, 0);
+                hipLaunchKernelGGL(kern, dim3(sp.nq * (sp.nbands > 1 ? sp.nbands : 1)),
+                                   dim3(threads), lds, s, sp, nullptr, nullptr, nullptr, 0);
             }
             TSW_HIP(hipGetLastError());
             return;
@@ -752,6 +752,41 @@ void launch_diag_sweep_batch_p(const DiagSweepParams<T> &rep, const DiagSweepPar
     }
 }
 
+// Lane-split sweeps on the reference layout (launch_split_ref): persistent with sp.work, as many workgroups as
+// the device holds at once.
+template <typename T, int P>
+void launch_split_ref_p(const DiagSweepParams<T> &sp, const SplitSources &src, int n, size_t lds, hipStream_t s) {
+    if constexpr (split_supported<T, P>()) {
+        const int threads = (split_lanes<P>() * band_rows_of(sp) + 63) / 64 * 64 + 64 * kSplitStorers;
+        if (threads > 512 || !sp.ainv || n < 1 || n > kSplitSources || (sp.nbands > 1 && (!sp.xtr || !sp.abort_flag)))
+            throw Error(TSW_E_ARG, "lane-split reference-layout sweep: inconsistent launch");
+        const int items = n * sp.nq * (sp.nbands > 1 ? sp.nbands : 1);
+        auto go = [&](auto kern) {
+            if (lds > 64 * 1024)
+                TSW_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            int grid = items;
+            if (sp.work) {
+                int per_cu = 0, dev = 0, cus = 0;
+                TSW_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)kern, threads, lds));
+                TSW_HIP(hipGetDevice(&dev));
+                TSW_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+                grid = std::max(1, std::min(items, std::max(per_cu, 1) * cus));
+            }
+            hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, s, sp, src, n, sp.work, sp.work_set);
+            TSW_HIP(hipGetLastError());
+        };
+        switch (sp.prefetch) {
+            case 2: go(k_split_ref<T, P, 2>); break;
+            case 3: go(k_split_ref<T, P, 3>); break;
+            case 4: go(k_split_ref<T, P, 4>); break;
+            case 6: go(k_split_ref<T, P, 6>); break;
+            default: throw Error(TSW_E_ARG, "prefetch depth must be 2, 3, 4 or 6");
+        }
+    } else {
+        throw Error(TSW_E_ARG, "lane-split sweep not built for this precision and degree");
+    }
+}
+
 // Inflow traces of a batch's sources from their reference-layout halos, as launch_inflow computes them
 // for one problem: tin_x [nq][ny][P] from the x-inflow halo cell of each row, tin_y [nq][nx][P] from the
 // y-inflow halo cell of each column.  Member blockIdx.y; x strides over ordinates x rows (columns).
@@ -792,12 +827,14 @@ void launch_diag_inflow_batch_p(const DiagSweepParams<T> *batch, int nprob, hipS
 
 #define TSW_SWEEP_INSTANTIATE(T, P)                                                                         \
     template void launch_diag_inflow_batch_p<T, P>(const DiagSweepParams<T> *, int, hipStream_t);          \
+    template void launch_split_ref_p<T, P>(const DiagSweepParams<T> &, const SplitSources &, int, size_t, hipStream_t); \
     template void launch_diag_sweep_p<T, P>(const DiagSweepParams<T> &, size_t, hipStream_t);              \
     template void launch_diag_sweep_batch_p<T, P>(const DiagSweepParams<T> &, const DiagSweepParams<T> *,   \
                                                   const int2 *, int, int, size_t, hipStream_t);
 
 #define TSW_SWEEP_EXTERN(T, P)                                                                              \
     extern template void launch_diag_inflow_batch_p<T, P>(const DiagSweepParams<T> *, int, hipStream_t);   \
+    extern template void launch_split_ref_p<T, P>(const DiagSweepParams<T> &, const SplitSources &, int, size_t, hipStream_t); \
     extern template void launch_diag_sweep_p<T, P>(const DiagSweepParams<T> &, size_t, hipStream_t);       \
     extern template void launch_diag_sweep_batch_p<T, P>(const DiagSweepParams<T> &, const DiagSweepParams<T> *, \
                                                          const int2 *, int, int, size_t, hipStream_t);

@@ -1,26 +1,39 @@
-// Lane-split staggered sweep (k_diag_sweep_split), the material path with LG lanes per mesh row:
+// Lane-split staggered sweep (k_diag_sweep_split, k_split_ref), the material path with LG lanes per mesh row:
 // LG = 2 for P = 2 and 4 for P = 3, 4 (for P = 3 the fourth lane repeats the third and stores nothing).
 //
-// Lane g of row r owns the coefficients k = e + P*g (e < P) of the row's cell.  At a step it loads the
-// sources of its coefficients, forms their right-hand sides from the row's x-trace (held by every lane of
-// the row) and its own y-trace value, broadcasts them to the row's other lanes with DPP quad permutations,
-// applies its P rows of the element inverse to the whole right-hand side, stores its coefficients, and
-// gathers the row's solution back to form the outflow traces.  A wave then holds 16 rows instead of 64
-// and issues about 175 instructions per step instead of about 250 (FP32 Q2), and a band of 64 rows fills
-// four wavefronts, so an ordinate's sweep spreads over four times as many SIMDs.  Every value is computed by the same
-// operations, in the same order, as the material path of k_diag_sweep (sums of products are written as
-// explicit fused multiply-adds in both), so the two kernels give the same bits.
+// Lane g of row r owns the coefficients k = e + P*g (e < P) of the row's cell.  At a step it loads the sources of
+// its coefficients, forms their right-hand sides from the row's x-trace and its own y-trace value, broadcasts them
+// to the row's other lanes with DPP quad permutations, applies its P rows of the element inverse to the whole
+// right-hand side and leaves its coefficients in LDS, from which the row's lanes form the x-trace of the next step
+// and the row above its y-trace.  A band of 64 rows fills four wavefronts at degrees 2 and 3, so an ordinate's sweep
+// spreads over four times as many SIMDs as with a lane per row.  Every value is computed by the same operations, in
+// the same order, as the material path of k_diag_sweep (sums of products are written as explicit fused multiply-adds
+// in both), so the two kernels give the same bits.
 //
-// Bands, exchange records, prefetch ring and the wave-uniform skip of diagonals without a cell follow
-// k_diag_sweep; stores are direct (no storer wave), and the band's first and last rows consume and fill
-// the exchange records themselves, as the one-wave variant does.
+// Bands and exchange records follow k_diag_sweep; the band's first and last rows consume and fill the records
+// themselves, as its one-wave variant does.  A wave works only on the steps at which one of its rows has a cell.
 //
-// MODE bit 4 (with bit 1, sources only): the source is read from `qref` and psi written to `psi_ref`, both in
-// the reference layout [i][j][q][d][e], where lane g's coefficients are one contiguous run of P doubles
-// (16-byte accesses, and an 8-byte one for odd P) and the LG lanes of a row cover the cell's run, so no layout
-// conversion is needed and a wavefront's accesses are RPW whole cell runs.  BATCH: the workgroup's
-// parameters are batch[items[b].x], and items[b].y = band * nq + ordinate, numbered band-major so that a
-// band's upstream band is always dispatched first; items with a negative problem index are padding.
+// MODE bit 4 (with bit 1, sources only): the source is read from `qref` and psi written to `psi_ref`, both in the
+// reference layout [i][j][q][d][e], and the inflow is read from the halo cells of qref, so no layout conversion and
+// no launch for the traces is needed.  Lane g's coefficients are one contiguous run of P doubles there, and the LG
+// lanes of a row cover the cell's run.  Two further waves (kSplitStorers) write the results.
+// BATCH: the workgroup's parameters are batch[items[b].x], and items[b].y = band * nq + ordinate, numbered band-major
+// so that a band's upstream band is always dispatched first; items with a negative problem index are padding.
+//
+// What bounds the reference layout (Q2 S12 on 280 x 280, 561 steps a workgroup, FP64, kernel time): not HBM, which
+// would take 190 us, nor the arithmetic of the chain of steps (290 us with the loads and stores taken out), but the
+// memory instructions' way through the address unit and the L1 between a step's barriers: each takes 16 cycles
+// whatever its width, a load of 16 rows' 72-byte runs about 50 from the L2, and a store about 5 cycles per 64-byte
+// segment that it touches.  Against 527 us for stores by the compute lanes (each segment in two or three pieces) and
+// items in plain order:
+//   - one L2 sees the whole cache lines of neighbouring ordinates (take_item): less HBM traffic, and loads from the
+//     L2 instead of behind it;
+//   - stores as whole runs, read back from LDS by two storer waves a step later: 472 us; by the compute lanes
+//     themselves 489 us, by one storer wave 514 us;
+//   - the x-trace from LDS instead of 18 DPP moves, no address arithmetic in the step, idle waves only at barriers.
+// Two or four ordinates side by side in a workgroup (whole lines per access, shorter bands) took 490 to 530 us, all
+// memory instructions in two memory waves 706 us.  Other kernels, before and after: Q1 280 x 280 250 -> 215 us; Q2
+// 32 x 32 53 -> 39, 128 x 128 172 -> 145; Q3 32 x 32 97 -> 61, 128 x 128 270 -> 223, 256 x 256 667 -> 461 us.
 #pragma once
 
 namespace tsw {
@@ -37,19 +50,32 @@ __host__ __device__ constexpr bool split_supported() {
     return P >= 2 && P <= 4 && P * P * P * (int)sizeof(T) <= 64 * 8;
 }
 
-template <typename T, int P>
+template <typename T, int P, bool REF>
 struct SplitLds {  // LDS carve-up in units of T, 16-byte aligned arrays and rows
     static constexpr int N = P * P;
     static constexpr int PS = vround<T>(P), RS = vround<T>(P * N);
-    size_t ex, in, inv, total;
-    // slots: row slots of the workgroup; M: materials ([M][P][RS] inverse rows, lane g's block at g)
-    __host__ __device__ SplitLds(int slots, int nx, int M) {
-        ex = 0;                               // [2][slots][PS] y-traces between rows
-        in = ex + (size_t)2 * slots * PS;     // [nx][PS] y-inflow traces of row 0
-        inv = in + (size_t)nx * PS;           // [M][P][RS]
+    // row stride of the solved cells: P runs of PS values, and a 16-byte pad where P runs are a multiple of
+    // 128 bytes, so that a wave's rows do not all start in one LDS bank
+    static constexpr int XS = P * PS + (P * PS * (int)sizeof(T) % 128 == 0 ? Vec16<T>::W : 0);
+    static constexpr int YR = 64 / split_lanes<P>();  // columns of the y-inflow ring: the rows of a wave
+    size_t ex, xs, lin, inv, total;
+    // slots: row slots of the workgroup; M: materials ([M][P][RS] inverse rows, lane g's block at g).  The
+    // reference layout keeps the solved cells of two steps ([2][slots][XS]): the rows above take their
+    // y-traces, and the storer wave the results, from the last step's
+    __host__ __device__ SplitLds(int slots, int M) {
+        ex = 0;                                                 // [slots][2][PS] y-traces between rows, by step parity
+        xs = ex + (REF ? 0 : (size_t)2 * slots * PS);           // [slots][XS] solved cells, for the rows' x-traces
+        lin = xs + (size_t)(REF ? 2 : 1) * slots * XS;          // [YR][PS] y-inflow traces of row 0 (reference layout)
+        inv = lin + (REF ? (size_t)YR * PS : 0);                // [M][P][RS]
         total = inv + (size_t)M * P * RS;
     }
 };
+// Storer waves of a reference-layout workgroup, and the most row slots of a workgroup of 512 threads.
+constexpr int kSplitStorers = 2;
+template <int P, bool REF>
+__host__ __device__ constexpr int split_max_slots() {
+    return (512 - (REF ? 64 * kSplitStorers : 0)) / split_lanes<P>();
+}
 
 // v read from lane K of its LG-lane group (quad permutation; K is a constant after unrolling)
 template <int LG>
@@ -107,15 +133,34 @@ __device__ __forceinline__ void ref_run_st(__amdgpu_buffer_rsrc_t r, unsigned of
     if constexpr (P % 2 != 0) buf_st<double>(r, off, 8 * (P - 1), (double)v[P - 1]);
 }
 
+// Waits until the exchange record value *rec (already loaded once into v) is filled; on the spin limit, or
+// when another band has given up (*abort_flag), returns zero and the caller proceeds.
+template <typename T>
+__device__ __forceinline__ typename ExchangeSentinel<T>::U wait_value(gptr<const typename ExchangeSentinel<T>::U> rec,
+                                                                      typename ExchangeSentinel<T>::U v,
+                                                                      gptr<int> abort_flag) {
+    using U = typename ExchangeSentinel<T>::U;
+#pragma unroll 1
+    for (int it = 0; v == ExchangeSentinel<T>::bits; ++it) {
+        if (it >= kSpinLimit || ((it & 255) == 255 && xload<int>(abort_flag) != 0)) {
+            if (it >= kSpinLimit) xstore<int>(abort_flag, 1);
+            return 0;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        v = xload<U>(rec);
+    }
+    return v;
+}
+
 // One item of the lane-split sweep: band wid / nq of ordinate wid % nq of the problem sp, by the whole
 // workgroup (every thread calls it; it ends with a workgroup barrier).
 template <typename T, int P, int MODE, int D>
 __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigned wid) {
     constexpr int N = P * P, LG = split_lanes<P>(), RPW = 64 / LG;  // rows per wavefront
-    using Lds = SplitLds<T, P>;
-    constexpr int PS = Lds::PS, RS = Lds::RS;
-    using U = typename ExchangeSentinel<T>::U;
     constexpr bool HASQ = (MODE & 1) != 0, HASPHI = (MODE & 2) != 0, REF = (MODE & 4) != 0;
+    using Lds = SplitLds<T, P, REF>;
+    constexpr int PS = Lds::PS, RS = Lds::RS, XS = Lds::XS;
+    using U = typename ExchangeSentinel<T>::U;
     static_assert(!REF || MODE == 5, "reference-layout lane-split sweep: sources only");
     using PQ = typename std::conditional<REF, double, T>::type;  // prefetched source (converted at use)
     const int nb = sp.nbands < 2 ? 1 : sp.nbands;
@@ -127,14 +172,11 @@ __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigne
     const int BR = nb > 1 ? sp.band_rows : ny;
     const int R0 = band * BR;
     const int nrows = BR < ny - R0 ? BR : ny - R0;
-    const int slots = (int)blockDim.x / LG;
-    const Lds L(slots, nx, sp.M);
-    T *ex = lds + L.ex, *lin = lds + L.in, *linv = lds + L.inv;
+    const int slots = ((int)blockDim.x - (REF ? 64 * kSplitStorers : 0)) / LG;
+    const Lds L(slots, sp.M);
+    T *linv = lds + L.inv;
     const DiagMap dm{nx, ny};
     const size_t ncell = (size_t)dm.cells();
-    const gptr<U> xin = (nb > 1 && band > 0) ? G(reinterpret_cast<U *>(sp.xtr)) + ((size_t)q * (nb - 1) + band - 1) * nx * P : nullptr;
-    const gptr<U> xout = (nb > 1 && band < nb - 1) ? G(reinterpret_cast<U *>(sp.xtr)) + ((size_t)q * (nb - 1) + band) * nx * P : nullptr;
-
     const int Q = q >= sp.qo3 ? 3 : (q >= sp.qo2 ? 2 : (q >= sp.qo1 ? 1 : 0));
     const int tid = threadIdx.x;
     const T xi = G(sp.xi)[q], eta = G(sp.eta)[q];
@@ -145,75 +187,147 @@ __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigne
         const int m = k / (N * N), e = k - m * N * N, row = e / N, col = e - row * N;
         linv[((size_t)m * P + row / P) * RS + (row % P) * N + col] = G(sp.ainv)[((size_t)m * sp.nq + q) * N * N + e];
     }
-    if (band == 0)
-        for (int k = tid; k < nx * P; k += blockDim.x) {
-            const int c = k / P, d = k - c * P;
-            lin[(size_t)c * PS + d] = sp.tin_y ? G(sp.tin_y)[(size_t)q * nx * P + k] : T(0);
+
+    // Wave w holds row slots [w RPW, (w + 1) RPW) and works on its own steps t = 0 .. live_n - 1 (row rw of the
+    // wave solves column t - rw), starting w RPW barriers after the workgroup's first step; every wave passes
+    // nbar barriers in all.
+    const int rw = (tid & 63) / LG, g = tid % LG;
+    const int w0 = __builtin_amdgcn_readfirstlane(tid >> 6) * RPW;  // first row slot of this wave
+    auto run_of = [&](int first) {  // steps of the wave at row `first`, rounded up to whole rings
+        const int n = nrows - first < RPW ? nrows - first : RPW;
+        return n > 0 ? (n - 1 + nx + D - 1) / D * D : 0;
+    };
+    const int last0 = (nrows - 1) / RPW * RPW;
+    int nbar = last0 + run_of(last0);
+    if (last0 > 0 && last0 - RPW + run_of(last0 - RPW) > nbar) nbar = last0 - RPW + run_of(last0 - RPW);
+    const int nrun = run_of(w0);
+    const unsigned long long ref_bytes = REF ? (unsigned long long)(nx + 2) * (ny + 2) * sp.nq * N * 8 : 0;
+    const unsigned dstep = REF ? (unsigned)((xneg ? -1LL : 1LL) * (ny + 2) * sp.nq * N * 8) : 0;  // one column on
+    // stores of lanes without a cell go to this offset, past the end of the buffer, where they are dropped: a
+    // store then always issues, and the waits for the loads behind it count it (behind a branch it might not,
+    // and each wait would also cover the loads of one or two later steps)
+    const unsigned long long nplanes = (unsigned long long)N * ncell * sizeof(T);  // bytes of one ordinate
+    const unsigned nowhere = REF ? (unsigned)ref_bytes : (unsigned)nplanes;
+    const __amdgpu_buffer_rsrc_t rout = REF ? buf_rsrc(sp.psi_ref, ref_bytes) : buf_rsrc(sp.psi + (size_t)q * N * ncell, nplanes);
+
+    if (REF && w0 >= slots) {
+        // The storer waves: step t's cells during step t + 1, from LDS, as the band's runs one after the other
+        // (access m of lane l, m dealt round the storers, is values (l + 64 m) SW of them).  A 64-byte segment of L2
+        // takes a write request of its own, about one in 4 cycles per CU: written by the compute lanes, a cell's run
+        // goes out in pieces, each segment in two requests or more, and the compute waves wait for the queue.
+        constexpr int SW = P % 2 == 0 ? 2 : 1, SM = (split_max_slots<P, true>() * N / SW + 64 * kSplitStorers - 1) / (64 * kSplitStorers);
+        int lane = tid & 63;
+        asm volatile("" : "+v"(lane));  // (keeps these tables out of the compute waves' registers)
+        const int m0 = __builtin_amdgcn_readfirstlane((tid >> 6) - slots * LG / 64);
+        unsigned soff[SM];   // byte offset of step t's cell
+        int c0[SM], at[SM];  // its column is t - c0 (far outside the mesh past the band's rows), its LDS offset
+#pragma unroll
+        for (int m = 0; m < SM; ++m) {
+            const int e = (lane + 64 * (m * kSplitStorers + m0)) * SW, row = e / N, k = e - row * N;
+            const bool ok = row < nrows;
+            c0[m] = ok ? row : (1 << 30);
+            at[m] = ok ? row * XS + k / P * PS + k % P : 0;
+            soff[m] = ref_off(0, R0 + (ok ? row : 0), nx, ny, sp.nq, q, N, xneg, yneg) + 8u * (unsigned)k - (unsigned)c0[m] * dstep;
         }
+        lds_barrier();
+        for (int t = 0; t < nbar; ++t) {
+            lds_barrier();
+            const T *xt = lds + L.xs + (t & 1) * slots * XS;
+            T v[SM][SW];
+#pragma unroll
+            for (int m = 0; m < SM; ++m)
+#pragma unroll
+                for (int k = 0; k < SW; ++k) v[m][k] = xt[at[m] + k];
+#pragma unroll
+            for (int m = 0; m < SM; ++m) {
+                if (64 * (m * kSplitStorers + m0) * SW < nrows * N)  // wave-uniform
+                    ref_run_st<T, SW>(rout, (unsigned)(t - c0[m]) < (unsigned)nx ? soff[m] : nowhere, v[m]);
+                soff[m] += dstep;
+            }
+        }
+        return;
+    }
 
-    const int steps = nx + nrows - 1;
-    const int nsteps = ((steps + D - 1) / D) * D;
-    const unsigned plane = (unsigned)(ncell * sizeof(T));
-    const DiagWalk walk0{R0, (int)(dm.base(R0) - dm.rlo(R0))};
-
-    const int rl = tid / LG, g = tid % LG;
+    const int rl = w0 + rw;
     const int dd = g < P ? g : P - 1;  // the x-degree whose coefficients this lane owns
     const bool owner = g < P;
-    const int r = R0 + rl;
     const bool row_ok = rl < nrows;
-    T tx[P];
+    const int rc = row_ok ? rl : nrows - 1;  // slots past the band's rows load its last row and store nothing
+    const int r = R0 + rc;
+    const int ra = row_ok ? rw : (1 << 30);  // column at step t is t - ra: never inside the mesh without a row
+    T tx;  // x-trace of y-degree dd: the inflow, then the outflow of the row's last cell
+    if constexpr (REF) {
+        const gptr<const double> h = G(sp.qref) + (((size_t)(xneg ? nx + 1 : 0) * (ny + 2) + (yneg ? ny - r : r + 1)) * sp.nq + q) * N + dd;
+        double s = h[0];
 #pragma unroll
-    for (int d = 0; d < P; ++d) tx[d] = (row_ok && sp.tin_x) ? G(sp.tin_x)[((size_t)q * ny + r) * P + d] : T(0);
+        for (int a = 1; a < P; ++a) s += (xneg && (a & 1)) ? -h[P * a] : h[P * a];
+        tx = T(s);
+    } else {
+        tx = (row_ok && sp.tin_x) ? G(sp.tin_x)[((size_t)q * ny + r) * P + dd] : T(0);
+    }
 
-    const unsigned long long nplanes = (unsigned long long)N * plane;
+    // global addresses.  Diagonal layout: lane offset (row, first plane) plus a scalar offset (diagonal,
+    // plane); off(s) + r stays inside the array on every diagonal s of the mesh, whatever the row.
+    // Reference layout: the lane's byte offset of its run, moved by one column a step while inside the mesh.
+    const unsigned plane = (unsigned)(ncell * sizeof(T));
     const unsigned dplane = (unsigned)(dd * P) * plane;  // byte offset of this lane's first plane (< N * plane)
-    const unsigned long long ref_bytes = REF ? (unsigned long long)(nx + 2) * (ny + 2) * sp.nq * N * 8 : 0;
-    const unsigned dref = 8u * (unsigned)(dd * P);  // byte offset of this lane's run within a cell's run
     const __amdgpu_buffer_rsrc_t rq = REF ? buf_rsrc(sp.qref, ref_bytes)
                                           : buf_rsrc(HASQ ? sp.qsrc + (size_t)q * N * ncell : nullptr, HASQ ? nplanes : 0);
-    const __amdgpu_buffer_rsrc_t rout = REF ? buf_rsrc(sp.psi_ref, ref_bytes) : buf_rsrc(sp.psi + (size_t)q * N * ncell, nplanes);
-    DiagWalk cw = walk0;
     const __amdgpu_buffer_rsrc_t rphi = buf_rsrc(HASPHI ? sp.phi + (size_t)Q * N * ncell : nullptr, HASPHI ? nplanes : 0);
     const __amdgpu_buffer_rsrc_t rsigs = buf_rsrc(HASPHI ? sp.sig_s + (size_t)Q * ncell : nullptr, HASPHI ? plane : 0);
     const __amdgpu_buffer_rsrc_t rmat = buf_rsrc(sp.mat + (size_t)Q * ncell, ncell * 4);
-    const int w0 = __builtin_amdgcn_readfirstlane((tid & ~63) / LG);  // first row slot of this wave
-    const int live_n = w0 < nrows ? (nrows - 1 - w0 < RPW - 1 ? nrows - 1 - w0 : RPW - 1) + nx : 0;
-    const bool xwave = xin != nullptr && w0 == 0;
-    const bool xrow = xwave && rl == 0;
+    const unsigned dref = 8u * (unsigned)(dd * P);  // byte offset of this lane's run within a cell's run
+    const unsigned vrow0 = (unsigned)r * (unsigned)sizeof(T), vrow = vrow0 + dplane;
+    const unsigned vmat = (unsigned)r * 4u;
+    unsigned foff = REF ? ref_off(0, r, nx, ny, sp.nq, q, N, xneg, yneg) + dref : 0;  // run of the next fetch
+    const int s_last = nx + ny - 2;
+    DiagWalk fw{R0 + w0, (int)(dm.base(R0 + w0) - dm.rlo(R0 + w0))};  // diagonal of the next fetch
+    DiagWalk cw{fw.s - 1, fw.s > 0 ? (int)(dm.base(fw.s - 1) - dm.rlo(fw.s - 1)) : 0};  // diagonal of the last step
+    // exchange records: read from the band below (xin), written for the band above (xout)
+    const gptr<U> xtr = G(reinterpret_cast<U *>(sp.xtr)) + ((size_t)q * (nb - 1) + band) * nx * P;
+    const bool has_in = band > 0, has_out = band < nb - 1;
+    const gptr<U> xin = xtr - (size_t)nx * P, xout = xtr;
+    // y-inflow of the band's first row, column by column: the records of the band below, or the halo traces
+    // (the reference layout takes the latter from the halo cells themselves, through the LDS ring `lin`)
+    const gptr<const U> yin = has_in ? gptr<const U>(xin) : G(reinterpret_cast<const U *>(sp.tin_y)) + (size_t)q * nx * P;
+    const bool first = w0 == 0, ywave = first && (has_in || (!REF && sp.tin_y != nullptr));
+    const bool xrow = has_in && rl == 0;  // consumes the records of the band below
+    // reference layout, band 0: lane (rw, g) of the first wave loads the run of column c0 + rw's y-inflow halo
+    // cell, RPW columns ahead of their use
+    const bool yhalo = REF && first && band == 0;
+    double yr[REF ? P : 1];
+    auto yfetch = [&](int c0) {
+        if constexpr (REF) {
+            const int c = c0 + rw < nx ? c0 + rw : nx - 1, i = xneg ? nx - c : c + 1, j = yneg ? ny + 1 : 0;
+            ref_run_ld<P>(rq, (unsigned)((((long long)i * (ny + 2) + j) * sp.nq + q) * N * 8) + dref, yr);
+        }
+    };
+    const bool lastrow = has_out && owner && rl == nrows - 1;
 
     PQ pq[D][HASQ ? P : 1];
     T pf[D][HASPHI ? P : 1], ps[D];
     int pm[D];
     U px[D];
-    DiagWalk fw = walk0;
     int ft = 0;
     auto fetch = [&](int u) {
-        const bool live = ft < steps;
-        const int lo = live ? (fw.s - nx + 1 > R0 ? fw.s - nx + 1 : R0) : 0;
-        const int hi = live ? (fw.s < R0 + nrows - 1 ? fw.s : R0 + nrows - 1) : 0;
-        const int rc = r < lo ? lo : (r > hi ? hi : r);
-        const unsigned p = (unsigned)((live ? fw.off : 0) + rc);
-        const unsigned bt = p * (unsigned)sizeof(T), bi = p * 4u;
-        if constexpr (REF) {  // the cell (clamped into the mesh on padded steps) in the reference layout
-            const int cl = fw.s - rc < 0 ? 0 : (fw.s - rc >= nx ? nx - 1 : fw.s - rc);
-            ref_run_ld<P>(rq, ref_off(cl, rc, nx, ny, sp.nq, q, N, xneg, yneg) + dref, pq[u]);
+        const unsigned so = (unsigned)fw.off * (unsigned)sizeof(T), sm = (unsigned)fw.off * 4u;
+        if constexpr (REF) {
+            ref_run_ld<P>(rq, foff, pq[u]);
+            foff += (unsigned)(ft - ra) < (unsigned)(nx - 1) ? dstep : 0u;
         } else if (HASQ) {
 #pragma unroll
-            for (int e = 0; e < P; ++e) pq[u][e] = buf_ld<T>(rq, bt + dplane, e * plane);
+            for (int e = 0; e < P; ++e) pq[u][e] = buf_ld<T>(rq, vrow, so + e * plane);
         }
         if (HASPHI) {
 #pragma unroll
-            for (int e = 0; e < P; ++e) pf[u][e] = buf_ld<T>(rphi, bt + dplane, e * plane);
-            ps[u] = buf_ld<T>(rsigs, bt, 0);
+            for (int e = 0; e < P; ++e) pf[u][e] = buf_ld<T>(rphi, vrow, so + e * plane);
+            ps[u] = buf_ld<T>(rsigs, vrow0, so);
         }
-        pm[u] = buf_ld<int>(rmat, bi, 0);
-        if (xwave && ft < nx) px[u] = xload<U>(xin + (size_t)ft * P + dd);
-        fw.next(nx, ny);
+        pm[u] = buf_ld<int>(rmat, vmat, sm);
+        if (ywave && ft < nx) px[u] = xload<U>(yin + (size_t)ft * P + dd);
+        if (fw.s < s_last) fw.next(nx, ny);
         ++ft;
     };
-#pragma unroll
-    for (int u = 0; u < D; ++u) fetch(u);
-    lds_barrier();
 
     T Arow[P * N];  // rows dd*P .. dd*P + P-1 of the current material's dx dy A^{-1}
     int cur_mat = -1;
@@ -229,122 +343,217 @@ __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigne
     }
     T sx = xneg ? T(-1) : T(1), sy = yneg ? T(-1) : T(1);
     asm volatile("" : "+v"(sx), "+v"(sy));
-    for (int t0 = 0; t0 < nsteps; t0 += D) {
+    // LDS: the row below's y-trace (diagonal layout) or its cell's coefficients of this lane's x-degree
+    // (reference layout), and the row's own cell, of the last step; where this step's go
+    const int side = REF ? slots * XS : PS;  // between the two steps' copies
+    const int sb = rl > 0 ? rl - 1 : 0;  // the row below
+    const T *exr = REF ? lds + L.xs + (size_t)sb * XS + dd * PS : lds + L.ex + (size_t)sb * 2 * PS + dd;
+    T *exw = lds + L.ex + (size_t)rl * 2 * PS + dd;
+    const T *xsr = lds + L.xs + (size_t)rl * XS + dd;
+    T *xsw = lds + L.xs + (size_t)rl * XS + dd * PS;
+    auto y_trace = [&](const T (&c)[P]) {  // outflow y-trace of one x-degree: sum_b sy^b psi(d, b)
+        T v = c[0];
+#pragma unroll
+        for (int b = 1; b < P; ++b) v = (b & 1) ? v + sy * c[b] : v + c[b];
+        return v;
+    };
+    T *lin = lds + L.lin + dd;
+    T xo[P];  // this lane's coefficients of the last solved cell
+#pragma unroll
+    for (int e = 0; e < P; ++e) xo[e] = T(0);
+    bool act = false;  // the last step solved a cell in this lane's row
+
+    // results of the last step to memory (diagonal layout; cw stands at its diagonal)
+    auto store_last = [&]() {
+        if constexpr (!REF) {
+            const unsigned so = (unsigned)cw.off * (unsigned)sizeof(T), vo = act && owner ? vrow : nowhere;
+#pragma unroll
+            for (int e = 0; e < P; ++e) buf_st<T>(rout, vo, so + e * plane, xo[e]);
+            if (cw.s < s_last) cw.next(nx, ny);
+        }
+    };
+
+    if (nrun > 0) {
+        if (yhalo) yfetch(0);
+#pragma unroll
+        for (int u = 0; u < D - 1; ++u) fetch(u);
+    }
+    for (int k = 0; k <= w0 && k <= nbar; ++k) lds_barrier();  // the first one publishes the inverse table
+    for (int t0 = 0; t0 < nrun; t0 += D) {
 #pragma unroll
         for (int u = 0; u < D; ++u) {
             const int t = t0 + u;
-            const int c = t - rl;
-            const bool active = row_ok && (unsigned)c < (unsigned)nx;
-            const bool live = (unsigned)(t - w0) < (unsigned)live_n;
-            if (live) {
-                const int cc = c < 0 ? 0 : (c >= nx ? nx - 1 : c);
-                T ty = rl == 0 ? lin[(size_t)cc * PS + dd] : ex[((size_t)((t - 1) & 1) * slots + (rl - 1)) * PS + dd];
-                if (pm[u] != cur_mat) {
-                    cur_mat = pm[u];
-                    lds_get<T, P * N>(linv + ((size_t)cur_mat * P + dd) * RS, Arow);
-                }
-                if (xwave) {
-                    if (xrow && active && px[u] == ExchangeSentinel<T>::bits) {
-                        Record<U, 1> rec{{px[u]}};
-                        px[u] = wait_record<T, 1>(xin + (size_t)c * P + dd, rec, G(sp.abort_flag)).v[0];
-                    }
-                    ty = xrow ? (active ? from_bits<T>(px[u]) : T(0)) : ty;
-                }
-                T Bo[P];  // right-hand side of coefficients e + P dd
+            const int pr = D % 2 == 0 ? (u + 1) & 1 : (t + 1) & 1;  // LDS side of the last step
+            // the traces the cell needs come through LDS; meanwhile the last step's cell goes out and the ring
+            // slot it freed is refilled
+            T yv[P], xv[P];
+            if constexpr (REF) lds_get<T, P>(exr + pr * side, yv);
+            else yv[0] = exr[pr * side];
 #pragma unroll
-                for (int e = 0; e < P; ++e) {
-                    T a;
-                    if (HASPHI) {
-                        const T wsc = T(1) * ps[u] * T(kInv4Pi);
-                        a = HASQ ? fmadd(wsc, pf[u][e], T(pq[u][e])) : wsc * pf[u][e];
-                    } else {
-                        a = T(pq[u][e]);
-                    }
-                    Bo[e] = fmadd(kye[e], ty, fmadd(kxo, tx[e], a));
-                }
-                T B[N];
+            for (int d = 0; d < P; ++d) xv[d] = xsr[(REF ? pr * side : 0) + d * PS];
+            __builtin_amdgcn_sched_barrier(0);
+            store_last();
+            fetch((u + D - 1) % D);
+            __builtin_amdgcn_sched_barrier(0);
+            T v = xv[0];  // outflow x-trace: sum_a sx^a psi(a, dd)
 #pragma unroll
-                for (int d = 0; d < P; ++d)
-#pragma unroll
-                    for (int e = 0; e < P; ++e) B[e + P * d] = group_bcast<LG>(Bo[e], d);
-                T xo[P];
-#pragma unroll
-                for (int e = 0; e < P; ++e) {
-                    T acc = Arow[e * N] * B[0];
-#pragma unroll
-                    for (int col = 1; col < N; ++col) acc = fmadd(Arow[e * N + col], B[col], acc);
-                    xo[e] = acc;
-                }
-                if (active && owner) {
-                    if constexpr (REF) {
-                        ref_run_st<T, P>(rout, ref_off(c, r, nx, ny, sp.nq, q, N, xneg, yneg) + dref, xo);
-                    } else {
-                        const unsigned boff = (unsigned)(cw.off + r) * (unsigned)sizeof(T) + dplane;
-#pragma unroll
-                        for (int e = 0; e < P; ++e) buf_st<T>(rout, boff, e * plane, xo[e]);
-                    }
-                }
-                T x[N];
-#pragma unroll
-                for (int d = 0; d < P; ++d)
-#pragma unroll
-                    for (int e = 0; e < P; ++e) x[e + P * d] = group_bcast<LG>(xo[e], d);
-#pragma unroll
-                for (int e = 0; e < P; ++e) {  // outflow x-trace: sum_a sx^a psi(a, e)
-                    T v = x[e];
-#pragma unroll
-                    for (int a = 1; a < P; ++a) v = (a & 1) ? v + sx * x[e + P * a] : v + x[e + P * a];
-                    tx[e] = active ? v : tx[e];
-                }
-                T tyo = xo[0];  // outflow y-trace of x-degree dd: sum_b sy^b psi(dd, b)
-#pragma unroll
-                for (int b = 1; b < P; ++b) tyo = (b & 1) ? tyo + sy * xo[b] : tyo + xo[b];
-                ex[((size_t)(t & 1) * slots + rl) * PS + dd] = tyo;
-                if (xout && rl == nrows - 1 && active && owner) xstore(xout + (size_t)c * P + dd, to_bits(tyo));
-                if (xrow && active && owner) xstore(xin + (size_t)c * P + dd, ExchangeSentinel<T>::bits);
+            for (int a = 1; a < P; ++a) v = (a & 1) ? v + sx * xv[a] : v + xv[a];
+            tx = act ? v : tx;
+            T ty = REF ? y_trace(yv) : yv[0];
+            act = (unsigned)(t - ra) < (unsigned)nx;
+            if (pm[u] != cur_mat && act) {
+                cur_mat = pm[u];
+                lds_get<T, P * N>(linv + ((size_t)cur_mat * P + dd) * RS, Arow);
             }
-            cw.next(nx, ny);
-            __builtin_amdgcn_sched_barrier(0);
-            fetch(u);
-            __builtin_amdgcn_sched_barrier(0);
+            if (first) {
+                U y = 0;
+                if (REF && yhalo) {
+                    if (t % RPW == 0) {  // the next RPW columns' traces
+                        double s = yr[0];
+#pragma unroll
+                        for (int b = 1; b < (REF ? P : 1); ++b) s += (yneg && (b & 1)) ? -yr[b] : yr[b];
+                        lin[rw * PS] = T(s);
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+                        yfetch(t + RPW);
+                    }
+                    y = to_bits(lin[t % RPW * PS]);
+                } else if (ywave) {
+                    if (xrow && act) {
+                        px[u] = wait_value<T>(xin + (size_t)t * P + dd, px[u], G(sp.abort_flag));
+                        if (owner) xstore(xin + (size_t)t * P + dd, ExchangeSentinel<T>::bits);
+                    }
+                    y = px[u];
+                }
+                ty = rl == 0 ? (act ? from_bits<T>(y) : T(0)) : ty;
+            }
+            T Bo[P];  // right-hand side of coefficients e + P dd
+#pragma unroll
+            for (int e = 0; e < P; ++e) {
+                T a;
+                if (HASPHI) {
+                    const T wsc = T(1) * ps[u] * T(kInv4Pi);
+                    a = HASQ ? fmadd(wsc, pf[u][e], T(pq[u][e])) : wsc * pf[u][e];
+                } else {
+                    a = T(pq[u][e]);
+                }
+                Bo[e] = fmadd(kye[e], ty, fmadd(kxo, group_bcast<LG>(tx, e), a));
+            }
+            T B[N];
+#pragma unroll
+            for (int d = 0; d < P; ++d)
+#pragma unroll
+                for (int e = 0; e < P; ++e) B[e + P * d] = group_bcast<LG>(Bo[e], d);
+#pragma unroll
+            for (int e = 0; e < P; ++e) {
+                T acc = Arow[e * N] * B[0];
+#pragma unroll
+                for (int col = 1; col < N; ++col) acc = fmadd(Arow[e * N + col], B[col], acc);
+                xo[e] = acc;
+            }
+            if constexpr (!REF) exw[(1 - pr) * side] = y_trace(xo);
+            lds_put<T, P>(xsw + (REF ? (1 - pr) * side : 0), xo);
+            if (lastrow && act) xstore(xout + (size_t)(t - ra) * P + dd, to_bits(y_trace(xo)));
             lds_barrier();
         }
     }
+    if (nrun > 0) store_last();
+    for (int k = w0 + nrun; k < nbar; ++k) lds_barrier();
+}
+
+// Work counters of a persistent launch: two sets of one counter per XCD, each in a cache line of its own;
+// a launch takes items with one set and clears the other for the next launch.  Batch launches add the item
+// range of each XCD's queue.
+constexpr int kWorkStride = 16, kWorkSet = kXcds * kWorkStride, kWorkTable = kSplitWorkTable;
+static_assert(kWorkTable == 2 * kWorkSet, "two sets of counters before the table");
+
+// The next item of a persistent launch as {queue, position}, or position -1 when every queue is empty; by the
+// whole workgroup.  A workgroup drains its own XCD's queue first, then the others'.  Items with neighbouring
+// ordinates, whose cell runs share cache lines in the reference layout, are in one queue: one L2 then sees the
+// whole lines, where workgroups of several XCDs would each fetch them and write parts of them.  Items of a queue
+// are taken in order, so a band's upstream band, which is in the same queue before it, has always been taken by a
+// running workgroup.
+template <typename Len>
+__device__ __forceinline__ int2 take_item(int *work, Len len) {
+    __shared__ int2 next;
+    if (threadIdx.x < 64) {
+        const int lane = (int)threadIdx.x;
+        const int own = __builtin_amdgcn_s_getreg((3 << 11) | 20) & (kXcds - 1);  // XCC_ID
+        int pick = own, pos = -1;
+        for (;;) {  // leaves when an item is taken or every counter is past its queue's end
+            int k = 0;
+            if (lane == 0) k = atomicAdd(work + pick * kWorkStride, 1);
+            k = __builtin_amdgcn_readfirstlane(k);
+            if (k < len(pick)) {
+                pos = k;
+                break;
+            }
+            const bool more = lane < kXcds && xload<int>(G(work) + lane * kWorkStride) < len(lane);
+            const unsigned m = (unsigned)__ballot(more) & ((1u << kXcds) - 1);
+            if (m == 0) break;
+            pick = (own + __builtin_ctz((m >> own | m << (kXcds - own)) & ((1u << kXcds) - 1))) & (kXcds - 1);
+        }
+        if (lane == 0) next = int2{pick, pos};
+    }
+    __syncthreads();
+    const int2 k{__builtin_amdgcn_readfirstlane(next.x), __builtin_amdgcn_readfirstlane(next.y)};
+    __syncthreads();  // every thread has read `next` before it is written again
+    return k;
 }
 
 // One problem (sp1, workgroup = band x ordinate), a batch with one item per workgroup (items[b] = {problem,
-// band * nq + ordinate}, a negative problem marking padding), or a persistent batch launch (work != null):
-// each workgroup takes the next item index from *work until nwork are taken, so items start in list
-// order (band-major: a band's upstream band has always been taken, by a running workgroup, before it).
+// band * nq + ordinate}, a negative problem marking padding), or a persistent batch launch (work != null,
+// counter set `set`): items ordered by queue, work[kWorkTable + x] the first item of XCD x's queue.
 template <typename T, int P, int MODE, int D, bool BATCH>
 __global__ __launch_bounds__(512) void k_diag_sweep_split(DiagSweepParams<T> sp1, const DiagSweepParams<T> *__restrict__ batch,
-                                                          const int2 *__restrict__ items, int *__restrict__ work, int nwork) {
+                                                          const int2 *__restrict__ items, int *__restrict__ work, int set) {
     if constexpr (!BATCH) {
         if (sp1.skip && *G(sp1.skip)) return;  // a replayed iteration after the loop has stopped
         split_item<T, P, MODE, D>(sp1, blockIdx.x);
-    } else if (work == nullptr) {
-        const gptr<const int> it = G(reinterpret_cast<const int *>(items)) + 2 * (size_t)blockIdx.x;
-        const int item_p = it[0], item_v = it[1];
-        if (item_p < 0) return;  // padding of an XCD-ordered item list
-        const DiagSweepParams<T> sp = batch[item_p];
-        if (sp.skip && *G(sp.skip)) return;
-        split_item<T, P, MODE, D>(sp, (unsigned)item_v);
     } else {
-        __shared__ int next;
-        for (;;) {
-            if (threadIdx.x == 0) next = atomicAdd(work, 1);
-            __syncthreads();
-            const int k = __builtin_amdgcn_readfirstlane(next);  // workgroup-uniform: scalar item loads
-            __syncthreads();  // every thread has read `next` before it is taken again
-            if (k >= nwork) break;  // workgroup-uniform: every wave leaves
-            const gptr<const int> it = G(reinterpret_cast<const int *>(items)) + 2 * (size_t)k;
+        if (work && blockIdx.x == 0 && threadIdx.x < kXcds) work[(1 - set) * kWorkSet + threadIdx.x * kWorkStride] = 0;
+        const gptr<const int> table = G(static_cast<const int *>(work)) + kWorkTable;
+        size_t at = blockIdx.x;
+        do {
+            if (work) {
+                const int2 k = take_item(work + set * kWorkSet, [&](int x) { return table[x + 1] - table[x]; });
+                if (k.y < 0) break;  // workgroup-uniform: every wave leaves
+                at = (size_t)(table[k.x] + k.y);
+            }
+            const gptr<const int> it = G(reinterpret_cast<const int *>(items)) + 2 * at;
             const int item_p = it[0], item_v = it[1];
-            if (item_p < 0) continue;
+            if (item_p < 0) continue;  // padding of an XCD-ordered item list
             const DiagSweepParams<T> sp = batch[item_p];
             if (sp.skip && *G(sp.skip)) continue;
             split_item<T, P, MODE, D>(sp, (unsigned)item_v);
-        }
+        } while (work);
     }
+}
+
+// Sweeps of n right-hand sides src.psi[r] of the problem sp in place on the reference layout: items (source,
+// ordinate, band), the (source, ordinate) pairs split evenly into the XCDs' queues, each queue band-major.
+// work null: one workgroup per item, band-major.
+template <typename T, int P, int D>
+__global__ __launch_bounds__(512) void k_split_ref(DiagSweepParams<T> sp, SplitSources src, int n, int *__restrict__ work, int set) {
+    const int nb = sp.nbands < 2 ? 1 : sp.nbands, pairs = n * sp.nq;
+    T *const xtr = sp.xtr;
+    if (work && blockIdx.x == 0 && threadIdx.x < kXcds) work[(1 - set) * kWorkSet + threadIdx.x * kWorkStride] = 0;
+    auto first = [&](int x) { return x * pairs / kXcds; };
+    int pair = (int)(blockIdx.x % (unsigned)pairs), band = (int)(blockIdx.x / (unsigned)pairs);
+    do {
+        if (work) {
+            const int2 k = take_item(work + set * kWorkSet, [&](int x) { return (first(x + 1) - first(x)) * nb; });
+            if (k.y < 0) break;  // workgroup-uniform: every wave leaves
+            const int p0 = first(k.x), np = first(k.x + 1) - p0;
+            pair = p0 + k.y % np;
+            band = k.y / np;
+        }
+        const int r = pair / sp.nq;
+        sp.qref = src.psi[r];
+        sp.psi_ref = src.psi[r];
+        sp.xtr = xtr + (size_t)r * sp.nq * (nb - 1) * sp.nx * P;  // the source's exchange records
+        split_item<T, P, 5, D>(sp, (unsigned)(band * sp.nq + pair - r * sp.nq));
+    } while (work);
 }
 
 }  // namespace tsw

@@ -139,9 +139,10 @@ template <typename T> struct DiagSweepParams {
     const double *qref;
     double *psi_ref;
     int ref_stage;         // 1: reference-layout sources loaded through a per-wave LDS stage (coalesced)
-    // Batched lane-split launch only (host-side dispatch): work counter of a persistent launch, whose
-    // workgroups take items in order from *work until all are taken (null: one item per workgroup)
+    // Lane-split launches only (host-side dispatch): work counters of a persistent launch, whose workgroups
+    // take items until all are taken (null: one item per workgroup), and the counter set of this launch
     int *work;
+    int work_set;
 };
 
 // Ordinate-lane sweep on the reference layout (sweep_lanes.hpp).  An ordinate block is ordinates
@@ -171,6 +172,15 @@ template <typename T> struct LanesParams {
     int *abort_flag;
     const int *skip;            // device flag: the launch does nothing while *skip != 0 (null: always runs)
     int *work;                  // batch launches (host-side dispatch): counter of a persistent launch, or null
+};
+constexpr int kXcds = 8;  // MI355X: workgroup b runs on XCD b mod 8, each XCD with its own L2
+// Device words of a lane-split launch's work counters (sweep_split.hpp), cleared when allocated: two sets, and
+// the kXcds + 1 queue bounds of a batch launch from word kSplitWorkTable on.
+constexpr int kSplitWorkTable = 2 * kXcds * 16, kSplitWorkInts = kSplitWorkTable + kXcds + 1;
+// Right-hand sides of one launch of the lane-split kernel on the reference layout.
+constexpr int kSplitSources = 32;
+struct SplitSources {
+    double *psi[kSplitSources];
 };
 constexpr int kLanesStoreWaves = 3;  // compute waves per workgroup when a storer wave writes psi
 template <typename T, int P>
@@ -235,15 +245,19 @@ template <typename T>
 void launch_diag_sweep(const DiagSweepParams<T> &sp, int p, hipStream_t s);
 template <typename T>
 size_t diag_sweep_lds_bytes(const DiagSweepParams<T> &sp, int p);
-// LDS of a lane-split sweep workgroup of `rows` row slots over an nx-column mesh with M materials (0: the
-// lane-split kernel is not built for (T, p) or does not fit)
+// LDS of a lane-split workgroup of `rows` rows with M materials on the reference layout (0: the kernel is not
+// built for (T, p) or does not fit)
 template <typename T>
-size_t split_sweep_lds_bytes(int p, int rows, int nx, int M);
+size_t split_sweep_lds_bytes(int p, int rows, int M);
 // Batched sweep over work items {problem, ordinate}; `rep` fixes degree-independent choices (mode,
 // material path), probs/items are device arrays, lds >= diag_sweep_lds_bytes of every problem.
 template <typename T>
 void launch_diag_sweep_batch(const DiagSweepParams<T> &rep, const DiagSweepParams<T> *probs, const int2 *items,
                              int nitems, int max_ny, size_t lds, int p, hipStream_t s);
+// Lane-split sweeps of n <= kSplitSources right-hand sides of one problem in place on the reference layout
+// (16-byte aligned arrays below 4 GiB - 256 bytes; sp: material path, bands, sp.work / work_set; sp.prefetch the depth)
+template <typename T>
+void launch_split_ref(const DiagSweepParams<T> &sp, const SplitSources &src, int n, size_t lds, int p, hipStream_t s);
 // tin_x / tin_y of every member of a batch from the halos of its qref (device table of nprob members)
 template <typename T>
 void launch_diag_inflow_batch(const DiagSweepParams<T> *probs, int nprob, int p, hipStream_t s);

@@ -117,13 +117,13 @@ int tsw_set_xs_degree(tsw_ctx *ctx, int degree);
  * kernel on the caller's layout, and keeps the fastest.  Key "batch_split" (0 default, 1, -1): that
  * lane-split engine (DG degrees 1-3, row bands with exchange records, a band's workgroup at most 512
  * threads) forced, forbidden or autotuned; "batch_split_rows" (0 default = the most rows one workgroup
- * holds: 256 at degree 1, 128 at degrees 2-3, or 64 where the batch autotuner finds that faster; or
- * 16..256): rows per band; "batch_split_prefetch" (0
- * default = 4, or 2, 3, 6): its prefetch depth; "batch_xcd_tile" (0 default = dispatch order, or
+ * sweeps at its fastest: 192 at degree 1, 64 at degree 2, 96 at degree 3, or 64 where the batch
+ * autotuner finds that faster; or 16..256, of which at most 192 and 96 are used): rows per band; "batch_split_prefetch" (0
+ * default = 4, 3 in FP64 at degree 3; or 2, 3, 4, 6): its prefetch depth; "batch_xcd_tile" (0 default = dispatch order, or
  * 2..64): runs of that many consecutive items (neighbouring ordinates of a member) go to one XCD (with
  * "batch_persistent" 0); "batch_persistent" (1 default, 0): each lane-split and ordinate-lane group is one
- * persistent launch of as many workgroups as the device holds, taking items in order from a device counter
- * (0: one workgroup per item).  Key "ref_stage" (0 default, 1): sweeps on the caller's layout (batch groups,
+ * persistent launch of as many workgroups as the device holds, taking items in order from device
+ * counters (0: one workgroup per item).  Key "ref_stage" (0 default, 1): sweeps on the caller's layout (batch groups,
  * tsw_sweep_apply_multi) stage their source loads through LDS where it fits.  Results do not depend on
  * any of these settings (bit for bit).
  * Solver keys: "use_dsa" (0 default, 1): diffusion synthetic acceleration of tsw_gmres_solve and

@@ -101,6 +101,49 @@ def test_ref_split_band_stall_is_reported_and_recovered():
                 assert rel_err(out, ref) <= tol, prec
 
 
+# rows at the wave (16 or 32 row slots), workgroup (192, 64, 96) and band edges, columns below and at the prefetch
+# ring and the halo ring (rows of a wave), one ordinate per quadrant and more than a workgroup per XCD
+EDGES = [(1, 1, 1, 2), (3, 33, 1, 8), (33, 192, 1, 2), (31, 193, 1, 4), (2, 385, 1, 4), (1, 16, 2, 2), (15, 17, 2, 8),
+         (17, 64, 2, 2), (16, 65, 2, 4), (5, 129, 2, 12), (4, 15, 3, 4), (18, 96, 3, 2), (7, 97, 3, 8), (33, 193, 3, 4)]
+
+
+@pytest.mark.parametrize("persistent", [1, 0])
+@pytest.mark.parametrize("shape", EDGES)
+def test_ref_split_edges_match_the_diagonal_path(shape, persistent):
+    nx, ny, p, order = shape
+    o = ls_ordinates(order)
+    g, st, _, src = random_problem(nx, ny, p, o, seed=40 + nx + ny, materials=2)
+    print("ref split edges", shape, persistent, flush=True)
+    for prec, tol in ((tsw.FP64, 1e-12), (tsw.FP32, 2e-6)):
+        a, b, c2 = src.copy(), src.copy(), src.copy()
+        with _ctx(g, o, 1) as c:
+            c.set_tuning("batch_persistent", persistent)
+            c.sweep(a, st, 0.7, precision=prec)
+            c.sweep(c2, st, 0.7, precision=prec)  # the other set of counters
+        with _ctx(g, o, -1) as c:
+            c.sweep(b, st, 0.7, precision=prec)
+        assert rel_err(a, orc_sweep(g, o, st, src, 0.7)) <= tol, prec
+        np.testing.assert_array_equal(a, b)
+        np.testing.assert_array_equal(a, c2)
+
+
+def test_ref_split_more_sources_than_one_launch_takes():
+    import torch
+    o = ls_ordinates(4)
+    g, st, _, src = random_problem(6, 70, 2, o, seed=3, materials=2)
+    dev = torch.device("cuda:0")
+    with _ctx(g, o) as c:
+        st_d = torch.from_numpy(st).to(dev)
+        many = [torch.from_numpy(src * (1 + k % 3)).to(dev) for k in range(33)]
+        one = [torch.from_numpy(src * (1 + k)).to(dev) for k in range(3)]
+        for a in one:
+            c.sweep(a, st_d, math.inf)
+        c.sweep_multi(many, st_d, math.inf)
+        torch.cuda.synchronize()
+        for k, a in enumerate(many):
+            assert torch.equal(a, one[k % 3]), k
+
+
 def test_ref_split_tuning_key():
     o = ls_ordinates(4)
     g, st, _, src = random_problem(5, 5, 1, o, seed=1)
