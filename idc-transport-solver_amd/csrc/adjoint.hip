@@ -49,19 +49,55 @@ void launch_reverse_ordinates(const Geom &g, const double *in, double *out, int 
     TSW_HIP(hipGetLastError());
 }
 
+// k_reverse_ordinates without weights, and the halos of out from `halo` (null: zero; may be out), in one pass over the
+// array: bound by HBM (read and write once each), where a fill or copy of the whole array before it moved it twice.
+// Block (chunk, j, i): consecutive threads walk a cell's values in order.
+__global__ __launch_bounds__(256) void k_reverse_all(const double *__restrict__ in, const double *halo, double *out,
+                                                     int nx, int ny, int nq, int P, int kmode) {
+    const int N = P * P, per = nq * N, m = blockIdx.x * 256 + threadIdx.x;
+    if (m >= per) return;
+    const int q = m / N, k = m - q * N, d = k / P, e = k - d * P, from = (nq - 1 - q) * N + k;
+    const double wk = (double)((2 * d + 1) * (2 * e + 1));
+    for (int i = blockIdx.z; i < nx + 2; i += gridDim.z)
+        for (int j = blockIdx.y; j < ny + 2; j += gridDim.y) {
+            const size_t base = ((size_t)i * (ny + 2) + j) * per;
+            if (i >= 1 && j >= 1 && i <= nx && j <= ny) {
+                const double v = in[base + from];
+                out[base + m] = kmode == 1 ? v * wk : v / wk;
+            } else if (halo != out) {
+                out[base + m] = halo ? halo[base + m] : 0.0;
+            }
+        }
+}
+
+void launch_reverse_all(const Geom &g, const double *in, const double *halo, double *out, int kmode, hipStream_t s) {
+    if (in == out) throw Error(TSW_E_ARG, "ordinate reversal needs distinct buffers");
+    const int per = g.nq * g.N();
+    hipLaunchKernelGGL(k_reverse_all, dim3((per + 255) / 256, std::min(g.ny + 2, 65535), std::min(g.nx + 2, 65535)),
+                       dim3(256), 0, s, in, halo, out, g.nx, g.ny, g.nq, g.p + 1, kmode);
+    TSW_HIP(hipGetLastError());
+}
+
 // Per interior cell c (one wavefront per cell), written or (accumulate) added:
 //   gst[c] (+)= -scale sum_{q,k} zeta psi               (d/dsigma_t of <seed, psi>)
 //   gss[c] (+)=  scale sum_{q,k} zeta_qk phi_k / (4 pi)  (d/dsigma_s, when phi is given)
-// psi, zeta: reference layout; phi: phi layout; gst/gss: cell arrays (halo entries not written).
+// psi, zeta: reference layout; phi: phi layout; gst/gss: cell arrays (halo entries zero, or left when accumulating).
 __global__ __launch_bounds__(256) void k_cell_grads(const double *__restrict__ psi, const double *__restrict__ zeta,
                                                     const double *__restrict__ phi, double *__restrict__ gst,
                                                     double *__restrict__ gss, int nx, int ny, int nq, int N,
                                                     double scale, int accumulate) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const long long cell = (long long)blockIdx.x * 4 + wave;
-    if (cell >= (long long)nx * ny) return;  // whole wavefront leaves; no block barrier follows
-    const int ci = (int)(cell / ny) + 1, cj = (int)(cell % ny) + 1;
-    const size_t c = (size_t)ci * (ny + 2) + cj;
+    if (cell >= (long long)(nx + 2) * (ny + 2)) return;  // whole wavefront leaves; no block barrier follows
+    const size_t c = (size_t)cell;
+    const int ci = (int)(cell / (ny + 2)), cj = (int)(cell % (ny + 2));
+    if (ci < 1 || cj < 1 || ci > nx || cj > ny) {
+        if (lane == 0 && !accumulate) {
+            if (gst) gst[c] = 0.0;
+            if (gss) gss[c] = 0.0;
+        }
+        return;
+    }
     const int per = nq * N;
     const size_t base = c * per;
     double st = 0.0, ss = 0.0;
@@ -82,7 +118,7 @@ __global__ __launch_bounds__(256) void k_cell_grads(const double *__restrict__ p
 
 void launch_cell_grads(const Geom &g, const double *psi, const double *zeta, const double *phi, double *gst,
                        double *gss, hipStream_t s, double scale, bool accumulate) {
-    const long long cells = (long long)g.nx * g.ny;
+    const long long cells = (long long)(g.nx + 2) * (g.ny + 2);
     const int blocks = (int)((cells + 3) / 4);
     hipLaunchKernelGGL(k_cell_grads, dim3(blocks), dim3(256), 0, s, psi, zeta, phi, gst, gss, g.nx, g.ny, g.nq, g.N(),
                        scale, (int)accumulate);

@@ -54,6 +54,7 @@ struct tsw_ctx {
         unsigned long long build = 0;  // counts builds and cross-section changes
     } mat;
     DBuf same_flag;  // device flags of the input change checks
+    DBuf changed;    // the mark of the last check queued with a sweep that found a difference
     // input checks made ahead in one round trip (precheck_keys), each consumed by the same_as_key call on
     // the same key, array and length within the call that made them
     struct KeyCheck {
@@ -95,6 +96,7 @@ struct tsw_ctx {
         DBuf sigt64, sigt32, sigs64, sigs32, mat, tinx64, tiny64, tinx32, tiny32, q64, q32, psi64, psi32, res32,
             phid64, phid32, phiQ, ir64;
         bool inflow = false;
+        unsigned long long mat_build = 0;  // the material table's build that `mat` was converted from
     } diag;
 
     // captured sweep graphs keyed by (precision, psi, sigma, inv_dt)
@@ -281,10 +283,13 @@ struct tsw_ctx {
             if (graph) (void)hipGraphExecDestroy(graph);
         }
     } dsa;
-    DBuf xtr64, xtr32, abort_dev;
+    DBuf xtr64, xtr32;
     size_t xtr64_n = 0, xtr32_n = 0;
-    int *abort_host = nullptr;
+    // host_flags (pinned, written by kernels, read after a synchronisation): [0] the row-band stall flag, [1] the
+    // mark of the last input check that found a difference; flags_dev is their device address
+    int *host_flags = nullptr, *flags_dev = nullptr;
     bool bands_used = false;
+    int check_mark = 0;  // marks of the input checks made so far
     // test hook (tuning key stall_test): the next banded sweep starts with the stall flag raised, so every
     // bounded wait of its bands gives up within one poll interval and the call reports the stall
     bool stall_test = false;
@@ -302,7 +307,7 @@ struct tsw_ctx {
         if (fork_ev) (void)hipEventDestroy(fork_ev);
         batch.clear();
         adj.reset();
-        if (abort_host) (void)hipHostFree(abort_host);
+        if (host_flags) (void)hipHostFree(host_flags);
         if (si_ctl_host) (void)hipHostFree(si_ctl_host);
         if (gm_host) (void)hipHostFree(gm_host);
         if (stream && own_stream) (void)hipStreamDestroy(stream);
@@ -442,19 +447,27 @@ void refill_exchange(tsw_ctx *c) {
     if (M.xtr32_n) launch_exchange_fill<float>(M.xtr32.as<float>(), M.xtr32_n, c->stream);
 }
 
+// The context's flags (host_flags), allocated and cleared on first use.
+int *flags_of(tsw_ctx *c) {
+    if (!c->host_flags) {
+        TSW_HIP(hipHostMalloc((void **)&c->host_flags, 2 * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
+        c->host_flags[0] = c->host_flags[1] = 0;
+        TSW_HIP(hipHostGetDevicePointer((void **)&c->flags_dev, c->host_flags, 0));
+    }
+    return c->flags_dev;
+}
+volatile int &stall_flag(tsw_ctx *c) { return const_cast<volatile int &>(c->host_flags[0]); }
+
 // Waits for the context's stream; reports (and clears) a row-band stall of this context or of its
 // adjoint problem.
 void sync(tsw_ctx *c) {
     tsw_ctx *chk[2] = {c->bands_used ? c : nullptr, (c->adj && c->adj->bands_used) ? c->adj.get() : nullptr};
-    for (tsw_ctx *k : chk)
-        if (k) TSW_HIP(hipMemcpyAsync(k->abort_host, k->abort_dev.ptr, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     TSW_HIP(hipStreamSynchronize(c->stream));
     bool stalled = false;
     for (tsw_ctx *k : chk) {
-        if (k && *k->abort_host) {
+        if (k && stall_flag(k)) {
             stalled = true;
-            *k->abort_host = 0;
-            TSW_HIP(hipMemsetAsync(k->abort_dev.ptr, 0, sizeof(int), c->stream));
+            stall_flag(k) = 0;
             refill_exchange(k);
             for (auto &m : k->batch) refill_exchange(m.get());  // batch members' bands report through k
         }
@@ -1085,6 +1098,16 @@ T *dbuf(DBuf &b, size_t n) {
 
 void diag_load_source(tsw_ctx *c, const double *qref, bool need64, bool need32);
 
+// The material index in the diagonal layout, converted when the table was rebuilt.
+void diag_materials(tsw_ctx *c) {
+    const Geom &g = c->g;
+    auto &d = c->diag;
+    if (!c->mat.valid || d.mat_build == c->mat.build) return;
+    launch_cell_to_diag<int32_t, int32_t>(g, c->mat.idx.as<int32_t>(), dbuf<int32_t>(d.mat, 4 * (size_t)g.nx * g.ny), 1,
+                                          c->stream);
+    d.mat_build = c->mat.build;
+}
+
 // Builds the per-call inputs: materials or per-cell sigma_t, sigma_s, inflow traces and the source
 // from reference-layout arrays (sigma_s, qref may be null).  need64/need32 select the precisions; src32
 // false leaves out the FP32 source and inflow traces (callers whose FP32 sweeps only see residuals).
@@ -1095,8 +1118,7 @@ void diag_setup(tsw_ctx *c, const double *sigma_t, const double *sigma_s, const 
     const size_t ncell = (size_t)g.nx * g.ny;
     hipStream_t s = c->stream;
     prepare_materials(c, sigma_t, dt);
-    if (c->mat.valid)
-        launch_cell_to_diag<int32_t, int32_t>(g, c->mat.idx.as<int32_t>(), dbuf<int32_t>(d.mat, 4 * ncell), 1, s);
+    diag_materials(c);
     if (need64) launch_cell_to_diag<double, double>(g, sigma_t, dbuf<double>(d.sigt64, 4 * ncell), 1, s);
     if (need32) launch_cell_to_diag<double, float>(g, sigma_t, dbuf<float>(d.sigt32, 4 * ncell), 1, s);
     if (sigma_s) {
@@ -1158,16 +1180,11 @@ int band_rows_for(const tsw_ctx *c) {
     return br;
 }
 
-// The context's device stall flag (allocated and cleared on first use); sync(c) reports a stall.
+// The device address of the context's stall flag; sync(c) reports a stall.
 int *abort_flag_of(tsw_ctx *c) {
-    if (!c->abort_host) {
-        TSW_HIP(hipHostMalloc((void **)&c->abort_host, sizeof(int), hipHostMallocDefault));
-        *c->abort_host = 0;
-        c->abort_dev.reserve(sizeof(int));
-        TSW_HIP(hipMemsetAsync(c->abort_dev.ptr, 0, sizeof(int), c->stream));
-    }
+    int *flag = flags_of(c);
     c->bands_used = true;
-    return c->abort_dev.as<int>();
+    return flag;
 }
 
 // Fills the band fields of sp and makes sure the exchange records exist (filled with the sentinel).
@@ -1329,8 +1346,7 @@ void diag_sweep(tsw_ctx *c, double dt, const T *qsrc, const T *phi_d, bool inflo
     sp.skip = c->skip_flag;
     if (c->stall_test && sp.nbands > 1 && !c->skip_flag) {
         c->stall_test = false;
-        *c->abort_host = 1;
-        TSW_HIP(hipMemcpyAsync(c->abort_dev.ptr, c->abort_host, sizeof(int), hipMemcpyHostToDevice, c->stream));
+        stall_flag(c) = 1;
     }
     if (c->skip_flag) {  // inside a graph capture: the replay is timed as a whole
         launch_diag_sweep<T>(sp, c->g.p, c->stream);
@@ -1452,12 +1468,7 @@ T *lanes_records(tsw_ctx *c, int nbands) {
         have = n;
         launch_exchange_fill<T>(buf.as<T>(), n, c->stream);
     }
-    if (!c->abort_host) {
-        TSW_HIP(hipHostMalloc((void **)&c->abort_host, sizeof(int), hipHostMallocDefault));
-        *c->abort_host = 0;
-        c->abort_dev.reserve(sizeof(int));
-        TSW_HIP(hipMemsetAsync(c->abort_dev.ptr, 0, sizeof(int), c->stream));
-    }
+    (void)flags_of(c);
     if (nbands > 1) c->bands_used = true;
     return buf.as<T>();
 }
@@ -1537,7 +1548,7 @@ LanesParams<T> lanes_params(tsw_ctx *c, double dt, const double *src, const doub
     sp.band_rows = rows;
     sp.nbands = (g.ny + rows - 1) / rows;
     sp.xtr = lanes_records<T>(c, sp.nbands);
-    sp.abort_flag = c->abort_dev.as<int>();
+    sp.abort_flag = flags_of(c);
     sp.skip = c->skip_flag;
     const int N = g.N();
     auto lds_of = [&](bool table) {
@@ -1582,8 +1593,7 @@ void lanes_sweep(tsw_ctx *c, double dt, const double *src, const double *phi, co
     const LanesParams<T> sp = lanes_params<T>(c, dt, src, phi, sig_s, psi_out, mom, true, threads, lds);
     if (c->stall_test && sp.nbands > 1 && !c->skip_flag) {
         c->stall_test = false;
-        *c->abort_host = 1;
-        TSW_HIP(hipMemcpyAsync(c->abort_dev.ptr, c->abort_host, sizeof(int), hipMemcpyHostToDevice, s));
+        stall_flag(c) = 1;
     }
     if (c->skip_flag) {  // inside a graph capture: the replay is timed as a whole
         lanes_launch<T>(c->g.p, sp, threads, lds, s);
@@ -2440,16 +2450,23 @@ bool ref_sweep_ok(tsw_ctx *c, const double *psi) {
 
 // Plan of a lane-split sweep on the caller's layout (the batch engine's kernel for one problem): false
 // when it is not built for the degree, the element-inverse tables are missing or the LDS does not fit.
-// Sets up the material table and inverses of sig for dt; base has the bands of split_band_rows rows.
+// Sets up the material table (unless `known`: taken to be that of sig) and the inverses of sig for dt; base has
+// the bands of split_band_rows rows.
 template <typename T>
-bool split_ref_plan(tsw_ctx *c, const double *sig, double dt, DiagSweepParams<T> &base, size_t &lds) {
+bool split_ref_plan(tsw_ctx *c, const double *sig, double dt, bool known, DiagSweepParams<T> &base, size_t &lds) {
     const Geom &g = c->g;
     if (c->ref_split_opt < 0 || g.p < 1) return false;
     if (c->g.npsi() * sizeof(double) > kSplitRefBytes) return false;
     // a set band_rows, prefetch, one_wave or lane_split asks for the diagonal-layout kernels
     if (c->band_rows_opt != 0 || c->prefetch_opt != 0 || c->one_wave_opt != 0 || c->split_opt != 0) return false;
-    const bool f64 = sizeof(T) == 8;
-    diag_setup(c, sig, nullptr, nullptr, dt, f64, !f64);
+    if (!known) {
+        prepare_materials(c, sig, dt);
+    } else if (c->mat.inv_dt != inverse_dt(dt)) {
+        c->mat.inv_dt = inverse_dt(dt);
+        c->mat.have64 = c->mat.have32 = false;
+    }
+    if (!c->mat.valid) return false;
+    diag_materials(c);
     base = make_diag_params<T>(c, dt, nullptr, nullptr, false, nullptr);
     if (!base.ainv) return false;
     const int br = split_band_rows(c, g.p, g.ny);
@@ -2468,9 +2485,10 @@ bool split_ref_plan(tsw_ctx *c, const double *sig, double dt, DiagSweepParams<T>
 
 // The lane-split kernel sweeping every ordinate of each array arr[r] in place (reference layout, 16-byte
 // aligned), with base from split_ref_plan, in launches of up to kSplitSources sources; per-source exchange
-// records.  Counted as arr.size() sweeps.
+// records.  Counted as arr.size() sweeps.  changed (not null): the launches do nothing while *changed == mark.
 template <typename T>
-void split_ref_sweep(tsw_ctx *c, DiagSweepParams<T> base, size_t lds, const std::vector<double *> &arr) {
+void split_ref_sweep(tsw_ctx *c, DiagSweepParams<T> base, size_t lds, const std::vector<double *> &arr,
+                     const int *changed, int mark) {
     const Geom &g = c->g;
     auto &M = c->multi;
     hipStream_t s = c->stream;
@@ -2490,23 +2508,21 @@ void split_ref_sweep(tsw_ctx *c, DiagSweepParams<T> base, size_t lds, const std:
     base.prefetch = split_prefetch<T>(c, g.p);
     if (c->stall_test && per) {  // tuning key stall_test: every bounded wait of the banded sweep gives up
         c->stall_test = false;
-        int *flag = abort_flag_of(c);
-        *c->abort_host = 1;
-        TSW_HIP(hipMemcpyAsync(flag, c->abort_host, sizeof(int), hipMemcpyHostToDevice, s));
+        (void)abort_flag_of(c);
+        stall_flag(c) = 1;
     }
     int *work = c->batch_persistent_opt > 0 ? M.work.get(s) : nullptr;
     hipEvent_t e0 = next_event(c), e1 = next_event(c);
-    TSW_HIP(hipEventRecord(e0, s));
     for (int r0 = 0; r0 < n; r0 += kSplitSources) {
         SplitSources src{};
         const int k = std::min(n - r0, kSplitSources);
         for (int r = 0; r < k; ++r) src.psi[r] = arr[r0 + r];
         base.work = work;
         base.work_set = M.work.set;
-        launch_split_ref<T>(base, src, k, lds, g.p, s);
+        launch_split_ref<T>(base, src, k, lds, g.p, changed, mark, s, r0 == 0 ? e0 : nullptr,
+                            r0 + kSplitSources >= n ? e1 : nullptr);
         M.work.set ^= 1;
     }
-    TSW_HIP(hipEventRecord(e1, s));
     c->sweeps_done += n;
 }
 
@@ -2518,8 +2534,30 @@ bool try_split_ref(tsw_ctx *c, const std::vector<double *> &arr, const double *s
         if (!ref_sweep_ok(c, a)) return false;
     DiagSweepParams<T> base;
     size_t lds = 0;
-    if (!split_ref_plan<T>(c, sig, dt, base, lds)) return false;
-    split_ref_sweep<T>(c, base, lds, arr);
+    // A call with the cross sections of the last table (the usual one) queues their check and the sweep together and
+    // waits once: the sweep does nothing where the check has found a difference, and then the table is rebuilt below.
+    // Checked first and swept after the answer, the call waited twice, about 15 us of a 65 us call on a small mesh.
+    if (c->mat.keyed && c->mat.valid && c->mat.key.bytes >= c->g.ncell_h() * sizeof(double) &&
+        split_ref_plan<T>(c, sig, dt, true, base, lds)) {
+        int *changed = static_cast<int *>(c->changed.reserve(sizeof(int)));
+        int *host = flags_of(c);
+        const int mark = c->check_mark = c->check_mark % 0x3fffffff + 1;
+        if (mark == 1) {
+            TSW_HIP(hipMemsetAsync(changed, 0, sizeof(int), c->stream));
+            c->host_flags[1] = 0;
+        }
+        launch_differs_mark(c->g.ncell_h(), sig, c->mat.key.as<double>(), changed, host + 1, mark, c->stream);
+        split_ref_sweep<T>(c, base, lds, arr, changed, mark);
+        TSW_HIP(hipStreamSynchronize(c->stream));
+        if (static_cast<volatile int &>(c->host_flags[1]) != mark) {
+            c->last_sl = 1;
+            return true;
+        }
+        c->sweeps_done -= (long long)arr.size();  // the sweep that did nothing
+        c->ev_used -= 2;
+    }
+    if (!split_ref_plan<T>(c, sig, dt, false, base, lds)) return false;
+    split_ref_sweep<T>(c, base, lds, arr, nullptr, 0);
     c->last_sl = 1;
     return true;
 }
@@ -2840,8 +2878,6 @@ tsw_ctx *adjoint_ctx(tsw_ctx *ctx) {
 void vjp_finish(tsw_ctx *ctx, const double *psi, const double *phi, double *gsrc, double *gst, double *gss) {
     const Geom &g = ctx->g;
     hipStream_t s = ctx->stream;
-    if (gst) TSW_HIP(hipMemsetAsync(gst, 0, sizeof(double) * g.ncell_h(), s));
-    if (gss) TSW_HIP(hipMemsetAsync(gss, 0, sizeof(double) * g.ncell_h(), s));
     if (gst || gss) launch_cell_grads(g, psi, gsrc, phi, gst, gss, s);
     launch_inflow_grad(g, gsrc, gsrc, ctx->xi64.as<double>(), ctx->eta64.as<double>(), s);
 }
@@ -2855,11 +2891,9 @@ void sweep_vjp_device(tsw_ctx *ctx, const double *psi, const double *st, double 
     hipStream_t s = ctx->stream;
     tsw_ctx *a = adjoint_ctx(ctx);
     double *y = dbuf<double>(ctx->vjp_y, g.npsi());
-    TSW_HIP(hipMemsetAsync(y, 0, sizeof(double) * g.npsi(), s));
-    launch_reverse_ordinates(g, seed, y, 1, nullptr, 0, false, s);
+    launch_reverse_all(g, seed, nullptr, y, 1, s);
     sweep_device(a, y, st, dt, precision);
-    if (gsrc != seed) TSW_HIP(hipMemcpyAsync(gsrc, seed, sizeof(double) * g.npsi(), hipMemcpyDeviceToDevice, s));
-    launch_reverse_ordinates(g, y, gsrc, 2, nullptr, 0, false, s);
+    launch_reverse_all(g, y, seed, gsrc, 2, s);
     vjp_finish(ctx, psi, nullptr, gsrc, gst, nullptr);
 }
 
@@ -4306,9 +4340,8 @@ void batch_sweep(tsw_ctx *ctx, bool conv64, bool inplace64, bool corr, const std
                 banded = banded || gd.first->band_rows[m] < ctx->batch[gd.first->members[m]]->g.ny;
         if (banded) {
             ctx->stall_test = false;
-            int *flag = abort_flag_of(ctx);
-            *ctx->abort_host = 1;
-            TSW_HIP(hipMemcpyAsync(flag, ctx->abort_host, sizeof(int), hipMemcpyHostToDevice, ctx->stream));
+            (void)abort_flag_of(ctx);
+            stall_flag(ctx) = 1;
         }
     }
     hipEvent_t e0 = next_event(ctx), e1 = next_event(ctx);

@@ -382,6 +382,21 @@ void launch_differs(size_t n, const double *a, const double *b, int *flag, hipSt
     TSW_HIP(hipGetLastError());
 }
 
+__global__ void k_differs_mark(size_t n, const unsigned long long *__restrict__ a,
+                               const unsigned long long *__restrict__ b, int *flag, int *host, int mark) {
+    bool diff = false;
+    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x)
+        diff |= a[t] != b[t];
+    if (diff) *flag = *host = mark;  // every writer stores the same value
+}
+void launch_differs_mark(size_t n, const double *a, const double *b, int *flag, int *host, int mark, hipStream_t s) {
+    const size_t blocks = std::min<size_t>(grid_for(n), 1024);
+    hipLaunchKernelGGL(k_differs_mark, dim3((unsigned)blocks), dim3(kBlock), 0, s, n,
+                       reinterpret_cast<const unsigned long long *>(a), reinterpret_cast<const unsigned long long *>(b),
+                       flag, host, mark);
+    TSW_HIP(hipGetLastError());
+}
+
 // ---- FP64 vector kernels for the Krylov driver ----
 __global__ void k_axpby(size_t n, double a, const double *__restrict__ x, double b, double *__restrict__ y) {
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;

@@ -126,16 +126,19 @@ void launch_diag_sweep_batch(const DiagSweepParams<T> &rep, const DiagSweepParam
     }
 }
 template <typename T>
-void launch_split_ref(const DiagSweepParams<T> &sp, const SplitSources &src, int n, size_t lds, int p, hipStream_t s) {
+void launch_split_ref(const DiagSweepParams<T> &sp, const SplitSources &src, int n, size_t lds, int p,
+                      const int *changed, int mark, hipStream_t s, hipEvent_t start, hipEvent_t stop) {
     switch (p) {
-        case 1: launch_split_ref_p<T, 2>(sp, src, n, lds, s); break;
-        case 2: launch_split_ref_p<T, 3>(sp, src, n, lds, s); break;
-        case 3: launch_split_ref_p<T, 4>(sp, src, n, lds, s); break;
+        case 1: launch_split_ref_p<T, 2>(sp, src, n, lds, changed, mark, s, start, stop); break;
+        case 2: launch_split_ref_p<T, 3>(sp, src, n, lds, changed, mark, s, start, stop); break;
+        case 3: launch_split_ref_p<T, 4>(sp, src, n, lds, changed, mark, s, start, stop); break;
         default: throw Error(TSW_E_UNSUPPORTED, "lane-split sweep built for DG degrees 1-3");
     }
 }
-template void launch_split_ref<double>(const DiagSweepParams<double> &, const SplitSources &, int, size_t, int, hipStream_t);
-template void launch_split_ref<float>(const DiagSweepParams<float> &, const SplitSources &, int, size_t, int, hipStream_t);
+template void launch_split_ref<double>(const DiagSweepParams<double> &, const SplitSources &, int, size_t, int, const int *, int,
+                                       hipStream_t, hipEvent_t, hipEvent_t);
+template void launch_split_ref<float>(const DiagSweepParams<float> &, const SplitSources &, int, size_t, int, const int *, int,
+                                       hipStream_t, hipEvent_t, hipEvent_t);
 template <typename T>
 void launch_diag_inflow_batch(const DiagSweepParams<T> *probs, int nprob, int p, hipStream_t s) {
     switch (p) {

@@ -14,6 +14,8 @@
 // isotropic scattering source of Smv, TransportOperator.cpp:369-392, fused into the load).
 #pragma once
 
+#include <hip/hip_ext.h>
+
 #include <algorithm>
 #include <string>
 
@@ -755,7 +757,8 @@ void launch_diag_sweep_batch_p(const DiagSweepParams<T> &rep, const DiagSweepPar
 // Lane-split sweeps on the reference layout (launch_split_ref): persistent with sp.work, as many workgroups as
 // the device holds at once.
 template <typename T, int P>
-void launch_split_ref_p(const DiagSweepParams<T> &sp, const SplitSources &src, int n, size_t lds, hipStream_t s) {
+void launch_split_ref_p(const DiagSweepParams<T> &sp, const SplitSources &src, int n, size_t lds, const int *changed,
+                        int mark, hipStream_t s, hipEvent_t start, hipEvent_t stop) {
     if constexpr (split_supported<T, P>()) {
         const int threads = (split_lanes<P>() * band_rows_of(sp) + 63) / 64 * 64 + 64 * kSplitStorers;
         if (threads > 512 || !sp.ainv || n < 1 || n > kSplitSources || (sp.nbands > 1 && (!sp.xtr || !sp.abort_flag)))
@@ -772,7 +775,9 @@ void launch_split_ref_p(const DiagSweepParams<T> &sp, const SplitSources &src, i
                 TSW_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
                 grid = std::max(1, std::min(items, std::max(per_cu, 1) * cus));
             }
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, s, sp, src, n, sp.work, sp.work_set);
+            // (the events ride on the dispatch itself: no marker packets around it)
+            hipExtLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, s, start, stop, 0, sp, src, n, sp.work, sp.work_set,
+                                  changed, mark);
             TSW_HIP(hipGetLastError());
         };
         switch (sp.prefetch) {
@@ -827,14 +832,16 @@ void launch_diag_inflow_batch_p(const DiagSweepParams<T> *batch, int nprob, hipS
 
 #define TSW_SWEEP_INSTANTIATE(T, P)                                                                         \
     template void launch_diag_inflow_batch_p<T, P>(const DiagSweepParams<T> *, int, hipStream_t);          \
-    template void launch_split_ref_p<T, P>(const DiagSweepParams<T> &, const SplitSources &, int, size_t, hipStream_t); \
+    template void launch_split_ref_p<T, P>(const DiagSweepParams<T> &, const SplitSources &, int, size_t, const int *, int, hipStream_t, \
+                                             hipEvent_t, hipEvent_t);                                       \
     template void launch_diag_sweep_p<T, P>(const DiagSweepParams<T> &, size_t, hipStream_t);              \
     template void launch_diag_sweep_batch_p<T, P>(const DiagSweepParams<T> &, const DiagSweepParams<T> *,   \
                                                   const int2 *, int, int, size_t, hipStream_t);
 
 #define TSW_SWEEP_EXTERN(T, P)                                                                              \
     extern template void launch_diag_inflow_batch_p<T, P>(const DiagSweepParams<T> *, int, hipStream_t);   \
-    extern template void launch_split_ref_p<T, P>(const DiagSweepParams<T> &, const SplitSources &, int, size_t, hipStream_t); \
+    extern template void launch_split_ref_p<T, P>(const DiagSweepParams<T> &, const SplitSources &, int, size_t, const int *, int, hipStream_t, \
+                                             hipEvent_t, hipEvent_t);                                       \
     extern template void launch_diag_sweep_p<T, P>(const DiagSweepParams<T> &, size_t, hipStream_t);       \
     extern template void launch_diag_sweep_batch_p<T, P>(const DiagSweepParams<T> &, const DiagSweepParams<T> *, \
                                                          const int2 *, int, int, size_t, hipStream_t);

@@ -534,10 +534,12 @@ __global__ __launch_bounds__(512) void k_diag_sweep_split(DiagSweepParams<T> sp1
 // ordinate, band), the (source, ordinate) pairs split evenly into the XCDs' queues, each queue band-major.
 // work null: one workgroup per item, band-major.
 template <typename T, int P, int D>
-__global__ __launch_bounds__(512) void k_split_ref(DiagSweepParams<T> sp, SplitSources src, int n, int *__restrict__ work, int set) {
+__global__ __launch_bounds__(512) void k_split_ref(DiagSweepParams<T> sp, SplitSources src, int n, int *__restrict__ work, int set,
+                                                   const int *__restrict__ changed, int mark) {
     const int nb = sp.nbands < 2 ? 1 : sp.nbands, pairs = n * sp.nq;
     T *const xtr = sp.xtr;
     if (work && blockIdx.x == 0 && threadIdx.x < kXcds) work[(1 - set) * kWorkSet + threadIdx.x * kWorkStride] = 0;
+    if (changed && *G(changed) == mark) return;  // the inputs are not those the tables were built from
     auto first = [&](int x) { return x * pairs / kXcds; };
     int pair = (int)(blockIdx.x % (unsigned)pairs), band = (int)(blockIdx.x / (unsigned)pairs);
     do {

@@ -255,9 +255,11 @@ template <typename T>
 void launch_diag_sweep_batch(const DiagSweepParams<T> &rep, const DiagSweepParams<T> *probs, const int2 *items,
                              int nitems, int max_ny, size_t lds, int p, hipStream_t s);
 // Lane-split sweeps of n <= kSplitSources right-hand sides of one problem in place on the reference layout
-// (16-byte aligned arrays below 4 GiB - 256 bytes; sp: material path, bands, sp.work / work_set; sp.prefetch the depth)
+// (16-byte aligned arrays below 4 GiB - 256 bytes; sp: material path, bands, sp.work / work_set; sp.prefetch the depth).
+// The launch does nothing while *changed == mark (changed not null); start and stop (or null) are recorded around it.
 template <typename T>
-void launch_split_ref(const DiagSweepParams<T> &sp, const SplitSources &src, int n, size_t lds, int p, hipStream_t s);
+void launch_split_ref(const DiagSweepParams<T> &sp, const SplitSources &src, int n, size_t lds, int p,
+                      const int *changed, int mark, hipStream_t s, hipEvent_t start, hipEvent_t stop);
 // tin_x / tin_y of every member of a batch from the halos of its qref (device table of nprob members)
 template <typename T>
 void launch_diag_inflow_batch(const DiagSweepParams<T> *probs, int nprob, int p, hipStream_t s);
@@ -333,6 +335,8 @@ struct LinComb {
 void launch_lincomb(const Geom &g, size_t per_cell, const LinComb &L, double *y, hipStream_t s);
 // flag[0] <- 1 if a and b differ bitwise anywhere in n doubles, else 0
 void launch_differs(size_t n, const double *a, const double *b, int *flag, hipStream_t s);
+// *flag and *host (host memory) <- mark if a and b differ bitwise anywhere in n doubles, else left as they are
+void launch_differs_mark(size_t n, const double *a, const double *b, int *flag, int *host, int mark, hipStream_t s);
 // out[i] = sum_k X_i[k] * y[k], i < m, X_i = X + i*ld; uses `partials` scratch; result on device
 void launch_multi_dot(size_t n, int m, const double *X, size_t ld, const double *y, double *out, double *partials,
                       int nblocks, hipStream_t s);
@@ -348,6 +352,8 @@ int reduction_blocks();
 // adjoint path (adjoint.hip)
 void launch_reverse_ordinates(const Geom &g, const double *in, double *out, int kmode, const double *w, int qmode,
                               bool w_of_out, hipStream_t s);
+// the same without weights, and out's halos <- halo's (null: zero); halo may be out
+void launch_reverse_all(const Geom &g, const double *in, const double *halo, double *out, int kmode, hipStream_t s);
 void launch_cell_grads(const Geom &g, const double *psi, const double *zeta, const double *phi, double *gst,
                        double *gss, hipStream_t s, double scale = 1.0, bool accumulate = false);
 void launch_kt_apply(const Geom &g, const double *y, double *out, const double *ss, const double *w, double alpha,

@@ -144,6 +144,26 @@ def test_ref_split_more_sources_than_one_launch_takes():
             assert torch.equal(a, one[k % 3]), k
 
 
+@pytest.mark.parametrize("p", [1, 2, 3])
+def test_ref_split_follows_changes_of_the_inputs(p):
+    """The sweep queued behind the check of the cross sections leaves the array alone when they have changed (also
+    in one halo-side value, to more than 64 values and back), and each sweep is counted once."""
+    o = ls_ordinates(4)
+    g, st, _, src = random_problem(9, 35, p, o, seed=70 + p, materials=3)
+    one = st.copy()
+    one[g.nx, g.ny] *= 1.5
+    many = random_problem(9, 35, p, o, seed=71 + p)[1]
+    with _ctx(g, o) as c:
+        c.sweep_timing(reset=True)
+        seq = [(st, 0.3), (st, 0.3), (one, 0.3), (one, math.inf), (st, 0.3), (many, 0.3), (st, 0.3), (2 * st, 0.3)]
+        for k, (sig, dt) in enumerate(seq):
+            for prec, tol in ((tsw.FP64, 1e-12), (tsw.FP32, 2e-6)):
+                out = src.copy()
+                c.sweep(out, sig, dt, precision=prec)
+                assert rel_err(out, orc_sweep(g, o, sig, src, dt)) <= tol, (k, prec)
+                assert c.sweep_timing(reset=True)[0] == 1 or sig is many, (k, prec)
+
+
 def test_ref_split_tuning_key():
     o = ls_ordinates(4)
     g, st, _, src = random_problem(5, 5, 1, o, seed=1)
