@@ -1168,7 +1168,7 @@ const T *diag_inverses(tsw_ctx *c, double dt) {
 // one wavefront of rows per band when the mesh has more rows than that, so the ordinates' sweeps
 // spread over several times more compute units than there are ordinates.
 bool one_wave_for(const tsw_ctx *c) { return (c->tuned_w1 != INT_MIN ? c->tuned_w1 : c->one_wave_opt) == 1; }
-bool lane_split_for(const tsw_ctx *c) { return (c->tuned_sl != INT_MIN ? c->tuned_sl : c->split_opt) == 1; }
+int lane_split_for(const tsw_ctx *c) { return std::max(0, c->tuned_sl != INT_MIN ? c->tuned_sl : c->split_opt); }
 
 int band_rows_for(const tsw_ctx *c) {
     const int ny = c->g.ny;
@@ -1245,7 +1245,7 @@ DiagSweepParams<T> make_diag_params(tsw_ctx *c, double dt, const T *qsrc, const 
         sp.mat = d.mat.as<int32_t>();
         sp.M = c->mat.M;
         if (lane_split_for(c)) {  // kept where the lane-split kernel is built and its tables fit
-            sp.split = 1;
+            sp.split = lane_split_for(c);
             sp.wave1 = 0;
             if (diag_sweep_lds_bytes<T>(sp, g.p) == 0) sp.split = 0;
         }
@@ -1259,10 +1259,13 @@ DiagSweepParams<T> make_diag_params(tsw_ctx *c, double dt, const T *qsrc, const 
     }
     if (!sp.ainv) sp.sig_t = (const T *)(f64 ? d.sigt64.ptr : d.sigt32.ptr);
     c->last_w1 = sp.wave1;
-    c->last_sl = sp.split;
+    c->last_sl = sp.split != 0;
     sp.psi = psi_out;
     return sp;
 }
+
+// Rows of the largest workgroup of the lane-per-coefficient sweep.
+int kWideRows(int p) { return 896 / (p == 1 ? 4 : 16); }
 
 // Autotuning of the staggered sweep: the candidates are one band per ordinate and bands of 64..256 rows
 // (below ny), crossed with prefetch depths 2, 3, 4, 6; each runs twice into a scratch output (inputs
@@ -1283,7 +1286,7 @@ void select_tuning(tsw_ctx *c, double dt, const T *qsrc, const T *phi_d, bool in
         if (cap != hipStreamCaptureStatusNone) return;  // no timing inside a capture: defaults
         // (band rows, one wave, lane split): one-lane kernels over one band and bands of 64..256 rows,
         // the one-wave kernel over 64-row bands, the lane-split kernel over one band (meshes of at most
-        // 128 rows) and bands of 32..128 rows
+        // 128 rows) and bands of 32..128 rows, and as far as a workgroup reaches the lane-per-coefficient kernel (2)
         std::vector<std::array<int, 3>> shapes{{-1, 0, 0}};
         for (int br = 64; br <= 256 && br < g.ny; br += 64) shapes.push_back({br, 0, 0});
         if (g.ny > 64) shapes.push_back({64, 1, 0});
@@ -1292,6 +1295,10 @@ void select_tuning(tsw_ctx *c, double dt, const T *qsrc, const T *phi_d, bool in
             if (g.ny <= 128) shapes.push_back({-1, 0, 1});
             for (int br : {32, 64, 96, 128})
                 if (br < g.ny) shapes.push_back({br, 0, 1});
+            const int most = kWideRows(g.p);
+            if (g.ny <= most) shapes.push_back({-1, 0, 2});
+            for (int br : {32, 64, 96, 128})
+                if (br < g.ny && br <= most) shapes.push_back({br, 0, 2});
         }
         const int pfs[] = {2, 3, 4, 6};
         T *out = dbuf<T>(c->tune_out, (size_t)g.nq * g.N() * g.nx * g.ny);
@@ -2434,6 +2441,20 @@ int split_band_rows(const tsw_ctx *ctx, int p, int ny) {
     return (ny + nb - 1) / nb;
 }
 
+// Rows per band of the lane-per-coefficient kernel on the reference layout, 0 where the lane-split kernel is the faster:
+// its waves hold a quarter of the rows, so it pays while the chip holds the sweep's `rows` (of all ordinates and sources)
+// at about the same time.  Kernel us, lane-split against this, S8 or S12: Q3 32 x 32 60 -> 28, 128 x 128 222 -> 115,
+// 140 x 140 197 -> 129, 256 x 256 453 -> 308, 280 x 280 (23,520 rows) 543 -> 488; Q2 32 x 32 38 -> 24, 128 x 128 142 ->
+// 108, 256 x 256 267 -> 222, 210 x 210 (17,640 rows) 283 -> 258, but 280 x 280 467 -> 477; Q1 32 x 32 26 -> 17,
+// 128 x 128 84 -> 74, 256 x 256 (10,240 rows) 187 -> 163, but 280 x 280 214 -> 220.  One band up to the most rows of a
+// workgroup; more rows than that in bands of 24 (64 at degree 1, where a row takes 4 lanes), of which a CU holds three:
+// within 3% of the best of 16 .. 56 at all these sizes.
+int wide_band_rows(const tsw_ctx *c, int p, int ny, long long rows) {
+    if (c->batch_split_rows_opt > 0 || rows > (p == 3 ? 1 << 20 : 20000)) return 0;
+    const int most = kWideRows(p), R = p == 1 ? 64 : 24, nb = ny <= most ? 1 : (ny + R - 1) / R;
+    return (ny + nb - 1) / nb;
+}
+
 // Prefetch depth of the lane-split kernel on the reference layout: 3 for FP64 Q3, whose ring of 4 spills (256 x 256, S8,
 // 64 materials: 461 against 556 us), else kSplitBatchPrefetch, unless the tuning key batch_split_prefetch sets it.
 template <typename T>
@@ -2448,12 +2469,12 @@ bool ref_sweep_ok(tsw_ctx *c, const double *psi) {
            c->g.npsi() * sizeof(double) < (size_t(1) << 32) && c->g.ny <= 448 && ((uintptr_t)psi & 15) == 0;
 }
 
-// Plan of a lane-split sweep on the caller's layout (the batch engine's kernel for one problem): false
+// Plan of a lane-split sweep of n sources on the caller's layout (the batch engine's kernel for one problem): false
 // when it is not built for the degree, the element-inverse tables are missing or the LDS does not fit.
 // Sets up the material table (unless `known`: taken to be that of sig) and the inverses of sig for dt; base has
 // the bands of split_band_rows rows.
 template <typename T>
-bool split_ref_plan(tsw_ctx *c, const double *sig, double dt, bool known, DiagSweepParams<T> &base, size_t &lds) {
+bool split_ref_plan(tsw_ctx *c, const double *sig, double dt, bool known, int n, DiagSweepParams<T> &base, size_t &lds) {
     const Geom &g = c->g;
     if (c->ref_split_opt < 0 || g.p < 1) return false;
     if (c->g.npsi() * sizeof(double) > kSplitRefBytes) return false;
@@ -2469,10 +2490,17 @@ bool split_ref_plan(tsw_ctx *c, const double *sig, double dt, bool known, DiagSw
     diag_materials(c);
     base = make_diag_params<T>(c, dt, nullptr, nullptr, false, nullptr);
     if (!base.ainv) return false;
-    const int br = split_band_rows(c, g.p, g.ny);
+    int br = split_band_rows(c, g.p, g.ny);
     lds = split_sweep_lds_bytes<T>(g.p, br, base.M);
     if (lds == 0) return false;
     base.split = 1;
+    const int wr = wide_band_rows(c, g.p, g.ny, (long long)n * g.nq * g.ny);
+    if (const size_t l = wr > 0 ? wide_sweep_lds_bytes<T>(g.p, wr, base.M) : 0; l > 0) {
+        br = wr;
+        lds = l;
+        base.split = 2;
+        base.mat_cell = c->mat.idx.as<int32_t>();
+    }
     base.direct = 0;
     base.wave1 = 0;
     base.ref_stage = 0;
@@ -2505,13 +2533,14 @@ void split_ref_sweep(tsw_ctx *c, DiagSweepParams<T> base, size_t lds, const std:
         base.xtr = xb.as<T>();
         base.abort_flag = abort_flag_of(c);
     }
-    base.prefetch = split_prefetch<T>(c, g.p);
+    // (a ring of 3 takes 2 to 4% longer with a lane per coefficient, one of 6 up to 20%)
+    base.prefetch = base.split == 2 && c->batch_split_pf_opt == 0 ? 4 : split_prefetch<T>(c, g.p);
     if (c->stall_test && per) {  // tuning key stall_test: every bounded wait of the banded sweep gives up
         c->stall_test = false;
         (void)abort_flag_of(c);
         stall_flag(c) = 1;
     }
-    int *work = c->batch_persistent_opt > 0 ? M.work.get(s) : nullptr;
+    int *work = c->batch_persistent_opt > 0 && base.split == 1 ? M.work.get(s) : nullptr;
     hipEvent_t e0 = next_event(c), e1 = next_event(c);
     for (int r0 = 0; r0 < n; r0 += kSplitSources) {
         SplitSources src{};
@@ -2521,7 +2550,7 @@ void split_ref_sweep(tsw_ctx *c, DiagSweepParams<T> base, size_t lds, const std:
         base.work_set = M.work.set;
         launch_split_ref<T>(base, src, k, lds, g.p, changed, mark, s, r0 == 0 ? e0 : nullptr,
                             r0 + kSplitSources >= n ? e1 : nullptr);
-        M.work.set ^= 1;
+        if (base.split == 1) M.work.set ^= 1;  // (the other kernel neither takes from the counters nor clears them)
     }
     c->sweeps_done += n;
 }
@@ -2538,7 +2567,7 @@ bool try_split_ref(tsw_ctx *c, const std::vector<double *> &arr, const double *s
     // waits once: the sweep does nothing where the check has found a difference, and then the table is rebuilt below.
     // Checked first and swept after the answer, the call waited twice, about 15 us of a 65 us call on a small mesh.
     if (c->mat.keyed && c->mat.valid && c->mat.key.bytes >= c->g.ncell_h() * sizeof(double) &&
-        split_ref_plan<T>(c, sig, dt, true, base, lds)) {
+        split_ref_plan<T>(c, sig, dt, true, (int)arr.size(), base, lds)) {
         int *changed = static_cast<int *>(c->changed.reserve(sizeof(int)));
         int *host = flags_of(c);
         const int mark = c->check_mark = c->check_mark % 0x3fffffff + 1;
@@ -2556,7 +2585,7 @@ bool try_split_ref(tsw_ctx *c, const std::vector<double *> &arr, const double *s
         c->sweeps_done -= (long long)arr.size();  // the sweep that did nothing
         c->ev_used -= 2;
     }
-    if (!split_ref_plan<T>(c, sig, dt, false, base, lds)) return false;
+    if (!split_ref_plan<T>(c, sig, dt, false, (int)arr.size(), base, lds)) return false;
     split_ref_sweep<T>(c, base, lds, arr, nullptr, 0);
     c->last_sl = 1;
     return true;

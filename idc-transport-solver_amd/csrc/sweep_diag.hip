@@ -48,6 +48,18 @@ size_t split_sweep_lds_bytes(int p, int rows, int M) {
 }
 template size_t split_sweep_lds_bytes<double>(int, int, int);
 template size_t split_sweep_lds_bytes<float>(int, int, int);
+template <typename T>
+size_t wide_sweep_lds_bytes(int p, int rows, int M) {
+    const int lanes = p == 1 ? wide_lanes<2>() : wide_lanes<3>(), slots = (lanes * rows + 63) / 64 * 64 / lanes;
+    if (p < 1 || p > 3 || slots * lanes + 64 * kWideHelpers > kWideThreads) return 0;
+    const size_t total = p == 1   ? WideLds<T, 2>(slots, M).total
+                         : p == 2 ? WideLds<T, 3>(slots, M).total
+                                  : WideLds<T, 4>(slots, M).total;
+    const size_t bytes = total * sizeof(T);
+    return bytes + 16 <= max_lds_per_block() ? bytes : 0;
+}
+template size_t wide_sweep_lds_bytes<double>(int, int, int);
+template size_t wide_sweep_lds_bytes<float>(int, int, int);
 
 template <typename T>
 size_t diag_sweep_lds_bytes(const DiagSweepParams<T> &sp, int p) {
@@ -58,7 +70,7 @@ size_t diag_sweep_lds_bytes(const DiagSweepParams<T> &sp, int p) {
     if (sp.wave1 && BR > 64) return 0;
     if (sp.split) {
         if (!sp.ainv || sp.wave1) return 0;
-        return split_lds_bytes<T>(p, BR, sp.M, false);
+        return sp.split == 2 ? wide_sweep_lds_bytes<T>(p, BR, sp.M) : split_lds_bytes<T>(p, BR, sp.M, false);
     }
     const int cthreads = ((BR + 63) / 64) * 64;
     const int M = sp.ainv ? sp.M : 0;

@@ -641,10 +641,13 @@ void launch_ds_d(const DiagSweepParams<T> &sp, size_t lds, hipStream_t s, const 
     if (sp.split) {
         if constexpr (MAT && split_supported<T, P>() && ((MODE & 4) == 0 || MODE == 5)) {
             // LG lanes for each row slot, in whole wavefronts, and the reference layout's storer waves
-            const int threads = (split_lanes<P>() * rows + 63) / 64 * 64 + ((MODE & 4) != 0 ? 64 * kSplitStorers : 0);
-            if (threads > 512) throw Error(TSW_E_ARG, "lane-split sweep needs bands of at most 512 / lanes rows");
+            const bool wide = sp.split == 2;
+            const int threads = wide ? (wide_lanes<P>() * rows + 63) / 64 * 64 + 64 * kWideHelpers
+                                     : (split_lanes<P>() * rows + 63) / 64 * 64 + ((MODE & 4) != 0 ? 64 * kSplitStorers : 0);
+            if (wide && (batch || threads > kWideThreads)) throw Error(TSW_E_ARG, "lane-per-coefficient sweep: inconsistent launch");
+            if (!wide && threads > 512) throw Error(TSW_E_ARG, "lane-split sweep needs bands of at most 512 / lanes rows");
             if (batch) {
-                auto kern = k_diag_sweep_split<T, P, MODE, D, true>;
+                auto kern = k_diag_sweep_split<T, P, MODE, D, true, false>;
                 if (lds > 64 * 1024)
                     TSW_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
                 int grid = nitems;
@@ -658,7 +661,7 @@ void launch_ds_d(const DiagSweepParams<T> &sp, size_t lds, hipStream_t s, const 
                 hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, s, sp, batch, items, sp.work, sp.work_set);
             } else {
                 if constexpr ((MODE & 4) != 0) throw Error(TSW_E_ARG, "reference-layout lane-split sweep is built for batches");
-                auto kern = k_diag_sweep_split<T, P, MODE, D, false>;
+                auto kern = wide ? k_diag_sweep_split<T, P, MODE, D, false, true> : k_diag_sweep_split<T, P, MODE, D, false, false>;
                 if (lds > 64 * 1024)
                     TSW_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
                 hipLaunchKernelGGL(kern, dim3(sp.nq * (sp.nbands > 1 ? sp.nbands : 1)),
@@ -760,14 +763,24 @@ template <typename T, int P>
 void launch_split_ref_p(const DiagSweepParams<T> &sp, const SplitSources &src, int n, size_t lds, const int *changed,
                         int mark, hipStream_t s, hipEvent_t start, hipEvent_t stop) {
     if constexpr (split_supported<T, P>()) {
-        const int threads = (split_lanes<P>() * band_rows_of(sp) + 63) / 64 * 64 + 64 * kSplitStorers;
-        if (threads > 512 || !sp.ainv || n < 1 || n > kSplitSources || (sp.nbands > 1 && (!sp.xtr || !sp.abort_flag)))
+        const bool wide = sp.split == 2;
+        const int threads = wide ? (wide_lanes<P>() * band_rows_of(sp) + 63) / 64 * 64 + 64 * kWideHelpers
+                                 : (split_lanes<P>() * band_rows_of(sp) + 63) / 64 * 64 + 64 * kSplitStorers;
+        if (threads > (wide ? kWideThreads : 512) || !sp.ainv || n < 1 || n > kSplitSources || (sp.nbands > 1 && (!sp.xtr || !sp.abort_flag)))
             throw Error(TSW_E_ARG, "lane-split reference-layout sweep: inconsistent launch");
         const int items = n * sp.nq * (sp.nbands > 1 ? sp.nbands : 1);
+        // the most items of a queue, over all queues
+        const int queued = (n * sp.nq + kXcds - 1) / kXcds * kXcds * (sp.nbands > 1 ? sp.nbands : 1);
+        auto go_wide = [&](auto kern) {
+            if (lds > 64 * 1024)
+                TSW_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            hipExtLaunchKernelGGL(kern, dim3(queued), dim3(threads), lds, s, start, stop, 0, sp, src, n, changed, mark);
+            TSW_HIP(hipGetLastError());
+        };
         auto go = [&](auto kern) {
             if (lds > 64 * 1024)
                 TSW_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            int grid = items;
+            int grid = queued;
             if (sp.work) {
                 int per_cu = 0, dev = 0, cus = 0;
                 TSW_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)kern, threads, lds));
@@ -781,10 +794,10 @@ void launch_split_ref_p(const DiagSweepParams<T> &sp, const SplitSources &src, i
             TSW_HIP(hipGetLastError());
         };
         switch (sp.prefetch) {
-            case 2: go(k_split_ref<T, P, 2>); break;
-            case 3: go(k_split_ref<T, P, 3>); break;
-            case 4: go(k_split_ref<T, P, 4>); break;
-            case 6: go(k_split_ref<T, P, 6>); break;
+            case 2: wide ? go_wide(k_wide_ref<T, P, 2>) : go(k_split_ref<T, P, 2>); break;
+            case 3: wide ? go_wide(k_wide_ref<T, P, 3>) : go(k_split_ref<T, P, 3>); break;
+            case 4: wide ? go_wide(k_wide_ref<T, P, 4>) : go(k_split_ref<T, P, 4>); break;
+            case 6: wide ? go_wide(k_wide_ref<T, P, 6>) : go(k_split_ref<T, P, 6>); break;
             default: throw Error(TSW_E_ARG, "prefetch depth must be 2, 3, 4 or 6");
         }
     } else {

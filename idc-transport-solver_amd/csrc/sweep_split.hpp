@@ -461,6 +461,12 @@ __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigne
     for (int k = w0 + nrun; k < nbar; ++k) lds_barrier();
 }
 
+}  // namespace tsw
+
+#include "sweep_wide.hpp"
+
+namespace tsw {
+
 // Work counters of a persistent launch: two sets of one counter per XCD, each in a cache line of its own;
 // a launch takes items with one set and clears the other for the next launch.  Batch launches add the item
 // range of each XCD's queue.
@@ -504,12 +510,13 @@ __device__ __forceinline__ int2 take_item(int *work, Len len) {
 // One problem (sp1, workgroup = band x ordinate), a batch with one item per workgroup (items[b] = {problem,
 // band * nq + ordinate}, a negative problem marking padding), or a persistent batch launch (work != null,
 // counter set `set`): items ordered by queue, work[kWorkTable + x] the first item of XCD x's queue.
-template <typename T, int P, int MODE, int D, bool BATCH>
-__global__ __launch_bounds__(512) void k_diag_sweep_split(DiagSweepParams<T> sp1, const DiagSweepParams<T> *__restrict__ batch,
+template <typename T, int P, int MODE, int D, bool BATCH, bool WIDE>
+__global__ __launch_bounds__(WIDE ? kWideThreads : 512) void k_diag_sweep_split(DiagSweepParams<T> sp1, const DiagSweepParams<T> *__restrict__ batch,
                                                           const int2 *__restrict__ items, int *__restrict__ work, int set) {
     if constexpr (!BATCH) {
         if (sp1.skip && *G(sp1.skip)) return;  // a replayed iteration after the loop has stopped
-        split_item<T, P, MODE, D>(sp1, blockIdx.x);
+        if constexpr (WIDE) wide_item<T, P, MODE, D>(sp1, blockIdx.x);
+        else split_item<T, P, MODE, D>(sp1, blockIdx.x);
     } else {
         if (work && blockIdx.x == 0 && threadIdx.x < kXcds) work[(1 - set) * kWorkSet + threadIdx.x * kWorkStride] = 0;
         const gptr<const int> table = G(static_cast<const int *>(work)) + kWorkTable;
@@ -530,32 +537,51 @@ __global__ __launch_bounds__(512) void k_diag_sweep_split(DiagSweepParams<T> sp1
     }
 }
 
-// Sweeps of n right-hand sides src.psi[r] of the problem sp in place on the reference layout: items (source,
-// ordinate, band), the (source, ordinate) pairs split evenly into the XCDs' queues, each queue band-major.
-// work null: one workgroup per item, band-major.
+// Items (source, ordinate, band) of the sweeps of n right-hand sides src.psi[r] of one problem in place on the reference
+// layout: the (source, ordinate) pairs split evenly into the XCDs' queues, each queue band-major.
+struct RefItems {
+    int pairs, nb;
+    __device__ RefItems(const int n, const int nq, const int nbands) : pairs(n * nq), nb(nbands < 2 ? 1 : nbands) {}
+    __device__ int first(int x) const { return x * pairs / kXcds; }  // first pair of queue x
+    __device__ int count(int x) const { return (first(x + 1) - first(x)) * nb; }
+};
+// Makes sp the problem of position pos of queue x and returns its item number (band * nq + ordinate).
+template <typename T, int P>
+__device__ __forceinline__ unsigned ref_item(DiagSweepParams<T> &sp, const SplitSources &src, const RefItems &I, int x, int pos, T *xtr) {
+    const int p0 = I.first(x), np = I.first(x + 1) - p0, pair = p0 + pos % np, band = pos / np, r = pair / sp.nq;
+    sp.qref = src.psi[r];
+    sp.psi_ref = src.psi[r];
+    sp.xtr = xtr + (size_t)r * sp.nq * (I.nb - 1) * sp.nx * P;  // the source's exchange records
+    return (unsigned)(band * sp.nq + pair - r * sp.nq);
+}
+
+// One workgroup per item (work null: workgroup b takes item b / 8 of queue b % 8, the XCD that it is sent to), or a
+// persistent launch taking items.  The launch does nothing while *changed == mark.
 template <typename T, int P, int D>
 __global__ __launch_bounds__(512) void k_split_ref(DiagSweepParams<T> sp, SplitSources src, int n, int *__restrict__ work, int set,
                                                    const int *__restrict__ changed, int mark) {
-    const int nb = sp.nbands < 2 ? 1 : sp.nbands, pairs = n * sp.nq;
     T *const xtr = sp.xtr;
+    const RefItems I(n, sp.nq, sp.nbands);
     if (work && blockIdx.x == 0 && threadIdx.x < kXcds) work[(1 - set) * kWorkSet + threadIdx.x * kWorkStride] = 0;
     if (changed && *G(changed) == mark) return;  // the inputs are not those the tables were built from
-    auto first = [&](int x) { return x * pairs / kXcds; };
-    int pair = (int)(blockIdx.x % (unsigned)pairs), band = (int)(blockIdx.x / (unsigned)pairs);
+    int2 k{(int)(blockIdx.x % kXcds), (int)(blockIdx.x / kXcds)};
     do {
-        if (work) {
-            const int2 k = take_item(work + set * kWorkSet, [&](int x) { return (first(x + 1) - first(x)) * nb; });
-            if (k.y < 0) break;  // workgroup-uniform: every wave leaves
-            const int p0 = first(k.x), np = first(k.x + 1) - p0;
-            pair = p0 + k.y % np;
-            band = k.y / np;
-        }
-        const int r = pair / sp.nq;
-        sp.qref = src.psi[r];
-        sp.psi_ref = src.psi[r];
-        sp.xtr = xtr + (size_t)r * sp.nq * (nb - 1) * sp.nx * P;  // the source's exchange records
-        split_item<T, P, 5, D>(sp, (unsigned)(band * sp.nq + pair - r * sp.nq));
+        if (work) k = take_item(work + set * kWorkSet, [&](int x) { return I.count(x); });
+        if (k.y < 0 || k.y >= I.count(k.x)) break;  // workgroup-uniform: every wave leaves
+        split_item<T, P, 5, D>(sp, ref_item<T, P>(sp, src, I, k.x, k.y, xtr));
     } while (work);
+}
+
+// The same with a lane per coefficient and one workgroup per item: the loop of a persistent launch costs 40 registers,
+// and with them a third of the waves on a CU; the queue's atomics cost 2 us of a call.
+template <typename T, int P, int D>
+__global__ __launch_bounds__(kWideThreads) void k_wide_ref(DiagSweepParams<T> sp, SplitSources src, int n,
+                                                           const int *__restrict__ changed, int mark) {
+    const RefItems I(n, sp.nq, sp.nbands);
+    if (changed && *G(changed) == mark) return;
+    const int x = (int)(blockIdx.x % kXcds), pos = (int)(blockIdx.x / kXcds);
+    if (pos >= I.count(x)) return;  // past the end of a shorter queue
+    wide_item<T, P, 5, D>(sp, ref_item<T, P>(sp, src, I, x, pos, sp.xtr));
 }
 
 }  // namespace tsw

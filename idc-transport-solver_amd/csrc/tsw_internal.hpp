@@ -142,6 +142,7 @@ template <typename T> struct DiagSweepParams {
     // Lane-split launches only (host-side dispatch): work counters of a persistent launch, whose workgroups
     // take items until all are taken (null: one item per workgroup), and the counter set of this launch
     int *work;
+    const int32_t *mat_cell;  // material index in the cell layout [nx+2][ny+2] (lane-per-coefficient sweep)
     int work_set;
 };
 
@@ -249,6 +250,9 @@ size_t diag_sweep_lds_bytes(const DiagSweepParams<T> &sp, int p);
 // built for (T, p) or does not fit)
 template <typename T>
 size_t split_sweep_lds_bytes(int p, int rows, int M);
+// LDS bytes of the lane-per-coefficient sweep (either layout); 0 when it does not fit
+template <typename T>
+size_t wide_sweep_lds_bytes(int p, int rows, int M);
 // Batched sweep over work items {problem, ordinate}; `rep` fixes degree-independent choices (mode,
 // material path), probs/items are device arrays, lds >= diag_sweep_lds_bytes of every problem.
 template <typename T>

@@ -127,6 +127,57 @@ def test_ref_split_edges_match_the_diagonal_path(shape, persistent):
         np.testing.assert_array_equal(a, c2)
 
 
+# the lane-per-coefficient kernel: rows of a wave (4; 16 at degree 1), of a workgroup (56, 224) and of a band (24, 64),
+# columns below, at and past the 16 that its feeder holds, against the lane-split kernel (batch_split_rows set)
+WIDE_EDGES = [(1, 1, 2, 2), (2, 3, 2, 4), (15, 4, 2, 2), (16, 5, 2, 6), (17, 56, 2, 4), (33, 57, 2, 4), (40, 121, 2, 8),
+              (1, 57, 3, 2), (16, 56, 3, 4), (18, 73, 3, 6), (35, 200, 3, 4), (17, 15, 1, 2), (16, 17, 1, 4),
+              (9, 224, 1, 2), (30, 225, 1, 6), (3, 300, 1, 12)]
+
+
+@pytest.mark.parametrize("shape", WIDE_EDGES)
+def test_ref_wide_edges_match_the_lane_split_kernel(shape):
+    nx, ny, p, order = shape
+    o = ls_ordinates(order)
+    g, st, _, src = random_problem(nx, ny, p, o, seed=400 + nx + ny, materials=3)
+    print("ref wide edges", shape, flush=True)
+    for prec, tol in ((tsw.FP64, 1e-12), (tsw.FP32, 2e-6)):
+        outs = []
+        for rows in (0, 0, 32):
+            with _ctx(g, o, 1) as c:
+                if rows:
+                    c.set_tuning("batch_split_rows", rows)
+                a = src.copy()
+                for _ in range(2):  # a sweep leaves the exchange records empty for the next
+                    a[1:-1, 1:-1] = src[1:-1, 1:-1]
+                    c.sweep(a, st, 0.4, precision=prec)
+                outs.append(a)
+        assert rel_err(outs[0], orc_sweep(g, o, st, src, 0.4)) <= tol, prec
+        np.testing.assert_array_equal(outs[0], outs[2])
+        np.testing.assert_array_equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("prec", [tsw.FP64, tsw.FP32])
+def test_ref_sweeps_of_few_and_many_rows_alternate(prec):
+    """Single sweeps (a lane per coefficient) between calls with many sources (lane-split, taking items from counters)."""
+    import torch
+    o = ls_ordinates(8)
+    g, st, _, src = random_problem(6, 90, 2, o, seed=12, materials=2)
+    dev = torch.device("cuda:0")
+    with _ctx(g, o) as c:
+        st_d = torch.from_numpy(st).to(dev)
+        one = torch.from_numpy(src).to(dev)
+        c.sweep(one, st_d, math.inf, precision=prec)
+        for singles in (0, 1, 2, 3):
+            for _ in range(singles):
+                a = torch.from_numpy(src).to(dev)
+                c.sweep(a, st_d, math.inf, precision=prec)
+                assert torch.equal(a, one)
+            many = [torch.from_numpy(src).to(dev) for _ in range(7)]  # 25,200 rows
+            c.sweep_multi(many, st_d, math.inf, precision=prec)
+            for k, a in enumerate(many):
+                assert torch.equal(a, one), (singles, k)
+
+
 def test_ref_split_more_sources_than_one_launch_takes():
     import torch
     o = ls_ordinates(4)
