@@ -2443,10 +2443,10 @@ int split_band_rows(const tsw_ctx *ctx, int p, int ny) {
 
 // Rows per band of the lane-per-coefficient kernel on the reference layout, 0 where the lane-split kernel is the faster:
 // its waves hold a quarter of the rows, so it pays while the chip holds the sweep's `rows` (of all ordinates and sources)
-// at about the same time.  Kernel us, lane-split against this, S8 or S12: Q3 32 x 32 60 -> 28, 128 x 128 222 -> 115,
-// 140 x 140 197 -> 129, 256 x 256 453 -> 308, 280 x 280 (23,520 rows) 543 -> 488; Q2 32 x 32 38 -> 24, 128 x 128 142 ->
-// 108, 256 x 256 267 -> 222, 210 x 210 (17,640 rows) 283 -> 258, but 280 x 280 467 -> 477; Q1 32 x 32 26 -> 17,
-// 128 x 128 84 -> 74, 256 x 256 (10,240 rows) 187 -> 163, but 280 x 280 214 -> 220.  One band up to the most rows of a
+// at about the same time.  Kernel us, lane-split against this, S8 or S12: Q3 32 x 32 60 -> 28, 128 x 128 222 -> 104,
+// 140 x 140 197 -> 123, 256 x 256 453 -> 286, 280 x 280 (23,520 rows) 543 -> 497; Q2 32 x 32 38 -> 22, 128 x 128 142 ->
+// 91, 256 x 256 267 -> 186, 210 x 210 (17,640 rows) 283 -> 253, but 280 x 280 467 -> 477; Q1 32 x 32 26 -> 16,
+// 128 x 128 84 -> 74, 256 x 256 (10,240 rows) 187 -> 146, but 280 x 280 214 -> 220.  One band up to the most rows of a
 // workgroup; more rows than that in bands of 24 (64 at degree 1, where a row takes 4 lanes), of which a CU holds three:
 // within 3% of the best of 16 .. 56 at all these sizes.
 int wide_band_rows(const tsw_ctx *c, int p, int ny, long long rows) {

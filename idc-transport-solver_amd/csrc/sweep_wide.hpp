@@ -13,7 +13,7 @@
 // outflow are the work of two further waves, so that the compute waves, which all wait for the slowest at each barrier,
 // run the same few instructions in every row (inside the first wave it cost a third of a step).
 //
-// Measured on one band of Q2 (FP64): 0.18 us a step with 8 rows, 0.27 with 24, 0.37 with 56, where the lane-split
+// Measured on one band of Q2 (FP64): 0.18 us a step with 8 rows, 0.24 with 24, 0.37 with 56, where the lane-split
 // sweep takes 0.5; without its loads and stores 0.16, 0.20 and 0.31: what is left is the wave's own chain (LDS, 14
 // dependent FP64 operations, barrier) and, with many rows, the issue slots of a CU's four SIMDs.  Kernel times against
 // the lane-split sweep's stand at the rule that picks one (wide_band_rows).
@@ -189,37 +189,42 @@ __device__ __forceinline__ void wide_item(const DiagSweepParams<T> &sp, unsigned
         }
         // The feeder: column t + 1's y-inflow of the band's first row into LDS during step t.  Lane l holds x-degree l % 4
         // of the next column that is l / 4 modulo 16, from the records of the band below, the halo traces, or (reference
-        // layout) the halo cells.  Lanes without a value load every 4 steps and look 3 steps later, so that a band some
-        // 10 columns behind its upstream one never waits for a load.
+        // layout) the halo cells.  A load goes out every 4 steps and is looked at 7 steps later (with loads of 16 columns
+        // at once, looked at 3 steps later, Q2 128 x 128 took 108 us instead of 91: about 1 us from another CU's store to
+        // its value here held the step up), so a band some 14 columns behind
+        // its upstream one never waits.
         const gptr<const U> yin = has_in ? gptr<const U>(xin) : G(reinterpret_cast<const U *>(sp.tin_y)) + (size_t)q * nx * P;
         const bool halo = REF && !has_in, none = !REF && !has_in && sp.tin_y == nullptr;
         int mine = yc;  // this lane's column
         bool have = false;
-        U cur = 0, raw = 0;
-        double yr[P];
-        auto load = [&]() {  // (columns past the mesh: the last one, not used)
+        U cur = 0, raw[2] = {0, 0};
+        double yr[2][P];
+        int from[2] = {-1, -1};  // the column that buffer b was loaded from
+        auto load = [&](int b) {  // (columns past the mesh: the last one, not used)
+            from[b] = mine;
             const int c = mine < nx ? mine : nx - 1;
             if (halo) {
                 const int i = xneg ? nx - c : c + 1, j = yneg ? ny + 1 : 0;
-                ref_run_ld<P>(rq, (unsigned)((((long long)i * (ny + 2) + j) * sp.nq + q) * N * 8) + 8u * (unsigned)(yd * P), yr);
+                ref_run_ld<P>(rq, (unsigned)((((long long)i * (ny + 2) + j) * sp.nq + q) * N * 8) + 8u * (unsigned)(yd * P), yr[b]);
             } else if (!none) {
-                raw = xload<U>(yin + (size_t)c * P + yd);
+                raw[b] = xload<U>(yin + (size_t)c * P + yd);
             }
         };
-        auto look = [&]() {  // takes what the last load brought, if a value was missing
+        auto look = [&](int b) {  // takes what a load brought, if a value was missing
             if (halo) {
-                double s = yr[0];
+                double v = yr[b][0];
 #pragma unroll
-                for (int b = 1; b < P; ++b) s += (yneg && (b & 1)) ? -yr[b] : yr[b];
-                raw = to_bits(T(s));
+                for (int k = 1; k < P; ++k) v += (yneg && (k & 1)) ? -yr[b][k] : yr[b][k];
+                raw[b] = to_bits(T(v));
             }
-            cur = have ? cur : raw;
-            have = have || !has_in || raw != ExchangeSentinel<T>::bits;
+            // (a load that was under way when the lane moved on to another column is dropped)
+            const bool ok = !have && from[b] == mine && (!has_in || raw[b] != ExchangeSentinel<T>::bits);
+            cur = ok ? raw[b] : cur;
+            have = have || ok;
         };
         auto put = [&](int c) {
             if (c >= nx) return;
             const bool now = yc == (c & 15);
-            if ((c & 3) == 3 || c == 0) look();
             for (int it = 0; __ballot(now && !have) != 0; ++it) {
                 if (it >= kSpinLimit || ((it & 255) == 255 && xload<int>(G(sp.abort_flag)) != 0)) {
                     if (it >= kSpinLimit) xstore<int>(G(sp.abort_flag), 1);
@@ -227,22 +232,30 @@ __device__ __forceinline__ void wide_item(const DiagSweepParams<T> &sp, unsigned
                     break;
                 }
                 __builtin_amdgcn_s_sleep(1);
-                load();
-                look();
+                load(0);
+                look(0);
             }
             if (now) {
                 if ((lane & 3) < P) xs[((c + 1) & 1) * side + yd * PS] = from_bits<T>(cur);
                 have = false;
                 mine += 16;
             }
-            if ((c & 3) == 0) load();
         };
-        load();
+        load(0);
+        look(0);
         put(0);
         lds_barrier();
-        for (int t = 0; t < nbar; ++t) {
-            put(t + 1);
-            lds_barrier();
+        for (int t0 = 0; t0 < nbar; t0 += 8) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                if (t0 + k >= nbar) break;
+                if (k == 0) load(0);
+                if (k == 4) load(1);
+                if (k == 7) look(0);
+                if (k == 3 && t0 > 0) look(1);
+                put(t0 + k + 1);
+                lds_barrier();
+            }
         }
         return;
     }
