@@ -54,6 +54,26 @@ def test_sweep_degree_p_sigma_matches_oracle(p, pattern):
                 np.testing.assert_array_equal(out[0], src[0])
 
 
+# rows at the edges of a wave and of the workgroup that sweeps an ordinate (512 at degrees 0 and 1, 256 at 2, none at 3),
+# and the meshes past it, which take a launch per diagonal
+@pytest.mark.parametrize("shape", [(1, 1, 0, 2), (2, 64, 0, 4), (70, 3, 0, 2), (3, 512, 0, 2), (2, 513, 0, 2), (1, 65, 1, 4),
+                                   (66, 63, 1, 2), (2, 512, 1, 2), (3, 513, 1, 2), (5, 64, 2, 4), (1, 256, 2, 2),
+                                   (4, 257, 2, 2), (65, 2, 2, 4), (3, 5, 3, 4)])
+def test_wavefront_sweep_by_rows_matches_oracle(shape):
+    nx, ny, p, order = shape
+    g, o, st, _, src = _problem(nx, ny, p, order, seed=500 + nx + ny)
+    print("wavefront rows", shape, flush=True)
+    for deg in {0, p}:
+        sig = st if deg else np.ascontiguousarray(st[..., 0, 0])
+        with xs_degree(deg):
+            ref = orc_sweep(g, o, sig, src, 0.3)
+        with _ctx(g, o, deg, "hip-wavefront-eager") as c:
+            for prec, tol in ((tsw.FP64, 1e-12), (tsw.FP32, 2e-6)):
+                out = src.copy()
+                c.sweep(out, sig, 0.3, precision=prec)
+                assert rel_err(out, ref) <= tol, (deg, prec)
+
+
 @pytest.mark.parametrize("p", [1, 2, 3])
 def test_smv_lmv_degree_p_and_in_place_lmv(p):
     import torch
