@@ -74,6 +74,26 @@ def test_wavefront_sweep_by_rows_matches_oracle(shape):
                 assert rel_err(out, ref) <= tol, (deg, prec)
 
 
+# (cell, ordinate) pairs below, at and past a wave of 64 and a block of 256, in columns of one cell and of many
+@pytest.mark.parametrize("shape", [(1, 1, 0, 2), (1, 1, 3, 2), (4, 4, 1, 2), (16, 1, 2, 2), (1, 17, 2, 2), (3, 7, 1, 4),
+                                   (8, 8, 2, 2), (5, 13, 3, 4), (13, 5, 2, 6)])
+def test_lmv_of_part_waves_matches_oracle(shape):
+    nx, ny, p, order = shape
+    g, o, st, _, x = _problem(nx, ny, p, order, seed=700 + nx + ny)
+    y0 = np.random.default_rng(nx).uniform(-1, 1, size=x.shape)
+    for deg in {0, p}:
+        sig = st if deg else np.ascontiguousarray(st[..., 0, 0])
+        with _ctx(g, o, deg) as c:
+            for alpha, beta in ((1.0, 0.0), (-0.4, 0.7)):
+                y = y0.copy()
+                c.lmv(sig, x, y, alpha, beta)
+                with xs_degree(deg):
+                    ref = orc_lmv(g, o, sig, x, y0, alpha, beta)
+                assert rel_err(y[1:-1, 1:-1], ref[1:-1, 1:-1]) <= 1e-12, (deg, beta)
+                np.testing.assert_array_equal(y[0], y0[0])
+                np.testing.assert_array_equal(y[:, -1], y0[:, -1])
+
+
 @pytest.mark.parametrize("p", [1, 2, 3])
 def test_smv_lmv_degree_p_and_in_place_lmv(p):
     import torch
