@@ -132,7 +132,7 @@ template <typename T> struct DiagSweepParams {
     int direct;            // 1: no storer wave, the compute waves store psi (one band only; used when
                            // only that LDS layout, without the store staging buffer, fits)
     int wave1;             // 1: one wave per band of at most 64 rows, traces passed between lanes
-    int split;             // 1: lane-split kernel (2 or 4 lanes per row, material path, direct stores)
+    int split;             // 1: lane-split kernel (2 or 4 lanes per row, material path); 2: a lane per coefficient
     const int *skip;       // device flag: the launch does nothing while *skip != 0 (null: always runs)
     // Reference-layout I/O (batch members): Q from qref and psi to psi_ref ([nx+2][ny+2][nq][N] doubles,
     // may alias, 16-byte aligned) instead of qsrc / psi
@@ -258,7 +258,7 @@ size_t wide_sweep_lds_bytes(int p, int rows, int M);
 template <typename T>
 void launch_diag_sweep_batch(const DiagSweepParams<T> &rep, const DiagSweepParams<T> *probs, const int2 *items,
                              int nitems, int max_ny, size_t lds, int p, hipStream_t s);
-// Lane-split sweeps of n <= kSplitSources right-hand sides of one problem in place on the reference layout
+// Lane-split (sp.split 1) or lane-per-coefficient (2) sweeps of n <= kSplitSources right-hand sides of one problem in place on the reference layout
 // (16-byte aligned arrays below 4 GiB - 256 bytes; sp: material path, bands, sp.work / work_set; sp.prefetch the depth).
 // The launch does nothing while *changed == mark (changed not null); start and stop (or null) are recorded around it.
 template <typename T>

@@ -146,7 +146,7 @@ int tsw_set_tuning(tsw_ctx *ctx, const char *key, int value);
 
 /* Reads back "band_rows" (rows per band of the last staggered sweep, 0 = one band per ordinate),
  * "prefetch" (its prefetch depth), "one_wave" (1 if it ran the one-wavefront kernel), "lane_split" (1 if
- * it ran the lane-split kernel), "lanes" (1 if the last sweep, or for a batch context any member, ran on
+ * it ran the lane-split or lane-per-coefficient kernel), "lanes" (1 if the last sweep, or for a batch context any member, ran on
  * the ordinate-lane engine), "lanes_block" / "lanes_waves" (its shape), "batch_ref" (1 if the last
  * tsw_batch_sweep ran staggered or lane-split groups on the caller's layout), "batch_engine_p0" ..
  * "batch_engine_p3" (the engine tsw_batch_set chose for that DG degree: 0 staggered through conversions,
