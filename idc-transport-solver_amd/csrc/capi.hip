@@ -2550,7 +2550,7 @@ void split_ref_sweep(tsw_ctx *c, DiagSweepParams<T> base, size_t lds, const std:
         base.work_set = M.work.set;
         launch_split_ref<T>(base, src, k, lds, g.p, changed, mark, s, r0 == 0 ? e0 : nullptr,
                             r0 + kSplitSources >= n ? e1 : nullptr);
-        if (base.split == 1) M.work.set ^= 1;  // (the other kernel neither takes from the counters nor clears them)
+        if (work) M.work.set ^= 1;  // only a persistent launch takes from one set and clears the other
     }
     c->sweeps_done += n;
 }
@@ -4326,13 +4326,13 @@ void batch_group_launch(tsw_ctx *ctx, tsw_ctx::Group &G, bool corr, const std::v
         if (ctx->batch_persistent_opt > 0) {
             rep.work = G.work.get(ctx->stream);
             rep.work_set = G.work.set;
-            G.work.set ^= 1;
         }
     }
     const bool queues = rep.work != nullptr;
     launch_diag_sweep_batch<T>(rep, probs, queues ? G.dev_qitems.as<int2>() : G.dev_items.as<int2>(),
                                (int)(queues ? G.qitems.size() : G.items.size()) / 2, G.split ? G.rows : G.max_ny, lds,
                                G.p, sd);
+    if (queues) G.work.set ^= 1;  // launched: it takes from its set and clears the other
 }
 
 // One batched sweep over the current groups, all on the side streams, timed as one sweep.  Converted

@@ -178,6 +178,25 @@ def test_ref_sweeps_of_few_and_many_rows_alternate(prec):
                 assert torch.equal(a, one), (singles, k)
 
 
+@pytest.mark.parametrize("p,rows", [(1, 48), (2, 32), (3, 32)])
+def test_ref_split_persistent_switched_on_and_off(p, rows):
+    """A launch with one workgroup per item leaves the item counters alone: whichever launch follows takes every item."""
+    o = ls_ordinates(6)
+    g, st, _, src = random_problem(10, 100, p, o, seed=50 + p, materials=3)
+    print("ref split persistent on and off", p, flush=True)
+    with _ctx(g, o) as c:
+        c.set_tuning("batch_split_rows", rows)  # the lane-split kernel
+        first = None
+        for persistent in (1, 0, 1, 0, 0, 1, 1, 0, 1):
+            c.set_tuning("batch_persistent", persistent)
+            a = src.copy()
+            c.sweep(a, st, 0.7)
+            if first is None:
+                first = a
+                assert rel_err(a, orc_sweep(g, o, st, src, 0.7)) <= 1e-12
+            np.testing.assert_array_equal(a, first)
+
+
 def test_ref_split_more_sources_than_one_launch_takes():
     import torch
     o = ls_ordinates(4)
