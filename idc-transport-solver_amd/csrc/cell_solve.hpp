@@ -26,39 +26,44 @@ __device__ __forceinline__ T fmadd(T a, T b, T c) {
     else return __builtin_fma(a, b, c);
 }
 
-// Builds B (right-hand side) for one lane from the source and the two upwind neighbours.
+// Builds B (right-hand side) for one lane from the source and the two upwind neighbours.  Which products are rounded
+// before they are added is written out, so that every kernel rounds alike, whatever the compiler knows of the operands:
+// the couplings cx psi_up_x and cy psi_up_y are rounded and added with their coefficient, but unrounded where that is +1
+// for both directions; the source's product is rounded where the first coefficient of d has two signs (even d, P > 1),
+// fused where it has one (odd d) and at P = 1.
 template <typename T, int P>
-__device__ __forceinline__ void assemble_rhs(T (&B)[P * P], const T *__restrict__ src, const T *__restrict__ upx,
-                                             const T *__restrict__ upy, T xi, T eta, T dx, T dy) {
+__device__ __forceinline__ void assemble_rhs(T (&B)[P * P], const T *src, const T *upx, const T *upy, T xi, T eta, T dx,
+                                             T dy) {
+#pragma clang fp contract(off)
     constexpr int N = P * P;
     const bool xneg = xi <= T(0), yneg = eta <= T(0);
+    const T cx = dy * xi, cy = dx * eta, area = dx * dy;
     T W0[N], W1[N];
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-        W0[k] = upx[k] * (dy * xi);
-        W1[k] = upy[k] * (dx * eta);
+        W0[k] = cx * upx[k];
+        W1[k] = cy * upy[k];
     }
-    const T area = dx * dy;
-#pragma unroll
-    for (int k = 0; k < N; ++k) B[k] = area * src[k];
-#pragma unroll
-    for (int d = 0; d < P; ++d)
-#pragma unroll
-        for (int e = 0; e < P; ++e)
-#pragma unroll
-            for (int a = 0; a < P; ++a) {
-                const T c = xneg ? T(ipow_m1(a + 1) * (2 * d + 1)) : T(ipow_m1(d) * (2 * d + 1));
-                B[e + P * d] += W0[e + P * a] * c;
-            }
+    // acc + c w for the coefficients cn (xi or eta <= 0) and cp, w = rounded s u
+    auto add = [](T acc, bool neg, int cn, int cp, T w, T s, T u) {
+        if (cn == 1 && cp == 1) return fmadd(s, u, acc);
+        return fmadd(neg ? T(cn) : T(cp), w, acc);
+    };
 #pragma unroll
     for (int d = 0; d < P; ++d)
 #pragma unroll
-        for (int e = 0; e < P; ++e)
+        for (int e = 0; e < P; ++e) {
+            T acc;
+            if (d % 2 == 0 && P > 1) acc = add(area * src[e + P * d], xneg, -(2 * d + 1), 2 * d + 1, W0[e], cx, upx[e]);
+            else acc = fmadd(area, src[e + P * d], W0[e] * (xneg ? T(-(2 * d + 1)) : T(ipow_m1(d) * (2 * d + 1))));
 #pragma unroll
-            for (int b = 0; b < P; ++b) {
-                const T c = yneg ? T(ipow_m1(b + 1) * (2 * e + 1)) : T(ipow_m1(e) * (2 * e + 1));
-                B[e + P * d] += W1[b + P * d] * c;
-            }
+            for (int a = 1; a < P; ++a)
+                acc = add(acc, xneg, ipow_m1(a + 1) * (2 * d + 1), ipow_m1(d) * (2 * d + 1), W0[e + P * a], cx, upx[e + P * a]);
+#pragma unroll
+            for (int b = 0; b < P; ++b)
+                acc = add(acc, yneg, ipow_m1(b + 1) * (2 * e + 1), ipow_m1(e) * (2 * e + 1), W1[b + P * d], cy, upy[b + P * d]);
+            B[e + P * d] = acc;
+        }
 }
 
 // Builds A = Aq + diag_add * I (column-major, A[row + N*col]).

@@ -35,51 +35,6 @@ __device__ __forceinline__ void cell_matrix(T (&A)[P * P * P * P], const SweepPa
     }
 }
 
-// assemble_rhs with the multiply-adds written out as they are contracted in k_sweep_diag, so that both kernels round
-// alike whatever the compiler knows of the operands: a coefficient of +1 adds the unrounded product; where the first
-// coefficient of a sum has one sign for both directions (odd degree), the source's product is the fused one.
-template <typename T, int P>
-__device__ __forceinline__ void rows_rhs(T (&B)[P * P], const T (&src)[P * P], const T (&upx)[P * P], const T (&upy)[P * P],
-                                         T xi, T eta, T dx, T dy) {
-    constexpr int N = P * P;
-    const bool xneg = xi <= T(0), yneg = eta <= T(0);
-    const T cx = dy * xi, cy = dx * eta, area = dx * dy;
-    T W0[N], W1[N];
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-        W0[k] = cx * upx[k];
-        W1[k] = cy * upy[k];
-        asm volatile("" : "+v"(W0[k]), "+v"(W1[k]));  // (rounded)
-    }
-    // acc + c w for the coefficients cn (xi or eta <= 0) and cp, w = rounded s u
-    auto add = [](T acc, bool neg, int cn, int cp, T w, T s, T u) {
-        if (cn == 1 && cp == 1) return fmadd(s, u, acc);
-        return fmadd(neg ? T(cn) : T(cp), w, acc);
-    };
-#pragma unroll
-    for (int d = 0; d < P; ++d)
-#pragma unroll
-        for (int e = 0; e < P; ++e) {
-            T acc;
-            if (d % 2 == 0) {
-                T as = area * src[e + P * d];
-                asm volatile("" : "+v"(as));
-                acc = add(as, xneg, -(2 * d + 1), 2 * d + 1, W0[e], cx, upx[e]);
-            } else {
-                T w = W0[e] * T(2 * d + 1);
-                asm volatile("" : "+v"(w));
-                acc = fmadd(area, src[e + P * d], -w);
-            }
-#pragma unroll
-            for (int a = 1; a < P; ++a)
-                acc = add(acc, xneg, ipow_m1(a + 1) * (2 * d + 1), ipow_m1(d) * (2 * d + 1), W0[e + P * a], cx, upx[e + P * a]);
-#pragma unroll
-            for (int b = 0; b < P; ++b)
-                acc = add(acc, yneg, ipow_m1(b + 1) * (2 * e + 1), ipow_m1(e) * (2 * e + 1), W1[b + P * d], cy, upy[b + P * d]);
-            B[e + P * d] = acc;
-        }
-}
-
 // Most rows of a workgroup of k_sweep_rows: 8 waves, two a SIMD (with more, the SIMDs of the one CU that an ordinate has
 // would take longer than a launch per diagonal spread over the chip), 4 at degree 2 for 512 registers a lane; none at
 // degree 3, whose 16 x 16 matrix spills either way and where one CU an ordinate loses (40 x 40 S4 FP64: 2.59 against
@@ -144,8 +99,7 @@ __global__ __launch_bounds__(sweep_rows_most<P>() ? sweep_rows_most<P>() : 64) v
             cell_matrix<T, P>(A, sp, xi, eta, sig, sp.xs ? (AHEAD ? tc : tcell) : nullptr);
 #pragma unroll
             for (int k = 0; k < N; ++k) up[k] = first ? halo[k] : last[(((t + 1) & 1) * N + k) * R + r - 1];
-            if constexpr (P == 1) assemble_rhs<T, P>(B, src, x, up, xi, eta, sp.dx, sp.dy);
-            else rows_rhs<T, P>(B, src, x, up, xi, eta, sp.dx, sp.dy);
+            assemble_rhs<T, P>(B, src, x, up, xi, eta, sp.dx, sp.dy);
             load(c + 1);
             ge_solve<T, N>(A, B);
             if (now) {

@@ -74,6 +74,30 @@ def test_wavefront_sweep_by_rows_matches_oracle(shape):
                 assert rel_err(out, ref) <= tol, (deg, prec)
 
 
+@pytest.mark.parametrize("nx,p,rows", [(5, 0, 300), (7, 1, 270), (4, 2, 150)])
+def test_wavefront_kernels_give_the_same_bits(nx, p, rows):
+    """A mesh of 2 * rows rows (a launch per diagonal) against its two halves (one launch each): upward ordinates see
+    the lower half alone, downward ones the upper half."""
+    ny = 2 * rows
+    g, o, st, _, src = _problem(nx, ny, p, 4, seed=600 + nx)
+    up = np.asarray(o.eta) > 0
+    print("wavefront kernels", nx, ny, p, flush=True)
+    for deg in {0, p}:
+        sig = st if deg else np.ascontiguousarray(st[..., 0, 0])
+        for prec in (tsw.FP64, tsw.FP32):
+            outs = []
+            for j0, n in ((0, ny), (0, rows), (rows, rows)):  # dy is 1/64 in each
+                with tsw.Context(0) as c:
+                    c.problem_set(nx, n, p, o.xi, o.eta, o.w, o.quad_off, 0.0, nx / 32.0, 0.0, n / 64.0)
+                    c.set_pattern("hip-wavefront-eager")
+                    c.set_xs_degree(deg)
+                    out = src[:, j0:j0 + n + 2].copy()
+                    c.sweep(out, np.ascontiguousarray(sig[:, j0:j0 + n + 2]), 0.3, precision=prec)
+                    outs.append(out[1:-1, 1:-1])
+            np.testing.assert_array_equal(outs[0][:, :rows, up], outs[1][:, :, up])
+            np.testing.assert_array_equal(outs[0][:, rows:, ~up], outs[2][:, :, ~up])
+
+
 # (cell, ordinate) pairs below, at and past a wave of 64 and a block of 256, in columns of one cell and of many
 @pytest.mark.parametrize("shape", [(1, 1, 0, 2), (1, 1, 3, 2), (4, 4, 1, 2), (16, 1, 2, 2), (1, 17, 2, 2), (3, 7, 1, 4),
                                    (8, 8, 2, 2), (5, 13, 3, 4), (13, 5, 2, 6)])
