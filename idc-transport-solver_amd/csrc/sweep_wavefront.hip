@@ -147,14 +147,29 @@ __global__ __launch_bounds__(256) void k_sweep_diag(SweepParams<T> sp, int diag,
     for (int k = 0; k < N; ++k) self[k] = B[k];
 }
 
+// Most workgroups of k_sweep_rows a CU, by the waves of one: with more, a step waits for the other workgroups of its SIMD
+// or they run one after the other, and a launch per diagonal, spread over the chip, is the faster.  One launch against a
+// launch per diagonal, us, FP64, at and past the line: Q0 100 x 256 768 ordinates 658 and 849, 1024 930 and 846; Q1 100 x
+// 128 737 and 870, 1024 1206 and 1013, 100 x 256 512 1010 and 1270, 640 1731 and 1320, 60 x 512 256 869 and 1640, 320 1960
+// and 1880; Q2 100 x 128 512 878 and 1520, with degree-2 cross sections 640 2340 and 2080, 100 x 256 256 1776 and 3040, 320
+// 3341 and 3210.  FP32 differs at Q2 with one wave: 100 x 16 512 ordinates 355 and 543, 640 565 and 554.
+template <typename T, int P>
+constexpr int sweep_rows_per_cu(int waves) {
+    if (P == 1) return waves <= 2 ? 4 : 3;
+    if (P == 2) return waves == 1 ? 4 : waves == 2 ? 3 : waves <= 4 ? 2 : 1;
+    return waves == 1 ? (sizeof(T) == 8 ? 4 : 2) : waves == 2 ? 2 : 1;
+}
+
 template <typename T, int P>
 static void sweep_wavefront_p(const SweepParams<T> &sp, hipStream_t s) {
-    // One workgroup per ordinate while its rows fit one, in place of nx + ny - 1 launches of about 3 us each.  Before and
-    // after, FP64: Q1 64 x 64 S8 324 -> 171 us, with degree-1 cross sections 450 -> 127, 200 x 200 1.10 -> 0.58 ms, 150 x
-    // 500 S4 1.84 -> 0.94; Q2 64 x 64 S8 621 -> 400 us, with degree-2 cross sections 961 -> 493, 200 x 250 2.33 -> 1.49 ms.
+    // One workgroup per ordinate while its rows fit one and a CU has few of them, in place of nx + ny - 1 launches of about
+    // 3 us each.  Before and after, FP64: Q1 64 x 64 S8 324 -> 171 us, with degree-1 cross sections 450 -> 127, 200 x 200
+    // 1.10 -> 0.58 ms, 150 x 500 S4 1.84 -> 0.94; Q2 64 x 64 S8 621 -> 400 us, with degree-2 cross sections 961 -> 493,
+    // 200 x 250 2.33 -> 1.49 ms.
     if constexpr (sweep_rows_most<P>() > 0) {
-        if (sp.ny <= sweep_rows_most<P>()) {
-            const int threads = (sp.ny + 63) / 64 * 64;
+        const int waves = (sp.ny + 63) / 64;
+        if (sp.ny <= sweep_rows_most<P>() && sp.nq <= kCus * sweep_rows_per_cu<T, P>(waves)) {
+            const int threads = 64 * waves;
             const size_t lds = (size_t)2 * P * P * threads * sizeof(T);  // 36 KB at most
             hipLaunchKernelGGL((k_sweep_rows<T, P>), dim3(sp.nq), dim3(threads), lds, s, sp);
             TSW_HIP(hipGetLastError());

@@ -174,6 +174,7 @@ template <typename T> struct LanesParams {
     const int *skip;            // device flag: the launch does nothing while *skip != 0 (null: always runs)
     int *work;                  // batch launches (host-side dispatch): counter of a persistent launch, or null
 };
+constexpr int kCus = 256;  // compute units of an MI355X
 constexpr int kXcds = 8;  // MI355X: workgroup b runs on XCD b mod 8, each XCD with its own L2
 // Device words of a lane-split launch's work counters (sweep_split.hpp), cleared when allocated: two sets, and
 // the kXcds + 1 queue bounds of a batch launch from word kSplitWorkTable on.

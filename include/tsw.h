@@ -68,8 +68,9 @@ int tsw_problem_set(tsw_ctx *ctx, int nx, int ny, double ax, double bx, double a
                     const double *xi, const double *eta, const double *w, const int *quad_off);
 
 /* Selects the traversal, as the `sweep_pattern` factory key does (SweepPattern.cpp:314-359):
- *   "hip-wavefront"        one workgroup per ordinate (up to 512 rows at degrees 0 and 1, 256 at degree 2),
- *                          else one launch per diagonal i+j = const, all quadrants per launch, replayed
+ *   "hip-wavefront"        one workgroup per ordinate (up to 512 rows at degrees 0 and 1, 256 at degree 2,
+ *                          and 256 to 1,024 ordinates by degree and rows), else one launch per
+ *                          diagonal i+j = const, all quadrants per launch, replayed
  *                          from a captured HIP graph; reference layout;
  *   "hip-wavefront-eager"  the same launches issued directly;
  *   "hip-staggered"        (default) one launch per sweep, one workgroup per ordinate, a diagonal per

@@ -15,8 +15,8 @@ import pytest
 
 import idc
 import tsw
-from _common import (OracleIdcOps, ls_ordinates, orc_gmres, orc_lmv, orc_pmv, orc_si, orc_smv, orc_sweep,
-                     random_poly_sigma, random_problem, rel_err, xs_degree)
+from _common import (OracleIdcOps, Ordinates, ls_ordinates, orc_gmres, orc_lmv, orc_pmv, orc_si, orc_smv, orc_sweep,
+                     random_ordinates, random_poly_sigma, random_problem, rel_err, xs_degree)
 
 pytestmark = pytest.mark.gpu
 
@@ -96,6 +96,29 @@ def test_wavefront_kernels_give_the_same_bits(nx, p, rows):
                     outs.append(out[1:-1, 1:-1])
             np.testing.assert_array_equal(outs[0][:, :rows, up], outs[1][:, :, up])
             np.testing.assert_array_equal(outs[0][:, rows:, ~up], outs[2][:, :, ~up])
+
+
+# more ordinates than one workgroup each pays for (256 times 4 to 1, by degree and rows): a launch per diagonal, against a
+# subset of the ordinates in one launch
+@pytest.mark.parametrize("shape", [(2, 3, 0, 257), (2, 130, 0, 193), (2, 64, 1, 257), (3, 65, 1, 193), (2, 129, 1, 129),
+                                   (2, 257, 1, 65), (3, 4, 2, 257), (2, 66, 2, 129), (2, 130, 2, 65)])
+def test_wavefront_sweep_of_many_ordinates(shape):
+    nx, ny, p, per_quad = shape
+    rng = np.random.default_rng(ny)
+    o = random_ordinates(per_quad, rng)
+    few = np.concatenate([np.arange(k * per_quad, k * per_quad + 8) for k in range(4)])
+    s = Ordinates(o.xi[few].copy(), o.eta[few].copy(), o.w[few].copy(), np.arange(0, 33, 8, dtype=np.int32))
+    g, st, _, src = random_problem(nx, ny, p, o, seed=650 + ny)
+    print("wavefront ordinates", shape, flush=True)
+    for prec, tol in ((tsw.FP64, 1e-12), (tsw.FP32, 2e-6)):
+        with _ctx(g, o, 0, "hip-wavefront-eager") as c:
+            a = src.copy()
+            c.sweep(a, st, 0.3, precision=prec)
+        with _ctx(g, s, 0, "hip-wavefront-eager") as c:
+            b = np.ascontiguousarray(src[:, :, few])
+            c.sweep(b, st, 0.3, precision=prec)
+        np.testing.assert_array_equal(a[:, :, few], b)
+        assert rel_err(a, orc_sweep(g, o, st, src, 0.3)) <= tol, prec
 
 
 # (cell, ordinate) pairs below, at and past a wave of 64 and a block of 256, in columns of one cell and of many
