@@ -51,6 +51,7 @@ struct tsw_ctx {
         bool have64 = false, have32 = false;
         DBuf key;            // device copy of the sigma_t the table was built from
         bool keyed = false;  // key holds that copy
+        bool settled = false;  // the last check found the sigma_t of the table, or there was no table to check
         unsigned long long build = 0;  // counts builds and cross-section changes
     } mat;
     DBuf same_flag;  // device flags of the input change checks
@@ -588,6 +589,7 @@ void prepare_materials(tsw_ctx *c, const double *sigma, double dt) {
     }
     const Geom &g = c->g;
     const bool same = same_as_key(c, sigma, g.ncell_h(), m.key, m.keyed);
+    m.settled = same || !m.keyed;
     m.keyed = true;
     if (same) {
         if (m.inv_dt != inverse_dt(dt)) {
@@ -2487,7 +2489,6 @@ bool split_ref_plan(tsw_ctx *c, const double *sig, double dt, bool known, int n,
         c->mat.have64 = c->mat.have32 = false;
     }
     if (!c->mat.valid) return false;
-    diag_materials(c);
     base = make_diag_params<T>(c, dt, nullptr, nullptr, false, nullptr);
     if (!base.ainv) return false;
     int br = split_band_rows(c, g.p, g.ny);
@@ -2500,6 +2501,9 @@ bool split_ref_plan(tsw_ctx *c, const double *sig, double dt, bool known, int n,
         lds = l;
         base.split = 2;
         base.mat_cell = c->mat.idx.as<int32_t>();
+    } else {
+        diag_materials(c);
+        base.mat = c->diag.mat.as<int32_t>();
     }
     base.direct = 0;
     base.wave1 = 0;
@@ -2565,8 +2569,10 @@ bool try_split_ref(tsw_ctx *c, const std::vector<double *> &arr, const double *s
     size_t lds = 0;
     // A call with the cross sections of the last table (the usual one) queues their check and the sweep together and
     // waits once: the sweep does nothing where the check has found a difference, and then the table is rebuilt below.
-    // Checked first and swept after the answer, the call waited twice, about 15 us of a 65 us call on a small mesh.
-    if (c->mat.keyed && c->mat.valid && c->mat.key.bytes >= c->g.ncell_h() * sizeof(double) &&
+    // Checked first and swept after the answer, the call waited twice, about 15 us of a 65 us call on a small mesh; but
+    // where they change from call to call, the idle sweep and its wait would cost as much again, and after a check that
+    // has found a difference the next call checks first.
+    if (c->mat.keyed && c->mat.valid && c->mat.settled && c->mat.key.bytes >= c->g.ncell_h() * sizeof(double) &&
         split_ref_plan<T>(c, sig, dt, true, (int)arr.size(), base, lds)) {
         int *changed = static_cast<int *>(c->changed.reserve(sizeof(int)));
         int *host = flags_of(c);
@@ -2584,6 +2590,8 @@ bool try_split_ref(tsw_ctx *c, const std::vector<double *> &arr, const double *s
         }
         c->sweeps_done -= (long long)arr.size();  // the sweep that did nothing
         c->ev_used -= 2;
+        // (the answer for the table's own check: another comparison and wait, about 25 us)
+        c->key_checks.push_back({&c->mat.key, sig, c->g.ncell_h(), false});
     }
     if (!split_ref_plan<T>(c, sig, dt, false, (int)arr.size(), base, lds)) return false;
     split_ref_sweep<T>(c, base, lds, arr, nullptr, 0);

@@ -234,6 +234,22 @@ def test_ref_split_follows_changes_of_the_inputs(p):
                 assert c.sweep_timing(reset=True)[0] == 1 or sig is many, (k, prec)
 
 
+@pytest.mark.parametrize("rows", [0, 32])
+def test_ref_split_and_diagonal_path_follow_the_same_changes(rows):
+    """Sweeps on either layout by turns on one context, with other cross sections each time: the kernels read the material
+    index in different layouts (rows 0: the cells', 32: the diagonals' in both)."""
+    o = ls_ordinates(4)
+    g, st, _, src = random_problem(12, 40, 2, o, seed=77, materials=3)
+    sigs = [st, st[::-1, ::-1].copy(), 1.5 * st, np.where(st > st.mean(), 0.7, st)]
+    with _ctx(g, o) as c:
+        c.set_tuning("batch_split_rows", rows)
+        for k in range(12):
+            c.set_tuning("ref_split", (1, 1, -1)[k % 3])
+            out = src.copy()
+            c.sweep(out, sigs[k % 4], 0.3)
+            assert rel_err(out, orc_sweep(g, o, sigs[k % 4], src, 0.3)) <= 1e-12, k
+
+
 def test_ref_split_tuning_key():
     o = ls_ordinates(4)
     g, st, _, src = random_problem(5, 5, 1, o, seed=1)
