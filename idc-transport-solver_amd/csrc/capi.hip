@@ -143,7 +143,7 @@ struct tsw_ctx {
         // lane-split kernel (on the caller's layout, or on the diagonal layout when a call's arrays are not
         // 16-byte aligned): members in row bands of at most `rows` rows, items {slot, band * nq + ordinate}
         bool split = false;
-        int rows = 0;
+        int rows = 0, storers64 = 0, storers32 = 0;
         SplitWork work;  // persistent launch: the item counters, and its items ordered by queue
         std::vector<int> qitems;
         DBuf dev_qitems;
@@ -220,7 +220,8 @@ struct tsw_ctx {
     int batch_ref_opt = 0;   // batch engines: 1 / -1 force / forbid the reference-layout staggered groups
     // batch engines: 1 / -1 force / forbid the lane-split groups (tuning key batch_split); their rows per
     // band (batch_split_rows, 0: the most one workgroup holds) and prefetch depth (batch_split_prefetch)
-    int batch_split_opt = 0, batch_split_rows_opt = 0, batch_split_pf_opt = 0;
+    int batch_split_opt = 0, batch_split_rows_opt = 0, batch_split_pf_opt = 0, batch_split_storers_opt = 0;
+    int split_storers_p[4] = {kSplitStorers, kSplitStorers, kSplitStorers, kSplitStorers};  // storer waves of its FP64 groups
     int split_rows_p[4] = {0, 0, 0, 0};  // rows per band of the lane-split engine per DG degree (autotuned; 0: most)
     // lane-split groups: runs of this many consecutive items go to one XCD (tuning key batch_xcd_tile;
     // 0 or 1: dispatch order)
@@ -2429,16 +2430,51 @@ void multi_sweep(tsw_ctx *c, const std::vector<double *> &arr, const double *sig
 // Lanes per mesh row of the lane-split kernel for DG degree p (split_lanes<p + 1>).
 int split_lanes_of(int p) { return p == 1 ? 2 : 4; }
 
+// Storer waves of a lane-split workgroup on the reference layout.  They take stores off the compute waves, which is what
+// large meshes and calls that the chip holds at once gain from, but also registers: the waves of a workgroup go round the
+// four SIMDs, so that six (64 rows at degrees 2 and 3) leave no room for a second workgroup on a CU where a SIMD holds
+// three (FP64 Q2, FP32 Q3: 161 to 178 VGPRs) and a third of the rows are in flight.
+//
+// A batch's group (64 materials, us, with and without): degree 1 with, 64 x 48^2 S12 261 and 318, 24 x 200^2 S8 1221 and
+// 1317.  FP32 degree 2 with: 467 and 522, 1921 and 2419.  FP32 degree 3 without: 32 x 48^2 S12 941 and 730, 32 x 100^2 S12
+// 2423 and 1943, 24 x 200^2 S8 2478 and 2462.  FP64 degrees 2 and 3 as the batch's autotuner finds: Q2 32 x 48^2 694 and
+// 545, but 24 x 200^2 2220 and 2396; Q3 48^2 1196 and 1310, but, by bands of up to 128 rows in place of 96, 100^2 2954 and
+// 2196 (CUs with one workgroup for their LDS, which then has seven compute waves, not four).
+// (a row count that leaves no room for them means none)
+int storers_forced(const tsw_ctx *c, int p) {
+    if (c->batch_split_storers_opt != 0) return c->batch_split_storers_opt > 0 ? kSplitStorers : 0;
+    return c->batch_split_rows_opt > (512 - 64 * kSplitStorers) / split_lanes_of(p) ? 0 : -1;
+}
+template <typename T>
+int batch_storers(const tsw_ctx *c, int p) {
+    const int forced = storers_forced(c, p);
+    return forced >= 0 ? forced : sizeof(T) == 8 ? c->split_storers_p[p] : p == 3 ? 0 : kSplitStorers;
+}
+// n sources of one problem (64 materials, us, with and without): single sweeps gain from them, 280 x 280 S12 Q2 497 and 585,
+// Q3 579 and 663, FP32 553 and 677.  FP32 Q3 without on short rows of cells: 64 x 64 S12, 32 sources 1058 and 822, 100 x 100
+// S12, 12 sources 837 and 733, but 128 x 128 S8, 8 sources 438 and 518.  FP64 Q3 without where that saves a band of at most
+// 128 rows and each CU has several: 100 x 100 S12, 12 sources (1,008 ordinates) 1072 and 819, 128 x 128 S8, 16 sources
+// (640) 889 and 851, but 8 sources (320) 547 and 565.
+template <typename T>
+int ref_storers(const tsw_ctx *c, int n) {
+    const Geom &g = c->g;
+    const int forced = storers_forced(c, g.p);
+    if (forced >= 0) return forced;
+    if (g.p < 3) return kSplitStorers;
+    if (sizeof(T) == 4) return n > 1 && g.nx <= 100 ? 0 : kSplitStorers;
+    return g.ny <= 256 && (g.ny + 127) / 128 < (g.ny + 95) / 96 && n * g.nq >= 512 ? 0 : kSplitStorers;
+}
+
 // Rows per band of a problem (a batch member, or a single problem) on the lane-split kernel: the fewest
 // bands of at most R rows (R: the tuning key batch_split_rows, else the batch autotuner's choice for the
-// degree, else the rows one workgroup of 512 threads, two storer waves among them, holds, or 64 at degree 2),
+// degree, else the rows one workgroup of 512 threads, its storer waves among them, holds, or 64 at degree 2),
 // split evenly.  Degree 2: four compute waves, one per SIMD, against six (256 x 256, S8, 64 materials, FP64: 270 against
 // 296 us; 280 x 280 S12 lattice: 468 against 481); degrees 1 and 3 lose with fewer rows (a longer chain of bands:
 // 280 x 280 Q1 246 against 215 us).
-int split_band_rows(const tsw_ctx *ctx, int p, int ny) {
-    int R = p == 2 ? 64 : 384 / split_lanes_of(p);
+int split_band_rows(const tsw_ctx *ctx, int p, int ny, int storers) {
+    const int most = (512 - 64 * storers) / split_lanes_of(p);
     const int want = ctx->batch_split_rows_opt > 0 ? ctx->batch_split_rows_opt : ctx->split_rows_p[p & 3];
-    if (want > 0) R = std::min(R, want);
+    const int R = want > 0 ? std::min(most, want) : p == 2 ? 64 : most;
     const int nb = (ny + R - 1) / R;
     return (ny + nb - 1) / nb;
 }
@@ -2458,11 +2494,13 @@ int wide_band_rows(const tsw_ctx *c, int p, int ny, long long rows) {
 }
 
 // Prefetch depth of the lane-split kernel on the reference layout: 3 for FP64 Q3, whose ring of 4 spills (256 x 256, S8,
-// 64 materials: 461 against 556 us), else kSplitBatchPrefetch, unless the tuning key batch_split_prefetch sets it.
+// 64 materials: 461 against 556 us), and for several sources of FP32 Q2 (k_split_ref: 121 VGPRs in place of 129, four
+// waves a SIMD; 48 x 48 S12, 16 sources 307 -> 216 us, 128 x 128 S8, 32 sources 1132 -> 1100, but a single 250 x 250 S16
+// sweep 665 -> 723), else kSplitBatchPrefetch, unless the tuning key batch_split_prefetch sets it.
 template <typename T>
-int split_prefetch(const tsw_ctx *c, int p) {
+int split_prefetch(const tsw_ctx *c, int p, int sources = 1) {
     if (c->batch_split_pf_opt > 0) return c->batch_split_pf_opt;
-    return p == 3 && sizeof(T) == 8 ? 3 : kSplitBatchPrefetch;
+    return (p == 3 && sizeof(T) == 8) || (p == 2 && sizeof(T) == 4 && sources > 1) ? 3 : kSplitBatchPrefetch;
 }
 
 // Whether this context's sweeps can run the staggered kernel on the caller's layout for `psi`.
@@ -2491,8 +2529,9 @@ bool split_ref_plan(tsw_ctx *c, const double *sig, double dt, bool known, int n,
     if (!c->mat.valid) return false;
     base = make_diag_params<T>(c, dt, nullptr, nullptr, false, nullptr);
     if (!base.ainv) return false;
-    int br = split_band_rows(c, g.p, g.ny);
-    lds = split_sweep_lds_bytes<T>(g.p, br, base.M);
+    base.storers = ref_storers<T>(c, n);
+    int br = split_band_rows(c, g.p, g.ny, base.storers);
+    lds = split_sweep_lds_bytes<T>(g.p, br, base.M, base.storers);
     if (lds == 0) return false;
     base.split = 1;
     const int wr = wide_band_rows(c, g.p, g.ny, (long long)n * g.nq * g.ny);
@@ -2538,7 +2577,7 @@ void split_ref_sweep(tsw_ctx *c, DiagSweepParams<T> base, size_t lds, const std:
         base.abort_flag = abort_flag_of(c);
     }
     // (a ring of 3 takes 2 to 4% longer with a lane per coefficient, one of 6 up to 20%)
-    base.prefetch = base.split == 2 && c->batch_split_pf_opt == 0 ? 4 : split_prefetch<T>(c, g.p);
+    base.prefetch = base.split == 2 && c->batch_split_pf_opt == 0 ? 4 : split_prefetch<T>(c, g.p, n);
     if (c->stall_test && per) {  // tuning key stall_test: every bounded wait of the banded sweep gives up
         c->stall_test = false;
         (void)abort_flag_of(c);
@@ -3209,6 +3248,9 @@ int tsw_set_tuning(tsw_ctx *ctx, const char *key, int value) {
         } else if (k == "batch_split_rows") {
             require(value == 0 || (value >= 16 && value <= 256), TSW_E_ARG, "batch_split_rows must be 0 or 16..256");
             ctx->batch_split_rows_opt = value;
+        } else if (k == "batch_split_storers") {
+            require(value >= -1 && value <= 1, TSW_E_ARG, "batch_split_storers must be -1, 0 or 1");
+            ctx->batch_split_storers_opt = value;
         } else if (k == "ref_split") {
             require(value == -1 || value == 1, TSW_E_ARG, "ref_split must be -1 or 1");
             ctx->ref_split_opt = value;
@@ -3282,6 +3324,7 @@ int tsw_get_tuning(tsw_ctx *ctx, const char *key, int *value) {
         else if (k == "batch_split_rows") *value = ctx->batch_split_rows_opt;
         else if (k == "batch_xcd_tile") *value = ctx->batch_xcd_tile_opt;
         else if (k == "batch_persistent") *value = ctx->batch_persistent_opt;
+        else if (k == "batch_split_storers") *value = ctx->batch_split_storers_opt;
         else if (k == "ref_split") *value = ctx->ref_split_opt;
         else if (k == "batch_split_prefetch")
             *value = ctx->batch_split_pf_opt > 0 ? ctx->batch_split_pf_opt : kSplitBatchPrefetch;
@@ -3913,6 +3956,7 @@ int tsw_batch_set(tsw_ctx *ctx, int nprob, const tsw_problem *probs, const doubl
         ctx->lanes_able.assign(nprob, 0);
         ctx->split_able.assign(nprob, 0);
         for (int &r : ctx->split_rows_p) r = 0;
+        for (int &n : ctx->split_storers_p) n = kSplitStorers;
         ctx->batch_all.resize(nprob);
         for (int b = 0; b < nprob; ++b) ctx->batch_all[b] = b;
         ctx->batch_dt = dt;
@@ -3942,12 +3986,16 @@ int tsw_batch_set(tsw_ctx *ctx, int nprob, const tsw_problem *probs, const doubl
             ctx->lanes_able[b] = ctx->lanes_opt >= 0 && lanes_ok(sub.get()) && sub->mat.valid &&
                                  diag_inverses<double>(sub.get(), dt) && diag_inverses<float>(sub.get(), dt);
             // the lane-split kernel where it is built for the degree and the member's tables fit its LDS
-            const int sbr = g.p >= 1 ? split_band_rows(ctx, g.p, g.ny) : 0;
-            ctx->split_able[b] = ctx->batch_split_opt >= 0 && g.p >= 1 && sub->mat.valid &&
-                                 g.npsi() * sizeof(double) <= kSplitRefBytes &&
-                                 diag_inverses<double>(sub.get(), dt) && diag_inverses<float>(sub.get(), dt) &&
-                                 split_sweep_lds_bytes<double>(g.p, sbr, sub->mat.M) != 0 &&
-                                 split_sweep_lds_bytes<float>(g.p, sbr, sub->mat.M) != 0;
+            bool fits = ctx->batch_split_opt >= 0 && g.p >= 1 && sub->mat.valid && g.npsi() * sizeof(double) <= kSplitRefBytes &&
+                        diag_inverses<double>(sub.get(), dt) && diag_inverses<float>(sub.get(), dt);
+            const int forced = g.p >= 1 ? storers_forced(ctx, g.p) : 0;
+            for (int st : {0, kSplitStorers}) {
+                if (!fits || (forced >= 0 && st != forced)) continue;
+                const int br = split_band_rows(ctx, g.p, g.ny, st);
+                fits = split_sweep_lds_bytes<double>(g.p, br, sub->mat.M, st) != 0 &&
+                       split_sweep_lds_bytes<float>(g.p, br, sub->mat.M, st) != 0;
+            }
+            ctx->split_able[b] = fits;
             ctx->batch.push_back(std::move(sub));
         }
         ctx->batch_ref_ok = true;  // 32-bit byte offsets into every member's array
@@ -4015,7 +4063,7 @@ void batch_group_params(tsw_ctx *ctx, tsw_ctx::Group &G, bool corr, const std::v
                 sp.xtr = lanes_records<T>(sub, sp.nbands);
                 sp.abort_flag = abort_flag_of(ctx);  // a stall is reported (and the records refilled) by sync(ctx)
             }
-            const size_t b = split_sweep_lds_bytes<T>(g.p, G.rows, sp.M);
+            const size_t b = split_sweep_lds_bytes<T>(g.p, G.rows, sp.M, sizeof(T) == 8 ? G.storers64 : G.storers32);
             require(b != 0, TSW_E_UNSUPPORTED, "lane-split batch group does not fit one CU's LDS");
             lds = std::max(lds, b);
         }
@@ -4213,7 +4261,8 @@ void build_batch_groups(tsw_ctx *ctx, const std::vector<int> &members) {
         const bool split = e == tsw_ctx::kEngSplit;
         // staggered groups hold members of equal waves per workgroup, split groups of equal row slots
         const int rpw = split ? 64 / split_lanes_of(sub->g.p) : 64;
-        const int br = split ? split_band_rows(ctx, sub->g.p, sub->g.ny) : sub->g.ny;
+        const int st64 = split ? batch_storers<double>(ctx, sub->g.p) : 0;  // (FP32 has as many or none: the bands fit)
+        const int br = split ? split_band_rows(ctx, sub->g.p, sub->g.ny, st64) : sub->g.ny;
         const auto key = std::make_tuple(sub->g.p, (br + rpw - 1) / rpw, sub->mat.valid, e);
         auto it = gid.find(key);
         if (it == gid.end()) {
@@ -4225,6 +4274,8 @@ void build_batch_groups(tsw_ctx *ctx, const std::vector<int> &members) {
             G.mat = sub->mat.valid;
             G.ref = e == tsw_ctx::kEngRef || split;
             G.split = split;
+            G.storers64 = st64;
+            G.storers32 = split ? batch_storers<float>(ctx, sub->g.p) : 0;
         }
         auto &G = ctx->groups[it->second];
         G.members.push_back(b);
@@ -4331,6 +4382,7 @@ void batch_group_launch(tsw_ctx *ctx, tsw_ctx::Group &G, bool corr, const std::v
     if (G.split) {
         rep.split = 1;
         rep.prefetch = split_prefetch<T>(ctx, G.p);
+        rep.storers = !rep.qref ? 0 : sizeof(T) == 8 ? G.storers64 : G.storers32;
         if (ctx->batch_persistent_opt > 0) {
             rep.work = G.work.get(ctx->stream);
             rep.work_set = G.work.set;
@@ -4545,16 +4597,23 @@ void batch_choose_engines(tsw_ctx *ctx) {
                 cand.push_back(tsw_ctx::kEngConverted);
             if (cand.empty()) cand.push_back(tsw_ctx::kEngConverted);
         }
-        // the lane-split engine is tried with the most rows one workgroup holds and with 64-row bands
-        // (smaller workgroups, more of them per CU where the tables leave room), unless rows are set
-        std::vector<std::pair<char, int>> tries;
+        // the lane-split engine is tried at degree 1 with the most rows one workgroup holds and with 64-row bands
+        // (smaller workgroups, more of them per CU), at degrees 2 and 3 with and without storer waves, unless set
+        struct Try {
+            char engine;
+            int rows, storers;
+        };
+        std::vector<Try> tries;
         for (char e : cand) {
-            tries.emplace_back(e, 0);
-            if (e == tsw_ctx::kEngSplit && ctx->batch_split_rows_opt == 0) tries.emplace_back(e, 64);
+            tries.push_back({e, 0, kSplitStorers});
+            if (e == tsw_ctx::kEngSplit && ctx->batch_split_rows_opt == 0) {
+                if (p == 1) tries.push_back({e, 64, kSplitStorers});
+                else if (ctx->batch_split_storers_opt == 0) tries.push_back({e, 0, 0});
+            }
         }
-        char best = cand[0];
-        int best_rows = 0;
+        Try best = tries[0];
         ctx->split_rows_p[p] = 0;
+        ctx->split_storers_p[p] = kSplitStorers;
         if (tries.size() > 1 && ctx->autotune) {
             // the heaviest members up to the scratch budget
             std::sort(mem.begin(), mem.end(),
@@ -4580,9 +4639,9 @@ void batch_choose_engines(tsw_ctx *ctx) {
             }
             double best_ms = 0.0;
             for (size_t t = 0; t < tries.size(); ++t) {
-                const char e = tries[t].first;
-                ctx->split_rows_p[p] = tries[t].second;
-                for (int b : sub_members) ctx->engine[b] = e;
+                ctx->split_rows_p[p] = tries[t].rows;
+                ctx->split_storers_p[p] = tries[t].storers;
+                for (int b : sub_members) ctx->engine[b] = tries[t].engine;
                 build_batch_groups(ctx, sub_members);
                 batch_apply(ctx, sub_members, dev, TSW_FP64);  // first touch of tables and buffers
                 hipEvent_t t0 = next_event(ctx), t1 = next_event(ctx);
@@ -4594,19 +4653,19 @@ void batch_choose_engines(tsw_ctx *ctx) {
                 TSW_HIP(hipEventElapsedTime(&ms, t0, t1));
                 if (t == 0 || ms < best_ms) {
                     best_ms = ms;
-                    best = e;
-                    best_rows = tries[t].second;
+                    best = tries[t];
                 }
             }
-            ctx->split_rows_p[p] = best_rows;
+            ctx->split_rows_p[p] = best.rows;
+            ctx->split_storers_p[p] = best.storers;
             sync(ctx);
             ctx->ev_used = 0;  // the tuning sweeps are not counted
             ctx->sweeps_done = 0;
             ctx->ms_folded = 0.0;
         }
         for (int b : mem) {
-            ctx->engine[b] = best;
-            if (best != tsw_ctx::kEngConverted) {  // diagonal-layout buffers of the tuning sweeps
+            ctx->engine[b] = best.engine;
+            if (best.engine != tsw_ctx::kEngConverted) {  // diagonal-layout buffers of the tuning sweeps
                 auto &d = ctx->batch[b]->diag;
                 d.q64.release();
                 d.q32.release();
@@ -4614,7 +4673,7 @@ void batch_choose_engines(tsw_ctx *ctx) {
                 d.ir64.release();
             }
         }
-        ctx->batch_engine[p] = best;
+        ctx->batch_engine[p] = best.engine;
     }
     ctx->groups.clear();
     ctx->lane_groups.clear();

@@ -16,38 +16,39 @@ TSW_SWEEP_EXTERN(float, 2)
 TSW_SWEEP_EXTERN(float, 3)
 TSW_SWEEP_EXTERN(float, 4)
 
-// LDS of the lane-split sweep for bands of BR rows(0: not built for (T, P) or
-// too many rows)
+// LDS of the lane-split sweep for bands of BR rows (0: not built for (T, P) or too many rows)
 template <typename T, int P>
-size_t split_lds_total(int BR, int M, bool ref) {
+size_t split_lds_total(int BR, int M, bool ref, int storers) {
     if constexpr (!split_supported<T, P>()) {
         return 0;
     } else {
         const int threads = (split_lanes<P>() * BR + 63) / 64 * 64, slots = threads / split_lanes<P>();
-        if (slots > (ref ? split_max_slots<P, true>() : split_max_slots<P, false>())) return 0;
-        return ref ? SplitLds<T, P, true>(slots, M).total : SplitLds<T, P, false>(slots, M).total;
+        if (slots > split_max_slots<P>(storers)) return 0;
+        return storers ? SplitLds<T, P, true, true>(slots, M).total
+               : ref   ? SplitLds<T, P, true, false>(slots, M).total
+                       : SplitLds<T, P, false, false>(slots, M).total;
     }
 }
 
 // (the kernel's static LDS, the taken item, comes on top)
 template <typename T>
-size_t split_lds_bytes(int p, int rows, int M, bool ref) {
+size_t split_lds_bytes(int p, int rows, int M, bool ref, int storers) {
     size_t total = 0;
     switch (p) {
-        case 1: total = split_lds_total<T, 2>(rows, M, ref); break;
-        case 2: total = split_lds_total<T, 3>(rows, M, ref); break;
-        case 3: total = split_lds_total<T, 4>(rows, M, ref); break;
+        case 1: total = split_lds_total<T, 2>(rows, M, ref, storers); break;
+        case 2: total = split_lds_total<T, 3>(rows, M, ref, storers); break;
+        case 3: total = split_lds_total<T, 4>(rows, M, ref, storers); break;
         default: break;
     }
     const size_t bytes = total * sizeof(T);
     return bytes + 16 <= max_lds_per_block() ? bytes : 0;
 }
 template <typename T>
-size_t split_sweep_lds_bytes(int p, int rows, int M) {
-    return split_lds_bytes<T>(p, rows, M, true);
+size_t split_sweep_lds_bytes(int p, int rows, int M, int storers) {
+    return split_lds_bytes<T>(p, rows, M, true, storers);
 }
-template size_t split_sweep_lds_bytes<double>(int, int, int);
-template size_t split_sweep_lds_bytes<float>(int, int, int);
+template size_t split_sweep_lds_bytes<double>(int, int, int, int);
+template size_t split_sweep_lds_bytes<float>(int, int, int, int);
 template <typename T>
 size_t wide_sweep_lds_bytes(int p, int rows, int M) {
     const int lanes = p == 1 ? wide_lanes<2>() : wide_lanes<3>(), slots = (lanes * rows + 63) / 64 * 64 / lanes;
@@ -70,7 +71,7 @@ size_t diag_sweep_lds_bytes(const DiagSweepParams<T> &sp, int p) {
     if (sp.wave1 && BR > 64) return 0;
     if (sp.split) {
         if (!sp.ainv || sp.wave1) return 0;
-        return sp.split == 2 ? wide_sweep_lds_bytes<T>(p, BR, sp.M) : split_lds_bytes<T>(p, BR, sp.M, false);
+        return sp.split == 2 ? wide_sweep_lds_bytes<T>(p, BR, sp.M) : split_lds_bytes<T>(p, BR, sp.M, false, 0);
     }
     const int cthreads = ((BR + 63) / 64) * 64;
     const int M = sp.ainv ? sp.M : 0;

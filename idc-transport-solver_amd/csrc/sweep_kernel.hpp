@@ -643,11 +643,14 @@ void launch_ds_d(const DiagSweepParams<T> &sp, size_t lds, hipStream_t s, const 
             // LG lanes for each row slot, in whole wavefronts, and the reference layout's storer waves
             const bool wide = sp.split == 2;
             const int threads = wide ? (wide_lanes<P>() * rows + 63) / 64 * 64 + 64 * kWideHelpers
-                                     : (split_lanes<P>() * rows + 63) / 64 * 64 + ((MODE & 4) != 0 ? 64 * kSplitStorers : 0);
+                                     : (split_lanes<P>() * rows + 63) / 64 * 64 + ((MODE & 4) != 0 ? 64 * sp.storers : 0);
             if (wide && (batch || threads > kWideThreads)) throw Error(TSW_E_ARG, "lane-per-coefficient sweep: inconsistent launch");
             if (!wide && threads > 512) throw Error(TSW_E_ARG, "lane-split sweep needs bands of at most 512 / lanes rows");
             if (batch) {
-                auto kern = k_diag_sweep_split<T, P, MODE, D, true, false>;
+                constexpr int ST = (MODE & 4) != 0 ? kSplitStorers : 0;
+                if (sp.storers != 0 && sp.storers != ST) throw Error(TSW_E_ARG, "lane-split sweep: no or two storer waves");
+                auto kern = ST > 0 && sp.storers > 0 ? k_diag_sweep_split<T, P, MODE, D, true, false, ST>
+                                                     : k_diag_sweep_split<T, P, MODE, D, true, false, 0>;
                 if (lds > 64 * 1024)
                     TSW_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
                 int grid = nitems;
@@ -661,7 +664,7 @@ void launch_ds_d(const DiagSweepParams<T> &sp, size_t lds, hipStream_t s, const 
                 hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, s, sp, batch, items, sp.work, sp.work_set);
             } else {
                 if constexpr ((MODE & 4) != 0) throw Error(TSW_E_ARG, "reference-layout lane-split sweep is built for batches");
-                auto kern = wide ? k_diag_sweep_split<T, P, MODE, D, false, true> : k_diag_sweep_split<T, P, MODE, D, false, false>;
+                auto kern = wide ? k_diag_sweep_split<T, P, MODE, D, false, true, 0> : k_diag_sweep_split<T, P, MODE, D, false, false, 0>;
                 if (lds > 64 * 1024)
                     TSW_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
                 hipLaunchKernelGGL(kern, dim3(sp.nq * (sp.nbands > 1 ? sp.nbands : 1)),
@@ -765,8 +768,9 @@ void launch_split_ref_p(const DiagSweepParams<T> &sp, const SplitSources &src, i
     if constexpr (split_supported<T, P>()) {
         const bool wide = sp.split == 2;
         const int threads = wide ? (wide_lanes<P>() * band_rows_of(sp) + 63) / 64 * 64 + 64 * kWideHelpers
-                                 : (split_lanes<P>() * band_rows_of(sp) + 63) / 64 * 64 + 64 * kSplitStorers;
-        if (threads > (wide ? kWideThreads : 512) || !sp.ainv || n < 1 || n > kSplitSources || (sp.nbands > 1 && (!sp.xtr || !sp.abort_flag)))
+                                 : (split_lanes<P>() * band_rows_of(sp) + 63) / 64 * 64 + 64 * sp.storers;
+        if (threads > (wide ? kWideThreads : 512) || !sp.ainv || n < 1 || n > kSplitSources || (sp.nbands > 1 && (!sp.xtr || !sp.abort_flag)) ||
+            (sp.storers != 0 && sp.storers != kSplitStorers))
             throw Error(TSW_E_ARG, "lane-split reference-layout sweep: inconsistent launch");
         const int items = n * sp.nq * (sp.nbands > 1 ? sp.nbands : 1);
         // the most items of a queue, over all queues
@@ -794,10 +798,10 @@ void launch_split_ref_p(const DiagSweepParams<T> &sp, const SplitSources &src, i
             TSW_HIP(hipGetLastError());
         };
         switch (sp.prefetch) {
-            case 2: wide ? go_wide(k_wide_ref<T, P, 2>) : go(k_split_ref<T, P, 2>); break;
-            case 3: wide ? go_wide(k_wide_ref<T, P, 3>) : go(k_split_ref<T, P, 3>); break;
-            case 4: wide ? go_wide(k_wide_ref<T, P, 4>) : go(k_split_ref<T, P, 4>); break;
-            case 6: wide ? go_wide(k_wide_ref<T, P, 6>) : go(k_split_ref<T, P, 6>); break;
+            case 2: wide ? go_wide(k_wide_ref<T, P, 2>) : sp.storers ? go(k_split_ref<T, P, 2, kSplitStorers>) : go(k_split_ref<T, P, 2, 0>); break;
+            case 3: wide ? go_wide(k_wide_ref<T, P, 3>) : sp.storers ? go(k_split_ref<T, P, 3, kSplitStorers>) : go(k_split_ref<T, P, 3, 0>); break;
+            case 4: wide ? go_wide(k_wide_ref<T, P, 4>) : sp.storers ? go(k_split_ref<T, P, 4, kSplitStorers>) : go(k_split_ref<T, P, 4, 0>); break;
+            case 6: wide ? go_wide(k_wide_ref<T, P, 6>) : sp.storers ? go(k_split_ref<T, P, 6, kSplitStorers>) : go(k_split_ref<T, P, 6, 0>); break;
             default: throw Error(TSW_E_ARG, "prefetch depth must be 2, 3, 4 or 6");
         }
     } else {

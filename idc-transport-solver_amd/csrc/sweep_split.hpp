@@ -16,7 +16,8 @@
 // MODE bit 4 (with bit 1, sources only): the source is read from `qref` and psi written to `psi_ref`, both in the
 // reference layout [i][j][q][d][e], and the inflow is read from the halo cells of qref, so no layout conversion and
 // no launch for the traces is needed.  Lane g's coefficients are one contiguous run of P doubles there, and the LG
-// lanes of a row cover the cell's run.  Two further waves (kSplitStorers) write the results.
+// lanes of a row cover the cell's run.  Two further waves (kSplitStorers) write the results, or, where more workgroups
+// on a CU or more rows in one pay more, the lanes themselves (which of the two: storers_forced and the rules after it).
 // BATCH: the workgroup's parameters are batch[items[b].x], and items[b].y = band * nq + ordinate, numbered band-major
 // so that a band's upstream band is always dispatched first; items with a negative problem index are padding.
 //
@@ -50,7 +51,8 @@ __host__ __device__ constexpr bool split_supported() {
     return P >= 2 && P <= 4 && P * P * P * (int)sizeof(T) <= 64 * 8;
 }
 
-template <typename T, int P, bool REF>
+// REF: reference layout; CELLS: with storer waves
+template <typename T, int P, bool REF, bool CELLS>
 struct SplitLds {  // LDS carve-up in units of T, 16-byte aligned arrays and rows
     static constexpr int N = P * P;
     static constexpr int PS = vround<T>(P), RS = vround<T>(P * N);
@@ -59,22 +61,21 @@ struct SplitLds {  // LDS carve-up in units of T, 16-byte aligned arrays and row
     static constexpr int XS = P * PS + (P * PS * (int)sizeof(T) % 128 == 0 ? Vec16<T>::W : 0);
     static constexpr int YR = 64 / split_lanes<P>();  // columns of the y-inflow ring: the rows of a wave
     size_t ex, xs, lin, inv, total;
-    // slots: row slots of the workgroup; M: materials ([M][P][RS] inverse rows, lane g's block at g).  The
-    // reference layout keeps the solved cells of two steps ([2][slots][XS]): the rows above take their
-    // y-traces, and the storer wave the results, from the last step's
+    // slots: row slots of the workgroup; M: materials ([M][P][RS] inverse rows, lane g's block at g).  With
+    // storer waves the solved cells of two steps are kept ([2][slots][XS]): the rows above take their
+    // y-traces, and the storers the results, from the last step's
     __host__ __device__ SplitLds(int slots, int M) {
         ex = 0;                                                 // [slots][2][PS] y-traces between rows, by step parity
-        xs = ex + (REF ? 0 : (size_t)2 * slots * PS);           // [slots][XS] solved cells, for the rows' x-traces
-        lin = xs + (size_t)(REF ? 2 : 1) * slots * XS;          // [YR][PS] y-inflow traces of row 0 (reference layout)
+        xs = ex + (CELLS ? 0 : (size_t)2 * slots * PS);         // [slots][XS] solved cells, for the rows' x-traces
+        lin = xs + (size_t)(CELLS ? 2 : 1) * slots * XS;        // [YR][PS] y-inflow traces of row 0 (reference layout)
         inv = lin + (REF ? (size_t)YR * PS : 0);                // [M][P][RS]
         total = inv + (size_t)M * P * RS;
     }
 };
-// Storer waves of a reference-layout workgroup, and the most row slots of a workgroup of 512 threads.
-constexpr int kSplitStorers = 2;
-template <int P, bool REF>
-__host__ __device__ constexpr int split_max_slots() {
-    return (512 - (REF ? 64 * kSplitStorers : 0)) / split_lanes<P>();
+// Most row slots of a workgroup of 512 threads with `storers` storer waves.
+template <int P>
+__host__ __device__ constexpr int split_max_slots(int storers) {
+    return (512 - 64 * storers) / split_lanes<P>();
 }
 
 // v read from lane K of its LG-lane group (quad permutation; K is a constant after unrolling)
@@ -153,15 +154,15 @@ __device__ __forceinline__ typename ExchangeSentinel<T>::U wait_value(gptr<const
 }
 
 // One item of the lane-split sweep: band wid / nq of ordinate wid % nq of the problem sp, by the whole
-// workgroup (every thread calls it; it ends with a workgroup barrier).
-template <typename T, int P, int MODE, int D>
+// workgroup (every thread calls it; it ends with a workgroup barrier).  ST: its storer waves (reference layout).
+template <typename T, int P, int MODE, int D, int ST>
 __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigned wid) {
     constexpr int N = P * P, LG = split_lanes<P>(), RPW = 64 / LG;  // rows per wavefront
-    constexpr bool HASQ = (MODE & 1) != 0, HASPHI = (MODE & 2) != 0, REF = (MODE & 4) != 0;
-    using Lds = SplitLds<T, P, REF>;
+    constexpr bool HASQ = (MODE & 1) != 0, HASPHI = (MODE & 2) != 0, REF = (MODE & 4) != 0, CELLS = ST > 0;
+    using Lds = SplitLds<T, P, REF, CELLS>;
     constexpr int PS = Lds::PS, RS = Lds::RS, XS = Lds::XS;
     using U = typename ExchangeSentinel<T>::U;
-    static_assert(!REF || MODE == 5, "reference-layout lane-split sweep: sources only");
+    static_assert(REF ? MODE == 5 : ST == 0, "reference-layout lane-split sweep: sources only; storers there alone");
     using PQ = typename std::conditional<REF, double, T>::type;  // prefetched source (converted at use)
     const int nb = sp.nbands < 2 ? 1 : sp.nbands;
     const int q = (int)(wid % (unsigned)sp.nq);
@@ -172,7 +173,7 @@ __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigne
     const int BR = nb > 1 ? sp.band_rows : ny;
     const int R0 = band * BR;
     const int nrows = BR < ny - R0 ? BR : ny - R0;
-    const int slots = ((int)blockDim.x - (REF ? 64 * kSplitStorers : 0)) / LG;
+    const int slots = ((int)blockDim.x - 64 * ST) / LG;
     const Lds L(slots, sp.M);
     T *linv = lds + L.inv;
     const DiagMap dm{nx, ny};
@@ -210,12 +211,12 @@ __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigne
     const unsigned nowhere = REF ? (unsigned)ref_bytes : (unsigned)nplanes;
     const __amdgpu_buffer_rsrc_t rout = REF ? buf_rsrc(sp.psi_ref, ref_bytes) : buf_rsrc(sp.psi + (size_t)q * N * ncell, nplanes);
 
-    if (REF && w0 >= slots) {
+    if constexpr (ST > 0) if (w0 >= slots) {
         // The storer waves: step t's cells during step t + 1, from LDS, as the band's runs one after the other
         // (access m of lane l, m dealt round the storers, is values (l + 64 m) SW of them).  A 64-byte segment of L2
         // takes a write request of its own, about one in 4 cycles per CU: written by the compute lanes, a cell's run
         // goes out in pieces, each segment in two requests or more, and the compute waves wait for the queue.
-        constexpr int SW = P % 2 == 0 ? 2 : 1, SM = (split_max_slots<P, true>() * N / SW + 64 * kSplitStorers - 1) / (64 * kSplitStorers);
+        constexpr int SW = P % 2 == 0 ? 2 : 1, SM = (split_max_slots<P>(ST) * N / SW + 64 * ST - 1) / (64 * ST);
         int lane = tid & 63;
         asm volatile("" : "+v"(lane));  // (keeps these tables out of the compute waves' registers)
         const int m0 = __builtin_amdgcn_readfirstlane((tid >> 6) - slots * LG / 64);
@@ -223,7 +224,7 @@ __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigne
         int c0[SM], at[SM];  // its column is t - c0 (far outside the mesh past the band's rows), its LDS offset
 #pragma unroll
         for (int m = 0; m < SM; ++m) {
-            const int e = (lane + 64 * (m * kSplitStorers + m0)) * SW, row = e / N, k = e - row * N;
+            const int e = (lane + 64 * (m * ST + m0)) * SW, row = e / N, k = e - row * N;
             const bool ok = row < nrows;
             c0[m] = ok ? row : (1 << 30);
             at[m] = ok ? row * XS + k / P * PS + k % P : 0;
@@ -240,7 +241,7 @@ __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigne
                 for (int k = 0; k < SW; ++k) v[m][k] = xt[at[m] + k];
 #pragma unroll
             for (int m = 0; m < SM; ++m) {
-                if (64 * (m * kSplitStorers + m0) * SW < nrows * N)  // wave-uniform
+                if (64 * (m * ST + m0) * SW < nrows * N)  // wave-uniform
                     ref_run_st<T, SW>(rout, (unsigned)(t - c0[m]) < (unsigned)nx ? soff[m] : nowhere, v[m]);
                 soff[m] += dstep;
             }
@@ -280,6 +281,7 @@ __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigne
     const unsigned vrow0 = (unsigned)r * (unsigned)sizeof(T), vrow = vrow0 + dplane;
     const unsigned vmat = (unsigned)r * 4u;
     unsigned foff = REF ? ref_off(0, r, nx, ny, sp.nq, q, N, xneg, yneg) + dref : 0;  // run of the next fetch
+    unsigned soff = foff;  // (no storers) run of the row's next result
     const int s_last = nx + ny - 2;
     DiagWalk fw{R0 + w0, (int)(dm.base(R0 + w0) - dm.rlo(R0 + w0))};  // diagonal of the next fetch
     DiagWalk cw{fw.s - 1, fw.s > 0 ? (int)(dm.base(fw.s - 1) - dm.rlo(fw.s - 1)) : 0};  // diagonal of the last step
@@ -343,11 +345,11 @@ __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigne
     }
     T sx = xneg ? T(-1) : T(1), sy = yneg ? T(-1) : T(1);
     asm volatile("" : "+v"(sx), "+v"(sy));
-    // LDS: the row below's y-trace (diagonal layout) or its cell's coefficients of this lane's x-degree
-    // (reference layout), and the row's own cell, of the last step; where this step's go
-    const int side = REF ? slots * XS : PS;  // between the two steps' copies
+    // LDS: the row below's y-trace or, with storer waves, its cell's coefficients of this lane's x-degree, and the
+    // row's own cell, of the last step; where this step's go
+    const int side = CELLS ? slots * XS : PS;  // between the two steps' copies
     const int sb = rl > 0 ? rl - 1 : 0;  // the row below
-    const T *exr = REF ? lds + L.xs + (size_t)sb * XS + dd * PS : lds + L.ex + (size_t)sb * 2 * PS + dd;
+    const T *exr = CELLS ? lds + L.xs + (size_t)sb * XS + dd * PS : lds + L.ex + (size_t)sb * 2 * PS + dd;
     T *exw = lds + L.ex + (size_t)rl * 2 * PS + dd;
     const T *xsr = lds + L.xs + (size_t)rl * XS + dd;
     T *xsw = lds + L.xs + (size_t)rl * XS + dd * PS;
@@ -363,9 +365,12 @@ __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigne
     for (int e = 0; e < P; ++e) xo[e] = T(0);
     bool act = false;  // the last step solved a cell in this lane's row
 
-    // results of the last step to memory (diagonal layout; cw stands at its diagonal)
+    // results of the last step to memory (diagonal layout: cw stands at its diagonal)
     auto store_last = [&]() {
-        if constexpr (!REF) {
+        if constexpr (REF && ST == 0) {
+            ref_run_st<T, P>(rout, act && owner ? soff : nowhere, xo);
+            soff += act ? dstep : 0u;
+        } else if constexpr (!REF) {
             const unsigned so = (unsigned)cw.off * (unsigned)sizeof(T), vo = act && owner ? vrow : nowhere;
 #pragma unroll
             for (int e = 0; e < P; ++e) buf_st<T>(rout, vo, so + e * plane, xo[e]);
@@ -387,10 +392,10 @@ __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigne
             // the traces the cell needs come through LDS; meanwhile the last step's cell goes out and the ring
             // slot it freed is refilled
             T yv[P], xv[P];
-            if constexpr (REF) lds_get<T, P>(exr + pr * side, yv);
+            if constexpr (CELLS) lds_get<T, P>(exr + pr * side, yv);
             else yv[0] = exr[pr * side];
 #pragma unroll
-            for (int d = 0; d < P; ++d) xv[d] = xsr[(REF ? pr * side : 0) + d * PS];
+            for (int d = 0; d < P; ++d) xv[d] = xsr[(CELLS ? pr * side : 0) + d * PS];
             __builtin_amdgcn_sched_barrier(0);
             store_last();
             fetch((u + D - 1) % D);
@@ -399,7 +404,7 @@ __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigne
 #pragma unroll
             for (int a = 1; a < P; ++a) v = (a & 1) ? v + sx * xv[a] : v + xv[a];
             tx = act ? v : tx;
-            T ty = REF ? y_trace(yv) : yv[0];
+            T ty = CELLS ? y_trace(yv) : yv[0];
             act = (unsigned)(t - ra) < (unsigned)nx;
             if (pm[u] != cur_mat && act) {
                 cur_mat = pm[u];
@@ -451,8 +456,8 @@ __device__ __forceinline__ void split_item(const DiagSweepParams<T> &sp, unsigne
                 for (int col = 1; col < N; ++col) acc = fmadd(Arow[e * N + col], B[col], acc);
                 xo[e] = acc;
             }
-            if constexpr (!REF) exw[(1 - pr) * side] = y_trace(xo);
-            lds_put<T, P>(xsw + (REF ? (1 - pr) * side : 0), xo);
+            if constexpr (!CELLS) exw[(1 - pr) * side] = y_trace(xo);
+            lds_put<T, P>(xsw + (CELLS ? (1 - pr) * side : 0), xo);
             if (lastrow && act) xstore(xout + (size_t)(t - ra) * P + dd, to_bits(y_trace(xo)));
             lds_barrier();
         }
@@ -510,13 +515,13 @@ __device__ __forceinline__ int2 take_item(int *work, Len len) {
 // One problem (sp1, workgroup = band x ordinate), a batch with one item per workgroup (items[b] = {problem,
 // band * nq + ordinate}, a negative problem marking padding), or a persistent batch launch (work != null,
 // counter set `set`): items ordered by queue, work[kWorkTable + x] the first item of XCD x's queue.
-template <typename T, int P, int MODE, int D, bool BATCH, bool WIDE>
+template <typename T, int P, int MODE, int D, bool BATCH, bool WIDE, int ST>
 __global__ __launch_bounds__(WIDE ? kWideThreads : 512) void k_diag_sweep_split(DiagSweepParams<T> sp1, const DiagSweepParams<T> *__restrict__ batch,
                                                           const int2 *__restrict__ items, int *__restrict__ work, int set) {
     if constexpr (!BATCH) {
         if (sp1.skip && *G(sp1.skip)) return;  // a replayed iteration after the loop has stopped
         if constexpr (WIDE) wide_item<T, P, MODE, D>(sp1, blockIdx.x);
-        else split_item<T, P, MODE, D>(sp1, blockIdx.x);
+        else split_item<T, P, MODE, D, ST>(sp1, blockIdx.x);
     } else {
         if (work && blockIdx.x == 0 && threadIdx.x < kXcds) work[(1 - set) * kWorkSet + threadIdx.x * kWorkStride] = 0;
         const gptr<const int> table = G(static_cast<const int *>(work)) + kWorkTable;
@@ -532,7 +537,7 @@ __global__ __launch_bounds__(WIDE ? kWideThreads : 512) void k_diag_sweep_split(
             if (item_p < 0) continue;  // padding of an XCD-ordered item list
             const DiagSweepParams<T> sp = batch[item_p];
             if (sp.skip && *G(sp.skip)) continue;
-            split_item<T, P, MODE, D>(sp, (unsigned)item_v);
+            split_item<T, P, MODE, D, ST>(sp, (unsigned)item_v);
         } while (work);
     }
 }
@@ -557,7 +562,7 @@ __device__ __forceinline__ unsigned ref_item(DiagSweepParams<T> &sp, const Split
 
 // One workgroup per item (work null: workgroup b takes item b / 8 of queue b % 8, the XCD that it is sent to), or a
 // persistent launch taking items.  The launch does nothing while *changed == mark.
-template <typename T, int P, int D>
+template <typename T, int P, int D, int ST>
 __global__ __launch_bounds__(512) void k_split_ref(DiagSweepParams<T> sp, SplitSources src, int n, int *__restrict__ work, int set,
                                                    const int *__restrict__ changed, int mark) {
     T *const xtr = sp.xtr;
@@ -568,7 +573,7 @@ __global__ __launch_bounds__(512) void k_split_ref(DiagSweepParams<T> sp, SplitS
     do {
         if (work) k = take_item(work + set * kWorkSet, [&](int x) { return I.count(x); });
         if (k.y < 0 || k.y >= I.count(k.x)) break;  // workgroup-uniform: every wave leaves
-        split_item<T, P, 5, D>(sp, ref_item<T, P>(sp, src, I, k.x, k.y, xtr));
+        split_item<T, P, 5, D, ST>(sp, ref_item<T, P>(sp, src, I, k.x, k.y, xtr));
     } while (work);
 }
 

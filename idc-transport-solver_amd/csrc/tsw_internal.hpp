@@ -144,6 +144,7 @@ template <typename T> struct DiagSweepParams {
     int *work;
     const int32_t *mat_cell;  // material index in the cell layout [nx+2][ny+2] (lane-per-coefficient sweep)
     int work_set;
+    int storers;           // lane-split on the reference layout: storer waves of a workgroup, 0 or kSplitStorers
 };
 
 // Ordinate-lane sweep on the reference layout (sweep_lanes.hpp).  An ordinate block is ordinates
@@ -179,6 +180,8 @@ constexpr int kXcds = 8;  // MI355X: workgroup b runs on XCD b mod 8, each XCD w
 // Device words of a lane-split launch's work counters (sweep_split.hpp), cleared when allocated: two sets, and
 // the kXcds + 1 queue bounds of a batch launch from word kSplitWorkTable on.
 constexpr int kSplitWorkTable = 2 * kXcds * 16, kSplitWorkInts = kSplitWorkTable + kXcds + 1;
+// Storer waves of a lane-split workgroup on the reference layout, where it has any.
+constexpr int kSplitStorers = 2;
 // Right-hand sides of one launch of the lane-split kernel on the reference layout.
 constexpr int kSplitSources = 32;
 struct SplitSources {
@@ -247,10 +250,10 @@ template <typename T>
 void launch_diag_sweep(const DiagSweepParams<T> &sp, int p, hipStream_t s);
 template <typename T>
 size_t diag_sweep_lds_bytes(const DiagSweepParams<T> &sp, int p);
-// LDS of a lane-split workgroup of `rows` rows with M materials on the reference layout (0: the kernel is not
-// built for (T, p) or does not fit)
+// LDS of a lane-split workgroup of `rows` rows and `storers` storer waves with M materials on the reference layout
+// (0: the kernel is not built for (T, p) or does not fit)
 template <typename T>
-size_t split_sweep_lds_bytes(int p, int rows, int M);
+size_t split_sweep_lds_bytes(int p, int rows, int M, int storers);
 // LDS bytes of the lane-per-coefficient sweep (either layout); 0 when it does not fit
 template <typename T>
 size_t wide_sweep_lds_bytes(int p, int rows, int M);

@@ -308,6 +308,31 @@ def test_split_batch_band_stall_is_reported_and_recovered():
                     assert rel_err(o, r) <= tol, (prec, P.name)
 
 
+@pytest.mark.parametrize("rows", [0, 32, 256])
+@pytest.mark.parametrize("precision", [tsw.FP64, tsw.FP32])
+def test_split_batch_with_and_without_storers(precision, rows):
+    """The lane-split engine with storer waves, without, and as the autotuner picks: the same bits as the conversions
+    (rows 256: bands of 256 rows at degree 1, 128 at degrees 2 and 3, which leave no room for storers unless forced)."""
+    batch = problems.batched(seed=11, count=9, n_range=(20, 140), degrees=(1, 2, 3), orders=(2, 4))
+    srcs = _random_halo_sources(batch, 5)
+    print("split batch storers", precision, rows, [(P.nx, P.p, P.nq) for P in batch], flush=True)
+    outs = {}
+    for storers in (None, 0, 1, -1):
+        with _split_ctx(rows) as ctx:
+            if storers is None:
+                ctx.set_tuning("batch_split", -1)
+            else:
+                ctx.set_tuning("batch_split_storers", storers)
+            ctx.batch_set([problems.as_batch_member(P) for P in batch], [P.sigma_t for P in batch])
+            for _ in range(2):
+                out = [s.copy() for s in srcs]
+                ctx.batch_sweep(out, precision=precision)
+            outs[storers] = out
+    for storers in (0, 1, -1):
+        for P, a, b in zip(batch, outs[None], outs[storers]):
+            np.testing.assert_array_equal(a, b, err_msg=f"{storers} {P.name}")
+
+
 def test_split_batch_tuning_keys():
     with tsw.Context(0) as ctx:
         for key, bad in (("batch_split", 2), ("batch_split_rows", 8), ("batch_split_rows", 300),

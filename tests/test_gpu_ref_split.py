@@ -127,6 +127,34 @@ def test_ref_split_edges_match_the_diagonal_path(shape, persistent):
         np.testing.assert_array_equal(a, c2)
 
 
+# the lane-split kernel itself (batch_split_rows set), with storer waves in bands of up to 192, 96 and 96 rows, and without
+# in bands of up to 256, 128 and 128
+@pytest.mark.parametrize("persistent", [1, 0])
+@pytest.mark.parametrize("storers", [1, -1])
+@pytest.mark.parametrize("shape", EDGES + [(3, 256, 1, 2), (2, 257, 1, 2), (5, 128, 2, 2), (3, 97, 2, 4), (6, 128, 3, 2)])
+def test_ref_split_with_and_without_storers(shape, storers, persistent):
+    nx, ny, p, order = shape
+    o = ls_ordinates(order)
+    g, st, _, src = random_problem(nx, ny, p, o, seed=60 + nx + ny, materials=2)
+    print("ref split storers", shape, storers, persistent, flush=True)
+    for prec, tol in ((tsw.FP64, 1e-12), (tsw.FP32, 2e-6)):
+        outs = []
+        with _ctx(g, o, 1) as c:
+            c.set_tuning("batch_split_rows", (192 if p == 1 else 96) if storers > 0 else (256 if p == 1 else 128))
+            c.set_tuning("batch_split_storers", storers)
+            c.set_tuning("batch_persistent", persistent)
+            for _ in range(2):
+                a = src.copy()
+                c.sweep(a, st, 0.7, precision=prec)
+                outs.append(a)
+        with _ctx(g, o, -1) as c:
+            b = src.copy()
+            c.sweep(b, st, 0.7, precision=prec)
+        assert rel_err(b, orc_sweep(g, o, st, src, 0.7)) <= tol, prec
+        np.testing.assert_array_equal(outs[0], b)
+        np.testing.assert_array_equal(outs[1], b)
+
+
 # the lane-per-coefficient kernel: rows of a wave (4; 16 at degree 1), of a workgroup (56, 224) and of a band (24, 64),
 # columns below, at and past the 16 that its feeder holds, against the lane-split kernel (batch_split_rows set)
 WIDE_EDGES = [(1, 1, 2, 2), (2, 3, 2, 4), (15, 4, 2, 2), (16, 5, 2, 6), (17, 56, 2, 4), (33, 57, 2, 4), (40, 121, 2, 8),
@@ -254,6 +282,9 @@ def test_ref_split_tuning_key():
     o = ls_ordinates(4)
     g, st, _, src = random_problem(5, 5, 1, o, seed=1)
     with _ctx(g, o) as c:
+        for bad in (-2, 2):
+            with pytest.raises(tsw.TswError):
+                c.set_tuning("batch_split_storers", bad)
         assert c.get_tuning("ref_split") == 1
         for bad in (0, 2):
             with pytest.raises(tsw.TswError):
