@@ -2479,18 +2479,42 @@ int split_band_rows(const tsw_ctx *ctx, int p, int ny, int storers) {
     return (ny + nb - 1) / nb;
 }
 
-// Rows per band of the lane-per-coefficient kernel on the reference layout, 0 where the lane-split kernel is the faster:
-// its waves hold a quarter of the rows, so it pays while the chip holds the sweep's `rows` (of all ordinates and sources)
-// at about the same time.  Kernel us, lane-split against this, S8 or S12: Q3 32 x 32 60 -> 28, 128 x 128 222 -> 104,
-// 140 x 140 197 -> 123, 256 x 256 453 -> 286, 280 x 280 (23,520 rows) 543 -> 497; Q2 32 x 32 38 -> 22, 128 x 128 142 ->
-// 91, 256 x 256 267 -> 186, 210 x 210 (17,640 rows) 283 -> 253, but 280 x 280 467 -> 477; Q1 32 x 32 26 -> 16,
-// 128 x 128 84 -> 74, 256 x 256 (10,240 rows) 187 -> 146, but 280 x 280 214 -> 220.  One band up to the most rows of a
-// workgroup; more rows than that in bands of 24 (64 at degree 1, where a row takes 4 lanes), of which a CU holds three:
-// within 3% of the best of 16 .. 56 at all these sizes.
-int wide_band_rows(const tsw_ctx *c, int p, int ny, long long rows) {
-    if (c->batch_split_rows_opt > 0 || rows > (p == 3 ? 1 << 20 : 20000)) return 0;
+// Rows per band of the lane-per-coefficient kernel on the reference layout: one band up to the most rows of a workgroup;
+// more rows than that in bands of 24 (64 at degree 1, where a row takes 4 lanes), of which a CU holds three: within 3% of
+// the best of 16 .. 56 rows on 128 x 128 to 280 x 280.
+int wide_band_rows(int p, int ny) {
     const int most = kWideRows(p), R = p == 1 ? 64 : 24, nb = ny <= most ? 1 : (ny + R - 1) / R;
     return (ny + nb - 1) / nb;
+}
+
+// Most rows (of all ordinates and sources of a launch) for which the lane-per-coefficient kernel, with bands of `rows` rows
+// and lds bytes a workgroup, is the faster on the reference layout; the lane-split kernel has bands of split_rows rows.  Its
+// waves hold a quarter of the rows, so it pays while the chip holds the sweep at about the same time, and where the columns
+// are so few that a band's start is much of its steps.  Calls of one source or n, S8 unless given, 64 materials, FP64 unless
+// given, lane-split against this, us:
+//   one source: Q3 128 x 128 277 -> 159; Q2 192 -> 146 (n = 2), 210 x 210 S12 (17,640 rows) 356 -> 292, but 280 x 280 S12
+//     516 -> 525 (2 materials); Q1 256 x 256 S12 (21,504 rows) 241 -> 229, but 300 x 150 S16 (21,600 rows) 215 -> 244.
+//   many sources: Q1 64 x 64 n = 32 (81,920 rows) 197 -> 172, but 100 x 100 S12 n = 12 (100,800 rows) 351 -> 381, 128 x 64 n =
+//     24 306 -> 334; Q2 64 x 64 S16 n = 32 (294,912 rows) 1310 -> 1108, 100 x 100 S12 n = 20 1200 -> 1163, but 32 x 32 S16
+//     n = 16 (73,728 rows) 209 -> 236; FP32 Q2 16 x 100 n = 32 372 -> 222, but 64 x 64 n = 9 (23,040 rows) 131 -> 145.
+//   Q3: a CU holds one workgroup of either with 64 materials, but three of this one with few, so that the line goes with the
+//     rows that a CU holds: 128 x 128 n = 5 (25,600 rows) 390 -> 370, but n = 6 392 -> 427; 2 materials 350 x 350 S16 (50,400
+//     rows) 1229 -> 1185, but 440 x 440 (63,360 rows) 1740 -> 1810; FP32 n = 4 (20,480 rows) 317 -> 313, but n = 5 333 ->
+//     369; 2 materials n = 5 298 -> 297, but n = 6 323 -> 347.  Few columns: 48 x 48 S12 n = 32 1084 -> 590, 100 x 100 S12 n =
+//     12, 2 materials 742 -> 632, but 64 materials, without storers, 819 -> 1047; FP32 in one band 56 x 56 S12 n = 20 494 ->
+//     446, in more 64 x 64 S12 n = 20 670 -> 797.
+template <typename T>
+double wide_most_rows(const Geom &g, int rows, size_t lds, int split_rows, int storers) {
+    constexpr double any = 1e300;
+    constexpr bool f64 = sizeof(T) == 8;
+    if (g.p == 1) return g.nx <= 100 ? 82000 : 20000;
+    if (g.p == 2) {
+        if (f64) return g.nx > 100 ? 20000 : g.ny <= 32 ? 41000 : any;
+        return g.nx <= 40 && g.ny > 32 ? any : 20000;
+    }
+    const double held = std::min<double>(3, (160 * 1024) / lds) * rows / split_rows;  // a CU's rows, against the lane-split's
+    if (f64 ? g.nx <= 100 && (storers || held >= 0.5) : rows >= g.ny) return any;
+    return f64 ? std::max(27000.0, 60000 * held) : std::max(21000.0, 30000 * held);
 }
 
 // Prefetch depth of the lane-split kernel on the reference layout: 3 for FP64 Q3, whose ring of 4 spills (256 x 256, S8,
@@ -2534,8 +2558,9 @@ bool split_ref_plan(tsw_ctx *c, const double *sig, double dt, bool known, int n,
     lds = split_sweep_lds_bytes<T>(g.p, br, base.M, base.storers);
     if (lds == 0) return false;
     base.split = 1;
-    const int wr = wide_band_rows(c, g.p, g.ny, (long long)n * g.nq * g.ny);
-    if (const size_t l = wr > 0 ? wide_sweep_lds_bytes<T>(g.p, wr, base.M) : 0; l > 0) {
+    const int wr = wide_band_rows(g.p, g.ny);
+    const size_t l = c->batch_split_rows_opt == 0 ? wide_sweep_lds_bytes<T>(g.p, wr, base.M) : 0;
+    if (l > 0 && (double)std::min(n, kSplitSources) * g.nq * g.ny <= wide_most_rows<T>(g, wr, l, br, base.storers)) {
         br = wr;
         lds = l;
         base.split = 2;

@@ -225,6 +225,30 @@ def test_ref_split_persistent_switched_on_and_off(p, rows):
             np.testing.assert_array_equal(a, first)
 
 
+# more rows of all sources than a lane per coefficient pays for (past 100 columns: 20,000 at degrees 1 and 2, 27,000 at 3,
+# where 13 sources of 112 rows in one band go without storers), and fewer columns, where the line is another
+@pytest.mark.parametrize("prec", [tsw.FP64, tsw.FP32])
+@pytest.mark.parametrize("shape", [(101, 60, 1, 8, 9), (101, 60, 2, 8, 9), (101, 112, 3, 8, 7), (101, 112, 3, 8, 13),
+                                   (30, 100, 1, 8, 21), (20, 32, 2, 8, 33), (50, 40, 2, 8, 13), (40, 60, 3, 8, 13)])
+def test_ref_sweeps_of_many_sources_equal_single_sweeps(shape, prec):
+    import torch
+    nx, ny, p, order, n = shape
+    o = ls_ordinates(order)
+    g, st, _, src = random_problem(nx, ny, p, o, seed=20 + nx + ny + p, materials=2)
+    print("ref many sources", shape, prec, flush=True)
+    dev = torch.device("cuda:0")
+    with _ctx(g, o) as c:
+        st_d = torch.from_numpy(st).to(dev)
+        one = [torch.from_numpy(src * (1 + k)).to(dev) for k in range(2)]
+        many = [one[k % 2].clone() for k in range(n)]
+        for a in one:
+            c.sweep(a, st_d, 0.5, precision=prec)
+        c.sweep_multi(many, st_d, 0.5, precision=prec)
+        for k, a in enumerate(many):
+            assert torch.equal(a, one[k % 2]), k
+    assert rel_err(one[0].cpu().numpy(), orc_sweep(g, o, st, src, 0.5)) <= (1e-12 if prec == tsw.FP64 else 2e-6)
+
+
 def test_ref_split_more_sources_than_one_launch_takes():
     import torch
     o = ls_ordinates(4)
