@@ -214,6 +214,7 @@ struct tsw_ctx {
     } lanes;
     int last_lanes = 0, last_lanes_J = 0, last_lanes_W = 0;
     int split_opt = 0;     // 1: 2 or 4 lanes per row on the material path (tuning key lane_split)
+    int wide_opt = 0;      // 1: a lane per coefficient there (tuning key lane_coefficient)
     // batch launch groups: -1 storer wave unless a table only fits without it, else (0, 1) direct stores
     // whenever every member has element-inverse tables (tuning key batch_direct)
     int batch_direct_opt = 0;
@@ -1171,7 +1172,9 @@ const T *diag_inverses(tsw_ctx *c, double dt) {
 // one wavefront of rows per band when the mesh has more rows than that, so the ordinates' sweeps
 // spread over several times more compute units than there are ordinates.
 bool one_wave_for(const tsw_ctx *c) { return (c->tuned_w1 != INT_MIN ? c->tuned_w1 : c->one_wave_opt) == 1; }
-int lane_split_for(const tsw_ctx *c) { return std::max(0, c->tuned_sl != INT_MIN ? c->tuned_sl : c->split_opt); }
+int lane_split_for(const tsw_ctx *c) {
+    return std::max(0, c->tuned_sl != INT_MIN ? c->tuned_sl : c->wide_opt ? 2 : c->split_opt);
+}
 
 int band_rows_for(const tsw_ctx *c) {
     const int ny = c->g.ny;
@@ -1262,7 +1265,7 @@ DiagSweepParams<T> make_diag_params(tsw_ctx *c, double dt, const T *qsrc, const 
     }
     if (!sp.ainv) sp.sig_t = (const T *)(f64 ? d.sigt64.ptr : d.sigt32.ptr);
     c->last_w1 = sp.wave1;
-    c->last_sl = sp.split != 0;
+    c->last_sl = sp.split;
     sp.psi = psi_out;
     return sp;
 }
@@ -1279,7 +1282,8 @@ int kWideRows(int p) { return 896 / (p == 1 ? 4 : 16); }
 template <typename T>
 void select_tuning(tsw_ctx *c, double dt, const T *qsrc, const T *phi_d, bool inflow) {
     c->tuned_br = c->tuned_pf = c->tuned_w1 = c->tuned_sl = INT_MIN;
-    if (!c->autotune || c->band_rows_opt != 0 || c->prefetch_opt != 0 || c->one_wave_opt != 0 || c->split_opt != 0)
+    if (!c->autotune || c->band_rows_opt != 0 || c->prefetch_opt != 0 || c->one_wave_opt != 0 || c->split_opt != 0 ||
+        c->wide_opt != 0)
         return;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     TSW_HIP(hipStreamIsCapturing(c->stream, &cap));
@@ -2553,8 +2557,9 @@ bool split_ref_plan(tsw_ctx *c, const double *sig, double dt, bool known, int n,
     const Geom &g = c->g;
     if (c->ref_split_opt < 0 || g.p < 1) return false;
     if (c->g.npsi() * sizeof(double) > kSplitRefBytes) return false;
-    // a set band_rows, prefetch, one_wave or lane_split asks for the diagonal-layout kernels
-    if (c->band_rows_opt != 0 || c->prefetch_opt != 0 || c->one_wave_opt != 0 || c->split_opt != 0) return false;
+    // a set band_rows, prefetch, one_wave, lane_split or lane_coefficient asks for the diagonal-layout kernels
+    if (c->band_rows_opt != 0 || c->prefetch_opt != 0 || c->one_wave_opt != 0 || c->split_opt != 0 || c->wide_opt != 0)
+        return false;
     if (!known) {
         prepare_materials(c, sig, dt);
     } else if (c->mat.inv_dt != inverse_dt(dt)) {
@@ -2660,7 +2665,7 @@ bool try_split_ref(tsw_ctx *c, const std::vector<double *> &arr, const double *s
         split_ref_sweep<T>(c, base, lds, arr, changed, mark);
         TSW_HIP(hipStreamSynchronize(c->stream));
         if (static_cast<volatile int &>(c->host_flags[1]) != mark) {
-            c->last_sl = 1;
+            c->last_sl = base.split;
             return true;
         }
         c->sweeps_done -= (long long)arr.size();  // the sweep that did nothing
@@ -2670,7 +2675,7 @@ bool try_split_ref(tsw_ctx *c, const std::vector<double *> &arr, const double *s
     }
     if (!split_ref_plan<T>(c, sig, dt, false, (int)arr.size(), base, lds)) return false;
     split_ref_sweep<T>(c, base, lds, arr, nullptr, 0);
-    c->last_sl = 1;
+    c->last_sl = base.split;
     return true;
 }
 
@@ -2980,6 +2985,7 @@ tsw_ctx *adjoint_ctx(tsw_ctx *ctx) {
     ctx->adj->gmres_refine = ctx->gmres_refine;
     ctx->adj->one_wave_opt = ctx->one_wave_opt;
     ctx->adj->split_opt = ctx->split_opt;
+    ctx->adj->wide_opt = ctx->wide_opt;
     ctx->adj->refine_steps = ctx->refine_steps;
     return ctx->adj.get();
 }
@@ -3268,6 +3274,9 @@ int tsw_set_tuning(tsw_ctx *ctx, const char *key, int value) {
         } else if (k == "lane_split") {
             require(value == 0 || value == 1, TSW_E_ARG, "lane_split must be 0 or 1");
             ctx->split_opt = value;
+        } else if (k == "lane_coefficient") {
+            require(value == 0 || value == 1, TSW_E_ARG, "lane_coefficient must be 0 or 1");
+            ctx->wide_opt = value;
         } else if (k == "batch_direct") {
             require(value >= -1 && value <= 1, TSW_E_ARG, "batch_direct must be -1, 0 or 1");
             ctx->batch_direct_opt = value;
@@ -3352,7 +3361,8 @@ int tsw_get_tuning(tsw_ctx *ctx, const char *key, int *value) {
         else if (k == "gmres_refine") *value = ctx->gmres_refine ? 1 : 0;
         else if (k == "fp32_safety") *value = (int)ctx->fp32_safety;
         else if (k == "one_wave") *value = ctx->last_w1;
-        else if (k == "lane_split") *value = ctx->last_sl;
+        else if (k == "lane_split") *value = ctx->last_sl != 0;
+        else if (k == "lane_coefficient") *value = ctx->last_sl == 2;
         else if (k == "batch_direct") *value = ctx->batch_direct_opt;
         else if (k == "batch_ref") *value = ctx->last_batch_ref ? 1 : 0;
         else if (k == "ref_stage") *value = ctx->ref_stage_opt;

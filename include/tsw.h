@@ -101,10 +101,11 @@ int tsw_set_xs_degree(tsw_ctx *ctx, int degree);
  * (0 default, 1): bands of at most 64 rows, each swept by a single wavefront that passes the y-traces
  * lane to lane instead of through LDS.  Key "lane_split" (0 default, 1): on the material-table path,
  * 2 (DG degree 1) or 4 (degrees 2, 3) lanes per row, each solving its share of the cell's coefficients
- * (degrees 1-3; degree 0 runs the one-lane kernel).  Key "batch_direct" (0 default or 1, -1): launch groups of
+ * (degrees 1-3; degree 0 runs the one-lane kernel); key "lane_coefficient" (0 default, 1): there, a lane per
+ * coefficient, where a band fits a workgroup (224 rows at degree 1, 56 at 2 and 3).  Key "batch_direct" (0 default or 1, -1): launch groups of
  * tsw_batch_sweep store from the compute lanes instead of a storer wave (smaller workgroups, more of
  * them per CU), or keep the storer wave where the tables fit with it.  Key "autotune" (1 default, 0
- * off): while band_rows, prefetch, one_wave and lane_split are all 0, the first sweep of each kind
+ * off): while band_rows, prefetch, one_wave, lane_split and lane_coefficient are all 0, the first sweep of each kind
  * (mesh, degree, ordinates, precision, source terms, material path) times every candidate (kernel, band
  * rows, prefetch) into scratch memory and keeps the fastest for later sweeps; inside a HIP graph capture
  * the defaults apply.  Key "lanes" (0 default, 1, -1): the ordinate-lane engine (J ordinates of a quadrant
@@ -151,8 +152,8 @@ int tsw_set_tuning(tsw_ctx *ctx, const char *key, int value);
 
 /* Reads back "band_rows" (rows per band of the last staggered sweep, 0 = one band per ordinate),
  * "prefetch" (its prefetch depth), "one_wave" (1 if it ran the one-wavefront kernel), "lane_split" (1 if
- * it ran the lane-split or lane-per-coefficient kernel), "lanes" (1 if the last sweep, or for a batch context any member, ran on
- * the ordinate-lane engine), "lanes_block" / "lanes_waves" (its shape), "batch_ref" (1 if the last
+ * it ran the lane-split or lane-per-coefficient kernel), "lane_coefficient" (1 if it ran the latter), "lanes" (1 if
+ * the last sweep, or for a batch context any member, ran on the ordinate-lane engine), "lanes_block" / "lanes_waves" (its shape), "batch_ref" (1 if the last
  * tsw_batch_sweep ran staggered or lane-split groups on the caller's layout), "batch_engine_p0" ..
  * "batch_engine_p3" (the engine tsw_batch_set chose for that DG degree: 0 staggered through conversions,
  * 1 staggered on the caller's layout, 2 ordinate lanes, 3 lane-split on the caller's layout, -1 none in

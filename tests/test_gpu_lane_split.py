@@ -111,3 +111,69 @@ def test_lane_split_tuning_key():
     with _ctx(g, o, 0, 0) as c:
         with pytest.raises(tsw.TswError):
             c.set_tuning("lane_split", 2)
+
+
+def _wide_ctx(g, o, band_rows, prefetch=0):
+    c = _ctx(g, o, band_rows, 0, prefetch)
+    c.set_tuning("lane_coefficient", 1)
+    return c
+
+
+# rows of a wave (4; 16 at degree 1) and of a workgroup (56; 224), bands of a few rows and ragged last ones, columns below,
+# at and past the 16 that the feeder holds
+@pytest.mark.parametrize("shape,band_rows", [((37, 150), 24), ((16, 33), 16), ((20, 56), -1), ((17, 57), 56), ((12, 64), 5),
+                                             ((1, 9), -1), ((70, 3), -1), ((15, 225), 32)])
+@pytest.mark.parametrize("p", [1, 2, 3])
+def test_lane_coefficient_sweep_matches_oracle_and_one_lane_kernel(shape, band_rows, p):
+    o = ls_ordinates(6)
+    g, st, _, src = random_problem(shape[0], shape[1], p, o, seed=1700 + p + shape[1], ax=0.0, bx=2.0, by=3.0, materials=5)
+    print(f"lane per coefficient {shape} bands {band_rows} p={p}", flush=True)
+    for dt in (math.inf, 0.3):
+        ref = orc_sweep(g, o, st, src, dt)
+        for prec, tol in ((tsw.FP64, 1e-12), (tsw.FP32, 2e-6)):
+            with _ctx(g, o, 0, 0, 2) as c:
+                one = src.copy()
+                c.sweep(one, st, dt, precision=prec)
+                assert (c.get_tuning("lane_split"), c.get_tuning("lane_coefficient")) == (0, 0)
+            assert rel_err(one, ref) <= tol, (dt, prec)
+            with _wide_ctx(g, o, band_rows) as c:
+                for _ in range(2):  # the second sweep reuses the emptied exchange records
+                    out = src.copy()
+                    c.sweep(out, st, dt, precision=prec)
+                    assert (c.get_tuning("lane_split"), c.get_tuning("lane_coefficient")) == (1, 1), prec
+                    np.testing.assert_array_equal(out, one)
+
+
+@pytest.mark.parametrize("p", [1, 2, 3])
+@pytest.mark.parametrize("band_rows", [-1, 24])
+@pytest.mark.parametrize("prefetch", [2, 3, 4, 6])
+def test_lane_coefficient_solves_equal_one_lane_kernel(p, band_rows, prefetch):
+    """GMRES and source iteration: sweeps of the source, of the scattering source and of both."""
+    o = ls_ordinates(4)
+    g, st, ss, src = random_problem(30, 50, p, o, seed=1800 + p, materials=4)
+    for prec in (tsw.FP64, tsw.FP32):
+        outs = []
+        for wide in (0, 1):
+            with (_wide_ctx(g, o, band_rows, prefetch) if wide else _ctx(g, o, 0, 0, prefetch)) as c:
+                c.set_tuning("si_graph", 0)
+                a, b = src.copy(), src.copy()
+                c.gmres_solve(a, st, ss, abs_tol=1e-12 if prec == tsw.FP64 else 1e-9, precision=prec)
+                assert c.get_tuning("lane_coefficient") == wide
+                c.si_solve(b, st, ss, abs_tol=1e-9 if prec == tsw.FP64 else 1e-5, max_its=300, precision=prec)
+                assert c.get_tuning("lane_coefficient") == wide
+                outs.append((a, b))
+        np.testing.assert_array_equal(outs[0][0], outs[1][0])
+        np.testing.assert_array_equal(outs[0][1], outs[1][1])
+
+
+def test_lane_coefficient_tuning_key_and_fallback():
+    o = ls_ordinates(2)
+    g, st, _, src = random_problem(6, 70, 2, o, seed=4, materials=2)
+    with _wide_ctx(g, o, -1) as c:
+        for bad in (-1, 2):
+            with pytest.raises(tsw.TswError):
+                c.set_tuning("lane_coefficient", bad)
+        out = src.copy()
+        c.sweep(out, st, 0.4)  # 70 rows in one band are more than a workgroup holds: the one-lane kernel
+        assert (c.get_tuning("lane_split"), c.get_tuning("lane_coefficient")) == (0, 0)
+        assert rel_err(out, orc_sweep(g, o, st, src, 0.4)) <= 1e-12

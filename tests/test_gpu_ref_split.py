@@ -147,6 +147,7 @@ def test_ref_split_with_and_without_storers(shape, storers, persistent):
                 a = src.copy()
                 c.sweep(a, st, 0.7, precision=prec)
                 outs.append(a)
+            assert (c.get_tuning("lane_split"), c.get_tuning("lane_coefficient")) == (1, 0)
         with _ctx(g, o, -1) as c:
             b = src.copy()
             c.sweep(b, st, 0.7, precision=prec)
@@ -225,12 +226,15 @@ def test_ref_split_persistent_switched_on_and_off(p, rows):
             np.testing.assert_array_equal(a, first)
 
 
-# more rows of all sources than a lane per coefficient pays for (past 100 columns: 20,000 at degrees 1 and 2, 27,000 at 3,
-# where 13 sources of 112 rows in one band go without storers), and fewer columns, where the line is another
+# sources of one launch by their rows (of all ordinates): which kernel takes them in FP64 and in FP32 (1: a lane per
+# coefficient).  Past 100 columns it gives way at 20,000 rows at degrees 1 and 2 and, with few materials, between 30,000
+# and 60,000 at degree 3, where 13 sources of 112 rows in one band go without storers; the line is another on few columns
 @pytest.mark.parametrize("prec", [tsw.FP64, tsw.FP32])
-@pytest.mark.parametrize("shape", [(101, 60, 1, 8, 9), (101, 60, 2, 8, 9), (101, 112, 3, 8, 7), (101, 112, 3, 8, 13),
-                                   (30, 100, 1, 8, 21), (20, 32, 2, 8, 33), (50, 40, 2, 8, 13), (40, 60, 3, 8, 13)])
-def test_ref_sweeps_of_many_sources_equal_single_sweeps(shape, prec):
+@pytest.mark.parametrize("shape,kernel", [((101, 60, 1, 8, 9), (0, 0)), ((101, 60, 2, 8, 9), (0, 0)), ((101, 60, 2, 8, 8), (1, 1)),
+                                          ((101, 112, 3, 8, 7), (1, 1)), ((101, 112, 3, 8, 13), (0, 0)),
+                                          ((30, 100, 1, 8, 21), (0, 0)), ((20, 32, 2, 8, 33), (1, 0)),
+                                          ((50, 40, 2, 8, 13), (1, 0)), ((40, 60, 3, 8, 13), (1, 0))])
+def test_ref_sweeps_of_many_sources_equal_single_sweeps(shape, kernel, prec):
     import torch
     nx, ny, p, order, n = shape
     o = ls_ordinates(order)
@@ -243,7 +247,10 @@ def test_ref_sweeps_of_many_sources_equal_single_sweeps(shape, prec):
         many = [one[k % 2].clone() for k in range(n)]
         for a in one:
             c.sweep(a, st_d, 0.5, precision=prec)
+        assert c.get_tuning("lane_coefficient") == 1
         c.sweep_multi(many, st_d, 0.5, precision=prec)
+        assert c.get_tuning("lane_split") == 1
+        assert c.get_tuning("lane_coefficient") == kernel[0 if prec == tsw.FP64 else 1]
         for k, a in enumerate(many):
             assert torch.equal(a, one[k % 2]), k
     assert rel_err(one[0].cpu().numpy(), orc_sweep(g, o, st, src, 0.5)) <= (1e-12 if prec == tsw.FP64 else 2e-6)
