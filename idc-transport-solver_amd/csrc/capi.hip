@@ -222,7 +222,6 @@ struct tsw_ctx {
     // batch engines: 1 / -1 force / forbid the lane-split groups (tuning key batch_split); their rows per
     // band (batch_split_rows, 0: the most one workgroup holds) and prefetch depth (batch_split_prefetch)
     int batch_split_opt = 0, batch_split_rows_opt = 0, batch_split_pf_opt = 0, batch_split_storers_opt = 0;
-    int split_storers_p[4] = {kSplitStorers, kSplitStorers, kSplitStorers, kSplitStorers};  // storer waves of its FP64 groups
     int split_rows_p[4] = {0, 0, 0, 0};  // rows per band of the lane-split engine per DG degree (autotuned; 0: most)
     // lane-split groups: runs of this many consecutive items go to one XCD (tuning key batch_xcd_tile;
     // 0 or 1: dispatch order)
@@ -2450,20 +2449,26 @@ int split_lanes_of(int p) { return p == 1 ? 2 : 4; }
 // four SIMDs, so that six (64 rows at degrees 2 and 3) leave no room for a second workgroup on a CU where a SIMD holds
 // three (FP64 Q2, FP32 Q3: 161 to 178 VGPRs) and a third of the rows are in flight.
 //
-// A batch's group (64 materials, us, with and without): degree 1 with, 64 x 48^2 S12 261 and 318, 24 x 200^2 S8 1221 and
-// 1317.  FP32 degree 2 with: 467 and 522, 1921 and 2419.  FP32 degree 3 without: 32 x 48^2 S12 941 and 730, 32 x 100^2 S12
-// 2423 and 1943, 24 x 200^2 S8 2478 and 2462.  FP64 degrees 2 and 3 as the batch's autotuner finds: Q2 32 x 48^2 694 and
-// 545, but 24 x 200^2 2220 and 2396; Q3 48^2 1196 and 1310, but, by bands of up to 128 rows in place of 96, 100^2 2954 and
-// 2196 (CUs with one workgroup for their LDS, which then has seven compute waves, not four).
+// Members of a batch (64 materials, us, with and without): degree 1 with, 64 x 48^2 S12 261 and 318, 24 x 200^2 S8 1221 and
+// 1317.  Degree 2 in FP32 with: 32 x 48^2 S12 467 and 522, 24 x 200^2 1921 and 2419; in FP64 without up to 100 rows: 694 and
+// 545, 64 x 64^2 S8 839 and 800, 32 x 100^2 S12 1894 and 1804, but 32 x 128^2 S8 1299 and 1324, 24 x 200^2 2220 and 2396.
+// Degree 3 without where a member is then one band of 97 to 128 rows, as a CU has one workgroup for their LDS, which then
+// has seven or eight compute waves in place of four: FP64 32 x 100^2 2954 and 2196, 32 x 128^2 1855 and 1563, but 64 x 64^2
+// 1377 and 1418; and in FP32 below that: 32 x 48^2 941 and 730, 64 x 64^2 1077 and 919; and in bands of 64 rows, of which a
+// CU holds two where there are few materials.  Two bands in place of three, 24 x 200^2, 2815 and 2541, but with arrays that
+// do not start on a cache line, where whole runs cost less, the 85 Q3 members of 32^2 to 256^2 8.3 and 9.2 ms.
 // (a row count that leaves no room for them means none)
 int storers_forced(const tsw_ctx *c, int p) {
     if (c->batch_split_storers_opt != 0) return c->batch_split_storers_opt > 0 ? kSplitStorers : 0;
     return c->batch_split_rows_opt > (512 - 64 * kSplitStorers) / split_lanes_of(p) ? 0 : -1;
 }
+bool one_band(int ny) { return ny > 96 && ny <= 128; }  // without storers at degree 3, two with them
 template <typename T>
-int batch_storers(const tsw_ctx *c, int p) {
-    const int forced = storers_forced(c, p);
-    return forced >= 0 ? forced : sizeof(T) == 8 ? c->split_storers_p[p] : p == 3 ? 0 : kSplitStorers;
+int batch_storers(const tsw_ctx *c, const Geom &g) {
+    const int forced = storers_forced(c, g.p);
+    if (forced >= 0) return forced;
+    if (g.p == 2) return sizeof(T) == 8 && g.ny <= 100 ? 0 : kSplitStorers;
+    return g.p == 3 && (c->split_rows_p[3] == 64 || one_band(g.ny) || (sizeof(T) == 4 && g.ny <= 96)) ? 0 : kSplitStorers;
 }
 // n sources of one problem (64 materials, us, with and without): single sweeps gain from them, 280 x 280 S12 Q2 497 and 585,
 // Q3 579 and 663, FP32 553 and 677.  FP32 Q3 without on short rows of cells: 64 x 64 S12, 32 sources 1058 and 822, 100 x 100
@@ -2477,7 +2482,7 @@ int ref_storers(const tsw_ctx *c, int n) {
     if (forced >= 0) return forced;
     if (g.p < 3) return kSplitStorers;
     if (sizeof(T) == 4) return n > 1 && g.nx <= 100 ? 0 : kSplitStorers;
-    return g.ny <= 256 && (g.ny + 127) / 128 < (g.ny + 95) / 96 && n * g.nq >= 512 ? 0 : kSplitStorers;
+    return one_band(g.ny) && n * g.nq >= 512 ? 0 : kSplitStorers;
 }
 
 // Rows per band of a problem (a batch member, or a single problem) on the lane-split kernel: the fewest
@@ -4002,7 +4007,6 @@ int tsw_batch_set(tsw_ctx *ctx, int nprob, const tsw_problem *probs, const doubl
         ctx->lanes_able.assign(nprob, 0);
         ctx->split_able.assign(nprob, 0);
         for (int &r : ctx->split_rows_p) r = 0;
-        for (int &n : ctx->split_storers_p) n = kSplitStorers;
         ctx->batch_all.resize(nprob);
         for (int b = 0; b < nprob; ++b) ctx->batch_all[b] = b;
         ctx->batch_dt = dt;
@@ -4288,7 +4292,7 @@ void split_queues(tsw_ctx *ctx, tsw_ctx::Group &G, const std::vector<std::tuple<
 void build_batch_groups(tsw_ctx *ctx, const std::vector<int> &members) {
     ctx->groups.clear();
     ctx->lane_groups.clear();
-    std::map<std::tuple<int, int, bool, int>, int> gid;
+    std::map<std::tuple<int, int, bool, int, int>, int> gid;
     std::map<int, int> lid;
     for (int b : members) {
         tsw_ctx *sub = ctx->batch[b].get();
@@ -4305,11 +4309,12 @@ void build_batch_groups(tsw_ctx *ctx, const std::vector<int> &members) {
         }
         const int e = ctx->engine[b];
         const bool split = e == tsw_ctx::kEngSplit;
-        // staggered groups hold members of equal waves per workgroup, split groups of equal row slots
+        // staggered groups hold members of equal waves per workgroup, split groups of equal row slots and storers
         const int rpw = split ? 64 / split_lanes_of(sub->g.p) : 64;
-        const int st64 = split ? batch_storers<double>(ctx, sub->g.p) : 0;  // (FP32 has as many or none: the bands fit)
+        // (the bands of st64 leave room for st32)
+        const int st64 = split ? batch_storers<double>(ctx, sub->g) : 0, st32 = split ? batch_storers<float>(ctx, sub->g) : 0;
         const int br = split ? split_band_rows(ctx, sub->g.p, sub->g.ny, st64) : sub->g.ny;
-        const auto key = std::make_tuple(sub->g.p, (br + rpw - 1) / rpw, sub->mat.valid, e);
+        const auto key = std::make_tuple(sub->g.p, (br + rpw - 1) / rpw, sub->mat.valid, e, st64 + 16 * st32);
         auto it = gid.find(key);
         if (it == gid.end()) {
             it = gid.emplace(key, (int)ctx->groups.size()).first;
@@ -4321,7 +4326,7 @@ void build_batch_groups(tsw_ctx *ctx, const std::vector<int> &members) {
             G.ref = e == tsw_ctx::kEngRef || split;
             G.split = split;
             G.storers64 = st64;
-            G.storers32 = split ? batch_storers<float>(ctx, sub->g.p) : 0;
+            G.storers32 = st32;
         }
         auto &G = ctx->groups[it->second];
         G.members.push_back(b);
@@ -4643,23 +4648,16 @@ void batch_choose_engines(tsw_ctx *ctx) {
                 cand.push_back(tsw_ctx::kEngConverted);
             if (cand.empty()) cand.push_back(tsw_ctx::kEngConverted);
         }
-        // the lane-split engine is tried at degree 1 with the most rows one workgroup holds and with 64-row bands
-        // (smaller workgroups, more of them per CU), at degrees 2 and 3 with and without storer waves, unless set
-        struct Try {
-            char engine;
-            int rows, storers;
-        };
-        std::vector<Try> tries;
+        // the lane-split engine is tried with the most rows one workgroup holds and, at degrees 1 and 3, with 64-row
+        // bands (smaller workgroups, more of them per CU where the tables leave room), unless rows are set
+        std::vector<std::pair<char, int>> tries;
         for (char e : cand) {
-            tries.push_back({e, 0, kSplitStorers});
-            if (e == tsw_ctx::kEngSplit && ctx->batch_split_rows_opt == 0) {
-                if (p == 1) tries.push_back({e, 64, kSplitStorers});
-                else if (ctx->batch_split_storers_opt == 0) tries.push_back({e, 0, 0});
-            }
+            tries.emplace_back(e, 0);
+            if (e == tsw_ctx::kEngSplit && ctx->batch_split_rows_opt == 0 && p != 2) tries.emplace_back(e, 64);
         }
-        Try best = tries[0];
+        char best = cand[0];
+        int best_rows = 0;
         ctx->split_rows_p[p] = 0;
-        ctx->split_storers_p[p] = kSplitStorers;
         if (tries.size() > 1 && ctx->autotune) {
             // the heaviest members up to the scratch budget
             std::sort(mem.begin(), mem.end(),
@@ -4685,9 +4683,9 @@ void batch_choose_engines(tsw_ctx *ctx) {
             }
             double best_ms = 0.0;
             for (size_t t = 0; t < tries.size(); ++t) {
-                ctx->split_rows_p[p] = tries[t].rows;
-                ctx->split_storers_p[p] = tries[t].storers;
-                for (int b : sub_members) ctx->engine[b] = tries[t].engine;
+                const char e = tries[t].first;
+                ctx->split_rows_p[p] = tries[t].second;
+                for (int b : sub_members) ctx->engine[b] = e;
                 build_batch_groups(ctx, sub_members);
                 batch_apply(ctx, sub_members, dev, TSW_FP64);  // first touch of tables and buffers
                 hipEvent_t t0 = next_event(ctx), t1 = next_event(ctx);
@@ -4699,19 +4697,19 @@ void batch_choose_engines(tsw_ctx *ctx) {
                 TSW_HIP(hipEventElapsedTime(&ms, t0, t1));
                 if (t == 0 || ms < best_ms) {
                     best_ms = ms;
-                    best = tries[t];
+                    best = e;
+                    best_rows = tries[t].second;
                 }
             }
-            ctx->split_rows_p[p] = best.rows;
-            ctx->split_storers_p[p] = best.storers;
+            ctx->split_rows_p[p] = best_rows;
             sync(ctx);
             ctx->ev_used = 0;  // the tuning sweeps are not counted
             ctx->sweeps_done = 0;
             ctx->ms_folded = 0.0;
         }
         for (int b : mem) {
-            ctx->engine[b] = best.engine;
-            if (best.engine != tsw_ctx::kEngConverted) {  // diagonal-layout buffers of the tuning sweeps
+            ctx->engine[b] = best;
+            if (best != tsw_ctx::kEngConverted) {  // diagonal-layout buffers of the tuning sweeps
                 auto &d = ctx->batch[b]->diag;
                 d.q64.release();
                 d.q32.release();
@@ -4719,7 +4717,7 @@ void batch_choose_engines(tsw_ctx *ctx) {
                 d.ir64.release();
             }
         }
-        ctx->batch_engine[p] = best.engine;
+        ctx->batch_engine[p] = best;
     }
     ctx->groups.clear();
     ctx->lane_groups.clear();

@@ -124,8 +124,7 @@ int tsw_set_xs_degree(tsw_ctx *ctx, int degree);
  * degree 3; or 16..256, of which at most 256, 128 and 128 are used, and which keeps tsw_sweep_apply and
  * tsw_sweep_apply_multi on the lane-split kernel where they would take one with a lane per coefficient): rows per
  * band; "batch_split_storers" (0 default, 1, -1): two waves of a workgroup that only store, always (at most 192, 96 and 96
- * rows then), never, or by degree, precision and size, and, in FP64 batches of degrees 2 and 3, as the autotuner finds
- * faster; "batch_split_prefetch" (0
+ * rows then), never, or by degree, precision and size; "batch_split_prefetch" (0
  * default = 4, 3 in FP64 at degree 3 and for several FP32 sources at degree 2; or 2, 3, 4, 6): its prefetch depth; "batch_xcd_tile" (0 default = dispatch order, or
  * 2..64): runs of that many consecutive items (neighbouring ordinates of a member) go to one XCD (with
  * "batch_persistent" 0); "batch_persistent" (1 default, 0): each lane-split and ordinate-lane group is one

@@ -333,6 +333,36 @@ def test_split_batch_with_and_without_storers(precision, rows):
             np.testing.assert_array_equal(a, b, err_msg=f"{storers} {P.name}")
 
 
+@pytest.mark.parametrize("precision", [tsw.FP64, tsw.FP32])
+def test_split_batch_aligned_and_misaligned_by_turns(precision):
+    """Calls on 16-byte aligned arrays and on arrays 8 bytes off (through the conversions) by turns, bands with and without
+    storer waves (97 to 130 rows), the same exchange records."""
+    import torch
+    batch = problems.batched(seed=23, count=6, n_range=(97, 130), degrees=(2, 3), orders=(2, 4))
+    srcs = _random_halo_sources(batch, 9)
+    print("split batch by turns", precision, [(P.nx, P.p, P.nq) for P in batch], flush=True)
+    dev = torch.device("cuda:0")
+    refs = [oracle_sweep(P, s) for P, s in zip(batch, srcs)]
+    with _split_ctx(0) as ctx:
+        ctx.batch_set([problems.as_batch_member(P) for P in batch], [P.sigma_t for P in batch])
+        first = None
+        for off in (0, 1, 0, 1, 1, 0):
+            out = []
+            for s in srcs:
+                flat = torch.zeros(s.size + 1, dtype=torch.float64, device=dev)
+                a = flat[off:off + s.size].view(s.shape)
+                a.copy_(torch.from_numpy(s))
+                out.append(a)
+            ctx.batch_sweep(out, precision=precision)
+            assert ctx.get_tuning("batch_ref") == 1 - off
+            if first is None:
+                first = out
+                for a, r, P in zip(out, refs, batch):
+                    assert rel_err(a.cpu().numpy(), r) <= (1e-12 if precision == tsw.FP64 else 2e-6), P.name
+            for a, b, P in zip(out, first, batch):
+                assert torch.equal(a, b), (off, P.name)
+
+
 def test_split_batch_tuning_keys():
     with tsw.Context(0) as ctx:
         for key, bad in (("batch_split", 2), ("batch_split_rows", 8), ("batch_split_rows", 300),
