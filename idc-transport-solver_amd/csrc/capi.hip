@@ -2449,14 +2449,16 @@ int split_lanes_of(int p) { return p == 1 ? 2 : 4; }
 // four SIMDs, so that six (64 rows at degrees 2 and 3) leave no room for a second workgroup on a CU where a SIMD holds
 // three (FP64 Q2, FP32 Q3: 161 to 178 VGPRs) and a third of the rows are in flight.
 //
-// Members of a batch (64 materials, us, with and without): degree 1 with, 64 x 48^2 S12 261 and 318, 24 x 200^2 S8 1221 and
+// Batches of several groups always have them: another group's workgroups take what room is left on a CU, and without them
+// 60 uneven batches of 4 to 160 problems took 4% longer on average, 5 of 32^2 to 221^2 395 us in place of 302.  A batch that
+// is one group (alone; 64 materials, us, with and without): degree 1 with, 64 x 48^2 S12 261 and 318, 24 x 200^2 S8 1221 and
 // 1317.  Degree 2 in FP32 with: 32 x 48^2 S12 467 and 522, 24 x 200^2 1921 and 2419; in FP64 without up to 100 rows: 694 and
 // 545, 64 x 64^2 S8 839 and 800, 32 x 100^2 S12 1894 and 1804, but 32 x 128^2 S8 1299 and 1324, 24 x 200^2 2220 and 2396.
 // Degree 3 without where a member is then one band of 97 to 128 rows, as a CU has one workgroup for their LDS, which then
 // has seven or eight compute waves in place of four: FP64 32 x 100^2 2954 and 2196, 32 x 128^2 1855 and 1563, but 64 x 64^2
 // 1377 and 1418; and in FP32 below that: 32 x 48^2 941 and 730, 64 x 64^2 1077 and 919; and in bands of 64 rows, of which a
 // CU holds two where there are few materials.  Two bands in place of three, 24 x 200^2, 2815 and 2541, but with arrays that
-// do not start on a cache line, where whole runs cost less, the 85 Q3 members of 32^2 to 256^2 8.3 and 9.2 ms.
+// do not start on a cache line, where whole runs cost less, 85 Q3 members of 32^2 to 256^2 8.3 and 9.2 ms.
 // (a row count that leaves no room for them means none)
 int storers_forced(const tsw_ctx *c, int p) {
     if (c->batch_split_storers_opt != 0) return c->batch_split_storers_opt > 0 ? kSplitStorers : 0;
@@ -2464,9 +2466,10 @@ int storers_forced(const tsw_ctx *c, int p) {
 }
 bool one_band(int ny) { return ny > 96 && ny <= 128; }  // without storers at degree 3, two with them
 template <typename T>
-int batch_storers(const tsw_ctx *c, const Geom &g) {
+int batch_storers(const tsw_ctx *c, const Geom &g, bool alone) {
     const int forced = storers_forced(c, g.p);
     if (forced >= 0) return forced;
+    if (!alone) return kSplitStorers;
     if (g.p == 2) return sizeof(T) == 8 && g.ny <= 100 ? 0 : kSplitStorers;
     return g.p == 3 && (c->split_rows_p[3] == 64 || one_band(g.ny) || (sizeof(T) == 4 && g.ny <= 96)) ? 0 : kSplitStorers;
 }
@@ -4289,7 +4292,8 @@ void split_queues(tsw_ctx *ctx, tsw_ctx::Group &G, const std::vector<std::tuple<
 // Launch groups of the members `members` by their engines: staggered groups by (DG degree, compute waves,
 // material path, layout), work items {member slot, ordinate} heaviest first; lane groups by DG degree, items
 // {member slot, ordinate block, band} band-major, heaviest members first within a band.
-void build_batch_groups(tsw_ctx *ctx, const std::vector<int> &members) {
+// (alone: the batch is one group, whose workgroups then have the CUs to themselves)
+void form_batch_groups(tsw_ctx *ctx, const std::vector<int> &members, bool alone) {
     ctx->groups.clear();
     ctx->lane_groups.clear();
     std::map<std::tuple<int, int, bool, int, int>, int> gid;
@@ -4312,7 +4316,8 @@ void build_batch_groups(tsw_ctx *ctx, const std::vector<int> &members) {
         // staggered groups hold members of equal waves per workgroup, split groups of equal row slots and storers
         const int rpw = split ? 64 / split_lanes_of(sub->g.p) : 64;
         // (the bands of st64 leave room for st32)
-        const int st64 = split ? batch_storers<double>(ctx, sub->g) : 0, st32 = split ? batch_storers<float>(ctx, sub->g) : 0;
+        const int st64 = split ? batch_storers<double>(ctx, sub->g, alone) : 0;
+        const int st32 = split ? batch_storers<float>(ctx, sub->g, alone) : 0;
         const int br = split ? split_band_rows(ctx, sub->g.p, sub->g.ny, st64) : sub->g.ny;
         const auto key = std::make_tuple(sub->g.p, (br + rpw - 1) / rpw, sub->mat.valid, e, st64 + 16 * st32);
         auto it = gid.find(key);
@@ -4333,6 +4338,14 @@ void build_batch_groups(tsw_ctx *ctx, const std::vector<int> &members) {
         G.band_rows.push_back(br);
         G.max_ny = std::max(G.max_ny, sub->g.ny);
         G.rows = std::max(G.rows, br);
+    }
+}
+void build_batch_groups(tsw_ctx *ctx, const std::vector<int> &members) {
+    auto one = [&] { return ctx->groups.size() == 1 && ctx->lane_groups.empty(); };
+    form_batch_groups(ctx, members, false);
+    if (one() && ctx->groups[0].split) {
+        form_batch_groups(ctx, members, true);
+        if (!one()) form_batch_groups(ctx, members, false);
     }
     for (auto &G : ctx->groups) {
         // (-work, slot, band * nq + ordinate), band-major: every band's upstream band is dispatched first

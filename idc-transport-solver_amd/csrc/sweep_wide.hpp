@@ -16,7 +16,7 @@
 // Measured on one band of Q2 (FP64): 0.18 us a step with 8 rows, 0.24 with 24, 0.37 with 56, where the lane-split
 // sweep takes 0.5; without its loads and stores 0.16, 0.20 and 0.31: what is left is the wave's own chain (LDS, 14
 // dependent FP64 operations, barrier) and, with many rows, the issue slots of a CU's four SIMDs.  Kernel times against
-// the lane-split sweep's stand at the rule that picks one (wide_band_rows).
+// the lane-split sweep's stand at the rule that picks one (wide_most_rows).
 #pragma once
 
 namespace tsw {

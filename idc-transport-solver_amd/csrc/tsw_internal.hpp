@@ -262,9 +262,10 @@ size_t wide_sweep_lds_bytes(int p, int rows, int M);
 template <typename T>
 void launch_diag_sweep_batch(const DiagSweepParams<T> &rep, const DiagSweepParams<T> *probs, const int2 *items,
                              int nitems, int max_ny, size_t lds, int p, hipStream_t s);
-// Lane-split (sp.split 1) or lane-per-coefficient (2) sweeps of n <= kSplitSources right-hand sides of one problem in place on the reference layout
-// (16-byte aligned arrays below 4 GiB - 256 bytes; sp: material path, bands, sp.work / work_set; sp.prefetch the depth).
-// The launch does nothing while *changed == mark (changed not null); start and stop (or null) are recorded around it.
+// Lane-split (sp.split 1) or lane-per-coefficient (2) sweeps of n <= kSplitSources right-hand sides of one problem in
+// place on the reference layout (16-byte aligned arrays below 4 GiB - 256 bytes; sp: material path, bands, sp.storers,
+// sp.work / work_set; sp.prefetch the depth).  The launch does nothing while *changed == mark (changed not null); start
+// and stop (or null) are recorded around it.
 template <typename T>
 void launch_split_ref(const DiagSweepParams<T> &sp, const SplitSources &src, int n, size_t lds, int p,
                       const int *changed, int mark, hipStream_t s, hipEvent_t start, hipEvent_t stop);

@@ -120,14 +120,14 @@ int tsw_set_xs_degree(tsw_ctx *ctx, int degree);
  * kernel on the caller's layout, and keeps the fastest.  Key "batch_split" (0 default, 1, -1): that
  * lane-split engine (DG degrees 1-3, row bands with exchange records, a band's workgroup at most 512
  * threads) forced, forbidden or autotuned; "batch_split_rows" (0 default = the most rows one workgroup
- * sweeps at its fastest: 192 at degree 1, or 64 where the batch autotuner finds that faster, 64 at degree 2, 96 or 128 at
- * degree 3; or 16..256, of which at most 256, 128 and 128 are used, and which keeps tsw_sweep_apply and
- * tsw_sweep_apply_multi on the lane-split kernel where they would take one with a lane per coefficient): rows per
- * band; "batch_split_storers" (0 default, 1, -1): two waves of a workgroup that only store, always (at most 192, 96 and 96
- * rows then), never, or by degree, precision and size; "batch_split_prefetch" (0
- * default = 4, 3 in FP64 at degree 3 and for several FP32 sources at degree 2; or 2, 3, 4, 6): its prefetch depth; "batch_xcd_tile" (0 default = dispatch order, or
- * 2..64): runs of that many consecutive items (neighbouring ordinates of a member) go to one XCD (with
- * "batch_persistent" 0); "batch_persistent" (1 default, 0): each lane-split and ordinate-lane group is one
+ * sweeps at its fastest: 192 at degree 1, 64 at degree 2, 96 or 128 at degree 3, or 64 at degrees 1 and 3 where
+ * the batch autotuner finds that faster; or 16..256, of which at most 256, 128 and 128 are used, and which keeps
+ * tsw_sweep_apply and tsw_sweep_apply_multi on the lane-split kernel where they would take one with a lane per
+ * coefficient): rows per band; "batch_split_storers" (0 default, 1, -1): two waves of a workgroup that only
+ * store, always (at most 192, 96 and 96 rows then), never, or by degree, precision and size;
+ * "batch_split_prefetch" (0 default = 4, 3 in FP64 at degree 3 and for several FP32 sources at degree 2; or
+ * 2, 3, 4, 6): its prefetch depth; "batch_xcd_tile" (0 default = dispatch order, or 2..64): runs of that many
+ * consecutive items (neighbouring ordinates of a member) go to one XCD (with "batch_persistent" 0); "batch_persistent" (1 default, 0): each lane-split and ordinate-lane group is one
  * persistent launch of as many workgroups as the device holds, taking items in order from device
  * counters (0: one workgroup per item).  Key "ref_stage" (0 default, 1): sweeps on the caller's layout (batch groups,
  * tsw_sweep_apply_multi) stage their source loads through LDS where it fits.  Results do not depend on
@@ -158,8 +158,8 @@ int tsw_set_tuning(tsw_ctx *ctx, const char *key, int value);
  * 1 staggered on the caller's layout, 2 ordinate lanes, 3 lane-split on the caller's layout, -1 none in
  * the batch), "batch_split_rows_p0" .. "batch_split_rows_p3" (the lane-split engine's rows per band the
  * batch autotuner chose for that degree, 0: the most a workgroup holds), or the setting of
- * "batch_direct", "ref_stage", "batch_split", "batch_split_rows",
- * "batch_split_storers", "batch_split_prefetch" (the depth in use), "batch_persistent", "batch_xcd_tile", "ref_split", "autotune",
+ * "batch_direct", "ref_stage", "batch_split", "batch_split_rows", "batch_split_storers",
+ * "batch_split_prefetch" (the setting, or 4), "batch_persistent", "batch_xcd_tile", "ref_split", "autotune",
  * "use_dsa", "dsa_cycles", "si_graph", "refine_steps", "gmres_refine", "fp32_safety". */
 int tsw_get_tuning(tsw_ctx *ctx, const char *key, int *value);
 
