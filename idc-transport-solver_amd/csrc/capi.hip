@@ -2519,35 +2519,44 @@ int wide_band_rows(int p, int ny) {
 //     516 -> 525 (2 materials); Q1 256 x 256 S12 (21,504 rows) 241 -> 229, but 300 x 150 S16 (21,600 rows) 215 -> 244.
 //   many sources: Q1 64 x 64 n = 32 (81,920 rows) 197 -> 172, but 100 x 100 S12 n = 12 (100,800 rows) 351 -> 381, 128 x 64 n =
 //     24 306 -> 334; Q2 64 x 64 S16 n = 32 (294,912 rows) 1310 -> 1108, 100 x 100 S12 n = 20 1200 -> 1163, but 32 x 32 S16
-//     n = 16 (73,728 rows) 209 -> 236; FP32 Q2 16 x 100 n = 32 372 -> 222, but 64 x 64 n = 9 (23,040 rows) 131 -> 145.
+//     n = 16 (73,728 rows) 209 -> 236; FP32 Q2 16 x 100 n = 32 372 -> 222, but 64 x 64 n = 9 (23,040 rows) 131 ->
+//     145, one source 16 x 400 S12 211 -> 253.
 //   Q3: a CU holds one workgroup of either with 64 materials, but three of this one with few, so that the line goes with the
 //     rows that a CU holds: 128 x 128 n = 5 (25,600 rows) 390 -> 370, but n = 6 392 -> 427; 2 materials 350 x 350 S16 (50,400
 //     rows) 1229 -> 1185, but 440 x 440 (63,360 rows) 1740 -> 1810; FP32 n = 4 (20,480 rows) 317 -> 313, but n = 5 333 ->
 //     369; 2 materials n = 5 298 -> 297, but n = 6 323 -> 347.  Few columns: 48 x 48 S12 n = 32 1084 -> 590, 100 x 100 S12 n =
 //     12, 2 materials 742 -> 632, but 64 materials, without storers, 819 -> 1047; FP32 in one band 56 x 56 S12 n = 20 494 ->
-//     446, in more 64 x 64 S12 n = 20 670 -> 797.
+//     446, in more 64 x 64 S12 n = 20 670 -> 797.  Narrow meshes: 16 x 100 n = 20 515 -> 418; FP32 16 x 448 S4 n = 8 373 ->
+//     235, 60 x 300 n = 3 343 -> 302, one source 16 x 400 S12 323 -> 207, 61 x 300 S16 (43,200 rows) 322 -> 296, but 100 x
+//     440 S16 (63,360 rows) 592 -> 649.
 template <typename T>
-double wide_most_rows(const Geom &g, int rows, size_t lds, int split_rows, int storers) {
+double wide_most_rows(const Geom &g, int n, int rows, size_t lds, int split_rows, int storers) {
     constexpr double any = 1e300;
     constexpr bool f64 = sizeof(T) == 8;
     if (g.p == 1) return g.nx <= 100 ? 82000 : 20000;
     if (g.p == 2) {
         if (f64) return g.nx > 100 ? 20000 : g.ny <= 32 ? 41000 : any;
-        return g.nx <= 40 && g.ny > 32 ? any : 20000;
+        return n > 1 && g.nx <= 40 && g.ny > 32 && g.ny <= 200 ? any : 20000;
     }
     const double held = std::min<double>(3, (160 * 1024) / lds) * rows / split_rows;  // a CU's rows, against the lane-split's
-    if (f64 ? g.nx <= 100 && (storers || held >= 0.5) : rows >= g.ny) return any;
-    return f64 ? std::max(27000.0, 60000 * held) : std::max(21000.0, 30000 * held);
+    if (g.ny >= 6 * g.nx) return any;
+    if (f64) return g.nx <= 100 && (storers || held >= 0.5) ? any : std::max(27000.0, 60000 * held);
+    if (rows >= g.ny || (n == 1 && g.nx <= 60)) return any;
+    return std::max(g.ny >= 5 * g.nx || (n == 1 && g.nx <= 100) ? 45000.0 : 21000.0, 30000 * held);
 }
 
 // Prefetch depth of the lane-split kernel on the reference layout: 3 for FP64 Q3, whose ring of 4 spills (256 x 256, S8,
-// 64 materials: 461 against 556 us), and for several sources of FP32 Q2 (k_split_ref: 121 VGPRs in place of 129, four
-// waves a SIMD; 48 x 48 S12, 16 sources 307 -> 216 us, 128 x 128 S8, 32 sources 1132 -> 1100, but a single 250 x 250 S16
-// sweep 665 -> 723), else kSplitBatchPrefetch, unless the tuning key batch_split_prefetch sets it.
+// 64 materials: 461 against 556 us), and for a launch of FP32 Q2 sources with more compute waves than the three a SIMD that
+// a ring of 4 leaves (k_split_ref: 121 VGPRs in place of 129, four waves a SIMD; 48 x 48 S12, 16 sources, 15.8 waves a CU,
+// 307 -> 216 us, 128 x 128 S8, 32 sources 1132 -> 1100, but 20 x 20 S8, 32 sources, 10 waves a CU, 142 -> 152, 16 x 448 S4,
+// 8 sources, 10.5 waves, 238 -> 248, and a single 250 x 250 S16 sweep 665 -> 723), else kSplitBatchPrefetch, unless the
+// tuning key batch_split_prefetch sets it.
 template <typename T>
-int split_prefetch(const tsw_ctx *c, int p, int sources = 1) {
+int split_prefetch(const tsw_ctx *c, int p, int sources = 1, int bands = 1, int rows = 0) {
     if (c->batch_split_pf_opt > 0) return c->batch_split_pf_opt;
-    return (p == 3 && sizeof(T) == 8) || (p == 2 && sizeof(T) == 4 && sources > 1) ? 3 : kSplitBatchPrefetch;
+    if (sizeof(T) == 8) return p == 3 ? 3 : kSplitBatchPrefetch;
+    const long long waves = (long long)sources * c->g.nq * bands * ((rows * split_lanes_of(p) + 63) / 64);
+    return p == 2 && sources > 1 && waves > 12 * kCus ? 3 : kSplitBatchPrefetch;
 }
 
 // Whether this context's sweeps can run the staggered kernel on the caller's layout for `psi`.
@@ -2584,7 +2593,7 @@ bool split_ref_plan(tsw_ctx *c, const double *sig, double dt, bool known, int n,
     base.split = 1;
     const int wr = wide_band_rows(g.p, g.ny);
     const size_t l = c->batch_split_rows_opt == 0 ? wide_sweep_lds_bytes<T>(g.p, wr, base.M) : 0;
-    if (l > 0 && (double)std::min(n, kSplitSources) * g.nq * g.ny <= wide_most_rows<T>(g, wr, l, br, base.storers)) {
+    if (l > 0 && (double)std::min(n, kSplitSources) * g.nq * g.ny <= wide_most_rows<T>(g, n, wr, l, br, base.storers)) {
         br = wr;
         lds = l;
         base.split = 2;
@@ -2626,7 +2635,7 @@ void split_ref_sweep(tsw_ctx *c, DiagSweepParams<T> base, size_t lds, const std:
         base.abort_flag = abort_flag_of(c);
     }
     // (a ring of 3 takes 2 to 4% longer with a lane per coefficient, one of 6 up to 20%)
-    base.prefetch = base.split == 2 && c->batch_split_pf_opt == 0 ? 4 : split_prefetch<T>(c, g.p, n);
+    base.prefetch = base.split == 2 && c->batch_split_pf_opt == 0 ? 4 : split_prefetch<T>(c, g.p, most, nb, base.band_rows);
     if (c->stall_test && per) {  // tuning key stall_test: every bounded wait of the banded sweep gives up
         c->stall_test = false;
         (void)abort_flag_of(c);

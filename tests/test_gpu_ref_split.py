@@ -233,7 +233,9 @@ def test_ref_split_persistent_switched_on_and_off(p, rows):
 @pytest.mark.parametrize("shape,kernel", [((101, 60, 1, 8, 9), (0, 0)), ((101, 60, 2, 8, 9), (0, 0)), ((101, 60, 2, 8, 8), (1, 1)),
                                           ((101, 112, 3, 8, 7), (1, 1)), ((101, 112, 3, 8, 13), (0, 0)),
                                           ((30, 100, 1, 8, 21), (0, 0)), ((20, 32, 2, 8, 33), (1, 0)),
-                                          ((50, 40, 2, 8, 13), (1, 0)), ((40, 60, 3, 8, 13), (1, 0))])
+                                          ((50, 40, 2, 8, 13), (1, 0)), ((40, 60, 3, 8, 13), (1, 0)),
+                                          ((40, 200, 2, 8, 3), (1, 1)), ((40, 201, 2, 8, 3), (1, 0)),
+                                          ((12, 100, 3, 8, 14), (1, 1)), ((50, 60, 2, 8, 20), (1, 0))])
 def test_ref_sweeps_of_many_sources_equal_single_sweeps(shape, kernel, prec):
     import torch
     nx, ny, p, order, n = shape
